@@ -17,7 +17,9 @@
  *  2. A device API (zccl_*_dev): device pointers only, explicit chunk count,
  *     asynchronous on a caller-supplied hipStream_t, caller-owned workspace.
  *     Every device stream travels with an index (block widths, tile and seed
- *     offsets, stream size) that the kernels use instead of walking the bytes.
+ *     offsets, stream size, for 36-value blocks the quantized value before
+ *     every 64 blocks) that the kernels use instead of walking the bytes; its
+ *     layout belongs to the library version that wrote it.
  *
  * Streams are byte-identical to the reference's for the same input, error
  * bound, block length and chunk count.

@@ -18,7 +18,8 @@ import torch
 
 from . import _lib
 from ._lib import check, lib
-from .codec import STAGED_L, DeviceStream, Workspace, _stream_handle, default_stage, default_workspace, staged_min_tiles
+from .codec import (STAGED_L, DeviceStream, Workspace, _stream_handle, default_stage, default_workspace, indexed,
+                    staged_min_tiles)
 
 
 class BatchPlan:
@@ -80,6 +81,7 @@ def homsum_plan(jobs: Sequence[Sequence[DeviceStream]], outs: Sequence[DeviceStr
     nj = len(jobs)
     if len(outs) != nj or nj == 0:
         raise ValueError("one output per job")
+    jobs = [[indexed(s) for s in ops] for ops in jobs]
     L, T = outs[0].L, outs[0].T
     for j, ops in enumerate(jobs):
         if not 1 <= len(ops) <= 32:
@@ -118,6 +120,7 @@ def compress_plan(xs: Sequence[torch.Tensor], ebs: Sequence[float], outs: Sequen
 
 
 def decompress_plan(streams: Sequence[DeviceStream], ebs: Sequence[float], outs: Sequence[torch.Tensor]) -> BatchPlan:
+    streams = [indexed(s) for s in streams]
     nj = len(streams)
     L, T = streams[0].L, streams[0].T
     for s, y in zip(streams, outs):

@@ -17,6 +17,7 @@ ZCCL/include/ZCCLd_float.h:21,29):
 from __future__ import annotations
 
 import ctypes
+import functools
 from dataclasses import dataclass, field
 from typing import Dict, Optional, Sequence, Tuple
 
@@ -44,6 +45,7 @@ def worst_case_bytes(n: int, L: int, T: int) -> int:
     return int(v)
 
 
+@functools.lru_cache(maxsize=4096)
 def index_bytes(n: int, L: int, T: int) -> int:
     return int(lib().zccl_index_bytes(n, L, T))
 
@@ -135,7 +137,8 @@ class DeviceStream:
     """A compressed stream resident in HBM together with its index.
 
     ``data[:size]`` are the stream bytes in the reference wire format;
-    ``index`` holds the per-block widths, tile and seed offsets and the size.
+    ``index`` holds the per-block widths, tile and seed offsets, the size and
+    (36-value blocks) the quantized value before each run of 64 blocks.
     """
 
     data: torch.Tensor
@@ -178,6 +181,14 @@ def empty_stream(n: int, L: int, T: int, capacity: Optional[int] = None,
     return DeviceStream(data, index, n, L, T)
 
 
+def indexed(s: DeviceStream) -> DeviceStream:
+    """s, or (its index kept from a library that wrote shorter ones) the same
+    bytes under an index of this library's size."""
+    if s.index.numel() >= index_bytes(s.n, s.L, s.T):
+        return s
+    return from_bytes(s.data, s.n, s.L, s.T)
+
+
 def _ws_for(n: int, L: int, T: int, ws: Optional[Workspace]) -> Workspace:
     tiles = num_tiles(n, L, T)
     if ws is None:
@@ -209,6 +220,7 @@ def decompress(s: DeviceStream, eb: float, out: Optional[torch.Tensor] = None,
     if y.numel() != s.n or y.dtype != torch.float32 or not y.is_contiguous():
         raise ValueError("out must be a contiguous float32 tensor of n elements")
     w = _ws_for(s.n, s.L, s.T, ws)
+    s = indexed(s)
     check(lib().zccl_decompress_dev(_ptr(s.data), _ptr(s.index), s.n, ctypes.c_float(eb), s.L, s.T,
                                     _ptr(y), w.ptr, w.nbytes, _stream_handle()), "decompress")
     return y
@@ -234,7 +246,7 @@ def homsum(streams: Sequence[DeviceStream], out: Optional[DeviceStream] = None,
         st = stage if stage is not None else default_stage(tiles)
         if st.max_tiles < tiles:
             raise _lib.ZcclError(-6, f"stage area holds {st.max_tiles} tiles, sum needs {tiles}")
-    ops = list(streams)
+    ops = [indexed(s) for s in streams]
     while len(ops) > MAX_OPERANDS:
         part = _homsum_launch(ops[:MAX_OPERANDS], None, w, st)
         ops = [part] + ops[MAX_OPERANDS:]

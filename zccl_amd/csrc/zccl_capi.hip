@@ -532,8 +532,6 @@ zccl_batch* batch_plan(BatchKind kind, const std::vector<Job>& jobs, uint32_t ch
     a.interleave = uniform && nj > 1;
     a.total_chains = chains;
     a.total_tiles = tile0[nj];
-    for (size_t j = 0; j < nj; j++)
-        a.max_segments = std::max(a.max_segments, jobs[j].g.S);
     if (uniform) {
         a.g = jobs[0].g;
         a.tl = jobs[0].tl;
@@ -777,6 +775,7 @@ extern "C" int zccl_parse_dev(const unsigned char* in, size_t in_cap, size_t n, 
     a.ws = (WsHeader*) ws;
     a.ws_bytes = ws_bytes;
     a.size_out = d_size;
+    a.carries = true;
     HIP_TRY(launch_parse(a, (hipStream_t) stream));
     return ZCCL_OK;
 }
@@ -920,9 +919,10 @@ unsigned long long* small_slot(Ctx& c, int i) { return (unsigned long long*) c.s
 // Make stream bytes available on the device and build their index.  A host
 // stream is copied exactly: cap bytes when its size is stated (cap_exact),
 // else the size its own header and width bytes prove.  For a device stream
-// the allocation bounds the read.
+// the allocation bounds the read.  `carries`: the index is for decompress (a
+// sum reads the seeds from the bytes, and its own index is not kept).
 int stage_stream(Ctx& c, const Geom& g, const unsigned char* bytes, size_t cap, bool cap_exact,
-    int slot, const unsigned char** dptr)
+    int slot, bool carries, const unsigned char** dptr)
 {
     size_t avail = 0;
     const bool dev = device_ptr(bytes, &avail);
@@ -957,6 +957,7 @@ int stage_stream(Ctx& c, const Geom& g, const unsigned char* bytes, size_t cap, 
     a.ws = (WsHeader*) c.ws.p;
     a.ws_bytes = c.ws.cap;
     a.size_out = nullptr;
+    a.carries = carries;
     HIP_TRY(launch_parse(a, c.stream));
     *dptr = d;
     return ZCCL_OK;
@@ -1027,7 +1028,7 @@ int dropin_decompress(float* newData, size_t n, float eb, int L, int T, const un
     if ((rc = ensure_ws(*c, zccl_num_tiles(n, L, T), n, L, T)))
         return rc;
     const unsigned char* din = nullptr;
-    if ((rc = stage_stream(*c, g, cmp, cmpSize, sized, 0, &din)))
+    if ((rc = stage_stream(*c, g, cmp, cmpSize, sized, 0, true, &din)))
         return rc;
     size_t avail = 0;
     bool odev = device_ptr(newData, &avail);
@@ -1067,7 +1068,7 @@ int dropin_add(unsigned char* out, size_t out_cap, bool out_cap_known, size_t* o
         return rc;
     const unsigned char* da = nullptr;
     const unsigned char* db = nullptr;
-    if ((rc = stage_stream(*c, g, a, asz, sized, 0, &da)) || (rc = stage_stream(*c, g, b, bsz, sized, 1, &db)))
+    if ((rc = stage_stream(*c, g, a, asz, sized, 0, false, &da)) || (rc = stage_stream(*c, g, b, bsz, sized, 1, false, &db)))
         return rc;
     uint64_t cap = worst_case_bytes(g);
     if ((rc = ensure(c->out, cap)))

@@ -260,6 +260,7 @@ struct IndexView {
     unsigned long long* group_off;
     unsigned long long* seed_off;
     unsigned long long* meta;
+    uint32_t* carry;  // g.ncarry entries
 };
 
 __device__ __forceinline__ IndexView index_view(const Geom& g, const uint8_t* ix)
@@ -269,6 +270,7 @@ __device__ __forceinline__ IndexView index_view(const Geom& g, const uint8_t* ix
     v.group_off = (unsigned long long*) (ix + g.ix_group);
     v.seed_off = (unsigned long long*) (ix + g.ix_seed);
     v.meta = (unsigned long long*) (ix + g.ix_meta);
+    v.carry = (uint32_t*) (ix + g.ix_carry);
     return v;
 }
 

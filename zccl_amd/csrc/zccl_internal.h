@@ -20,9 +20,11 @@
 //     straddles two segments);
 //   * a device-resident stream travels with an index: widths[nblocks] (one
 //     byte per block), group_off[ngroups] (byte offset of each group's first
-//     block), seed_off[S] (byte offset of each seed) and a meta word holding
-//     the stream size.  With the index every kernel finds its bytes without a
-//     sequential walk of the stream.
+//     block), seed_off[S] (byte offset of each seed), a meta word holding the
+//     stream size and, for 36-value blocks, carry[ncarry] (the quantized value
+//     before each run of 64 blocks of a segment).  With the index every kernel
+//     finds its bytes without a sequential walk of the stream, and decompress
+//     starts at any run without the deltas before it.
 #pragma once
 
 #include <stddef.h>
@@ -64,7 +66,9 @@ struct Geom {
     uint32_t gT, gR;     // groups per regular / remainder segment
     uint32_t ngroups;
     // index layout (byte offsets inside an index buffer)
-    uint32_t ix_group, ix_seed, ix_meta, ix_bytes;
+    uint32_t ix_group, ix_seed, ix_meta, ix_carry, ix_bytes;
+    uint32_t cT, cR;     // carries per regular / remainder segment (0: none kept)
+    uint32_t ncarry;
 };
 
 ZK_HD uint64_t ceil_div(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
@@ -78,6 +82,16 @@ ZK_HD uint32_t block_bytes(uint32_t b, uint32_t n)
         return 1;
     return 1 + ((n + 7) >> 3) + (b >> 3) * n + (((b & 7) * n + 7) >> 3);
 }
+
+// Lane layout (zccl_lane.hip): one lane per block of the reference's default
+// length, one wave per tile of 64 blocks (4 index groups), kLaneWaves tiles
+// per workgroup.  Its tiles are the runs the index keeps carries for: lane
+// tile t starts from carry[t].
+constexpr uint32_t kLaneL = 36;
+constexpr uint32_t kLaneTileBlocks = 64;
+constexpr uint32_t kLaneWaves = 4;
+
+ZK_HD bool lane_layout_ok(const Geom& g) { return g.L == kLaneL && g.IG == 16; }
 
 // Fill g for (n, L, T); false when the reference would be undefined (n < T:
 // ZCCL/src/ZCCL_float.c:543-544 underflows) or L is out of range.
@@ -103,7 +117,12 @@ ZK_HD bool make_geom(uint64_t n, uint32_t L, uint32_t T, Geom* g)
     g->ix_group = (uint32_t) align_up(g->nblocks, 16);
     g->ix_seed = g->ix_group + 8 * g->ngroups;
     g->ix_meta = (uint32_t) align_up(g->ix_seed + 8ull * g->S, 16);
-    g->ix_bytes = g->ix_meta + 32;
+    const bool lane = lane_layout_ok(*g);
+    g->cT = lane ? (uint32_t) ceil_div(g->gT, kLaneTileBlocks / g->IG) : 0u;
+    g->cR = lane ? (uint32_t) ceil_div(g->gR, kLaneTileBlocks / g->IG) : 0u;
+    g->ncarry = T * g->cT + g->cR;
+    g->ix_carry = g->ix_meta + 32;
+    g->ix_bytes = (uint32_t) align_up(g->ix_carry + 4ull * g->ncarry, 16);
     return true;
 }
 
@@ -154,15 +173,6 @@ ZK_HD Tiling make_tiling(const Geom& g, uint32_t target_threads)
     t.tile_bytes_max = t.G * block_bytes(32, g.L);
     return t;
 }
-
-// Lane layout (zccl_lane.hip): one lane per block of the reference's default
-// length, one wave per tile of 64 blocks (4 index groups), kLaneWaves tiles
-// per workgroup.
-constexpr uint32_t kLaneL = 36;
-constexpr uint32_t kLaneTileBlocks = 64;
-constexpr uint32_t kLaneWaves = 4;
-
-ZK_HD bool lane_layout_ok(const Geom& g) { return g.L == kLaneL && g.IG == 16; }
 
 // Compress in the lane layout: a workgroup of kLaneWaves waves per tile of
 // kLaneWaves x 64 blocks (one lookback per workgroup).

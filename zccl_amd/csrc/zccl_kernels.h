@@ -112,8 +112,6 @@ struct BatchArgs {
     uint32_t uniform;
     uint32_t interleave;
     uint32_t total_chains;
-    uint32_t max_segments;  // the most segments of any job
-    uint32_t pad0;
     uint64_t total_tiles;
     Geom g;
     Tiling tl;
@@ -129,6 +127,7 @@ struct ParseArgs {
     WsHeader* ws;
     uint64_t ws_bytes;             // the workspace's size (the parallel parse keeps its tables there)
     unsigned long long* size_out;
+    bool carries;                  // write the index carries too (36-value blocks)
 };
 
 // Parallel parse (zccl_kernels.hip): a chunk's block region (the bytes after
@@ -219,6 +218,8 @@ hipError_t launch_homsum_lane_wg_batch(const BatchArgs& b, hipStream_t s);
 hipError_t launch_compress_lane(const CompressArgs& a, hipStream_t s);
 hipError_t launch_compress_lane_batch(const BatchArgs& b, hipStream_t s);
 hipError_t launch_decompress_lane(const DecompressArgs& a, hipStream_t s);
+// Carries of a stream whose index lacks them alone (a foreign stream's parse).
+hipError_t launch_lane_carries(const DecompressArgs& a, hipStream_t s);
 hipError_t launch_decompress_lane_batch(const BatchArgs& b, hipStream_t s);
 // Workgroups per CU of the persistent lane decompress grid (1 ..
 // kDecGroupsMax; 0 restores the default, 4).

@@ -276,6 +276,22 @@ __device__ __forceinline__ void finish_tile(const Geom& g, const Tile& x, uint64
     }
 }
 
+// Carries of the lane tiles (runs of 64 blocks of a segment) that start in
+// tile x, one thread each: f(first element of the run, carry's index).  A
+// segment without blocks keeps its seed as its one carry.
+template <typename F>
+__device__ __forceinline__ void tile_carries(const Geom& g, const Tiling& tl, const Tile& x, uint8_t* index, F f)
+{
+    if (!g.ncarry)
+        return;
+    IndexView ix = index_view(g, index);
+    const uint32_t first = x.lt * tl.G;  // the tile's first block in its segment
+    const uint32_t c0 = (x.s < g.T ? x.s * g.cT : g.T * g.cT);
+    const uint32_t m = (first + kLaneTileBlocks - 1) / kLaneTileBlocks + threadIdx.x;
+    if (m * kLaneTileBlocks < first + x.nblk || (x.nblk == 0 && m == 0))
+        ix.carry[c0 + m] = f(x.seg_a + m * kLaneTileBlocks * g.L, c0 + m);
+}
+
 // Output side shared by compress and the homomorphic sum: per-block widths
 // from sh.bmax, block offsets, the lookback for the tile's stream offset,
 // encoding into LDS, the tile store, seed / header entry and output index.
@@ -416,6 +432,7 @@ __device__ __forceinline__ void compress_tile(const Geom& g, const Tiling& tl, c
     uint32_t seed = 0;
     if (x.lt == 0 && tid == 0)
         seed = (uint32_t) quant(io.x[x.seg_a], p.inv);
+    tile_carries(g, tl, x, io.index, [&](uint32_t e, uint32_t) { return (uint32_t) quant(io.x[e], p.inv); });
     encode_tile(g, tl, x, t, sh, buf, status, ws, un, d, seed, io.out, io.out_cap, io.index, io.size_out,
         t == tl.ntiles - 1, nchains);
 }
@@ -705,6 +722,12 @@ __device__ __forceinline__ void homsum_tile(const Geom& g, const Tiling& tl, con
         if (round + 1 < sp.nrounds && !overlap)
             issue_round(io.in, os, sp, round + 1, stage8);
     }
+    tile_carries(g, tl, x, io.index, [&](uint32_t, uint32_t c) {
+        uint32_t v = 0;
+        for (int r = 0; r < p.k; r++)
+            v += index_view(g, io.in[r].index).carry[c];
+        return v;
+    });
     uint32_t seed = 0;
     if (x.lt == 0 && tid == 0) {
         for (int r = 0; r < p.k; r++) {
@@ -994,6 +1017,12 @@ __device__ __forceinline__ void homsum_tile_slots(const Geom& g, const Tiling& t
     }
     if (bad)
         raise_error(ws, ZK_ERR_MISMATCH);
+    tile_carries(g, tl, x, io.index, [&](uint32_t, uint32_t c) {
+        uint32_t v = 0;
+        for (int r = 0; r < p.k; r++)
+            v += index_view(g, io.in[r].index).carry[c];
+        return v;
+    });
     uint32_t seed = 0;
     if (x.lt == 0 && tid == 0) {
         for (int r = 0; r < p.k; r++) {
@@ -1092,6 +1121,7 @@ __device__ __forceinline__ void compress_tile_slots(const Geom& g, const Tiling&
     uint32_t seed = 0;
     if (x.lt == 0 && tid == 0)
         seed = (uint32_t) quant(io.x[x.seg_a], p.inv);
+    tile_carries(g, tl, x, io.index, [&](uint32_t e, uint32_t) { return (uint32_t) quant(io.x[e], p.inv); });
     // (slot_output's first barrier also ends every read of the staged values,
     // so the encode may reuse the buffer)
     slot_output<L, W>(g, tl, x, t, sh, buf, jb0, nj, u, last_len, d, seed, io.out, io.out_cap, io.index,
@@ -2264,6 +2294,21 @@ hipError_t launch_batch(BatchKind kind, const BatchArgs& b, uint32_t threads, si
     return hipGetLastError();
 }
 
+// The carries of a parsed stream: its deltas' sums per lane tile, scanned.
+static hipError_t parse_carries(const ParseArgs& a, hipStream_t s)
+{
+    if (!a.carries || !a.g.ncarry)
+        return hipGetLastError();
+    DecompressArgs d;
+    memset(&d, 0, sizeof(d));
+    d.job.g = a.g;
+    d.job.tl = make_lane_tiling(a.g);
+    d.job.io.in[0].bytes = a.bytes;
+    d.job.io.in[0].index = a.index;
+    d.ws = a.ws;
+    return launch_lane_carries(d, s);
+}
+
 hipError_t launch_parse(const ParseArgs& a, hipStream_t s)
 {
     const ParseLayout pl = parse_layout(a.g);
@@ -2276,7 +2321,7 @@ hipError_t launch_parse(const ParseArgs& a, hipStream_t s)
         hipLaunchKernelGGL(k_parse_emit, dim3(groups), dim3(256), 0, s, a, pl);
         hipLaunchKernelGGL(k_parse_finish, dim3(1 + (uint32_t) std::min<uint64_t>(ceil_div(words, 256), 4096)), dim3(256),
             0, s, a, pl);
-        return hipGetLastError();
+        return parse_carries(a, s);
     }
     // the stream size starts at 0 (a fill kernel, safe under graph capture):
     // only a parse that reaches the stream's end writes it, so a failed parse
@@ -2285,7 +2330,7 @@ hipError_t launch_parse(const ParseArgs& a, hipStream_t s)
     if (a.size_out)
         hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, s, a.size_out, 1ull, 0ull);
     hipLaunchKernelGGL(k_parse, dim3(a.g.T), dim3(64), 0, s, a);
-    return hipGetLastError();
+    return parse_carries(a, s);
 }
 
 hipError_t launch_case_count(const uint8_t* w1, const uint8_t* w2, uint64_t nblocks,

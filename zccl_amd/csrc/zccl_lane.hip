@@ -492,12 +492,14 @@ __device__ __forceinline__ void homsum_tile_lane(const Geom& g, const Tiling& tl
     const uint8_t* tb_bytes = nullptr;
     const uint8_t* tb_index = nullptr;
     uint64_t tb_goff = 0, tb_size = 0;
+    uint32_t carry = 0;
     if (lane < (uint32_t) k) {
         tb_bytes = src.bytes((int) lane);
         tb_index = src.index((int) lane);
         const IndexView iv = index_view(g, tb_index);
         tb_goff = iv.group_off[x.grp0];
         tb_size = iv.meta[0];
+        carry = iv.carry[t];
     }
     // (readlane returns int: widen through uint32_t, never by sign extension)
     auto rl64 = [](uint64_t v, int r) -> uint64_t {
@@ -592,6 +594,11 @@ __device__ __forceinline__ void homsum_tile_lane(const Geom& g, const Tiling& tl
             o2 = op_of(1);
             wq2 = widths(o2);
         }
+        // the sum's carry into the tile: the operands' carries add in int32
+        // (while the first operand's bytes are on their way)
+        carry = wave_scan_dpp(carry);
+        if (lane == 63 && x.ngrp)
+            index_view(g, oindex).carry[t] = carry;
         for (int r = 0; r < k; r++) {
             const Loc c = cn;
             const bool staged = sn;
@@ -904,24 +911,20 @@ __device__ __forceinline__ void homsum_tile_lane(const Geom& g, const Tiling& tl
 
 // ---------------------------------------------------------------- decompress
 //
-// Two passes, no wait between tiles.  Pass one: lane j decodes block j of the
-// wave's tile (the sum's loaders and decoders, one operand) and the wave
-// writes the tile's sum of deltas.  A scan per segment turns the sums into
-// each tile's carry, starting from the segment's seed.  Pass two decodes the
-// tile again, takes the running sums of the deltas in the lane, places the
-// blocks with one scan of the block sums across the wave, dequantizes, and
-// stores the values through the wave's LDS buffer, half a tile at a time,
-// with 16-byte stores.  Arithmetic: prefix sums of the deltas in int32 from
-// the segment's seed, x' = (float) q * eb (ZCCL/src/ZCCLd_float.c:588-628).
+// One pass, no wait between tiles: the index holds the quantized value before
+// every tile (its carry).  Lane j decodes block j of the wave's tile (the sum's
+// loaders and decoders, one operand), takes the running sums of the deltas in
+// the lane, places the blocks with one scan of the block sums across the wave,
+// dequantizes, and stores the values through the wave's LDS buffer with 16-byte
+// stores.  Arithmetic: prefix sums of the deltas in int32 from the carry,
+// x' = (float) q * eb (ZCCL/src/ZCCLd_float.c:588-628).
 //
-// The tile sums live in the workspace's lookback status array of the parity
-// that the next lookback launch clears (the one other than its own), so the
-// two passes leave no state that a later launch must see cleared.
-__device__ __forceinline__ uint32_t* dec_sums(WsHeader* ws)
-{
-    const unsigned long long par = (__hip_atomic_load(&ws->seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 32) & 1ull;
-    return (uint32_t*) ((char*) ws + sizeof(WsHeader) + (par ^ 1ull) * ldc(&ws->capacity) * kStatusStride * 8);
-}
+// Compress has a tile's carry in a register and a sum adds its operands'; a
+// foreign stream's parse derives them: every tile's sum of deltas, scanned per
+// segment from its seed (kCarrySums below, then k_lane_carry_scan).  Decoding
+// every stream once more for those sums on each decompress, in two more
+// launches, took half the call: without them 38.9 -> 21.9 us for 2^24 values
+// (4.0 TB/s of stream and values) and 23.8 -> 11.4 us for 16 411.
 
 // The segment's seed (0 with an error when its offset is past the stream).
 __device__ __forceinline__ uint32_t segment_seed(const Geom& g, const uint8_t* bytes, const uint8_t* index,
@@ -1011,7 +1014,7 @@ struct DecPre {
     uint64_t idx;
     uint64_t goff, size;
     uint32_t wq;
-    uint32_t carry;    // pass two: the tile's carry
+    uint32_t carry;    // kValues: the tile's carry
 };
 
 struct DecLoc {
@@ -1020,9 +1023,13 @@ struct DecLoc {
     bool has, skip, staged;
 };
 
-// Issue the index reads of launch tile tg (and its carry in pass two).
-template <int Pass, typename Args>
-__device__ __forceinline__ DecPre dec_prefetch(const Args& a, uint64_t tg, const uint32_t* sums)
+// What a run over the tiles writes: their values, or (single streams) their
+// sums of deltas in the place of the index carries.
+enum DecMode : int { kValues, kCarrySums };
+
+// Issue the index reads of launch tile tg.
+template <int Mode, typename Args>
+__device__ __forceinline__ DecPre dec_prefetch(const Args& a, uint64_t tg)
 {
     DecPre p;
     DecJob d;
@@ -1037,7 +1044,7 @@ __device__ __forceinline__ DecPre dec_prefetch(const Args& a, uint64_t tg, const
     p.size = iv.meta[0];
     const uint32_t lane = threadIdx.x & 63;
     p.wq = lane < x.nblk ? (uint32_t) iv.widths[x.g0 + lane] : 0u;
-    p.carry = Pass == 2 ? sums[tg] : 0u;
+    p.carry = Mode == kValues ? iv.carry[d.t] : 0u;
     return p;
 }
 
@@ -1165,26 +1172,23 @@ __device__ __forceinline__ void store_blocks(float* base, const float (&v)[L], u
     }
 }
 
-// A decompress pass over launch tiles first, first + stride, ... of one
-// wave.  Pass 1 writes each tile's sum of deltas to sums[idx]; pass 2 reads
-// the tile's carry from sums[idx] and writes its values.  Per step, tile i
-// is decoded while tile i+1's bytes move into the other LDS half and tile
-// i+2's index entries are on their way.  The lane decoders are the sum's
+// A run over launch tiles first, first + stride, ... of one wave.  Per step,
+// tile i is decoded while tile i+1's bytes move into the other LDS half and
+// tile i+2's index entries are on their way.  The lane decoders are the sum's
 // (whole blocks below width 16 that the reads covered take the fast one, the
 // rest the general one; a lane that does not use the fast decoder runs it at
 // width 0, which adds zeros).
-template <int Pass, typename Args>
+template <int Mode, typename Args>
 __device__ __forceinline__ void dec_run(const Args& a, WsHeader* ws, uint64_t first, uint64_t stride, uint32_t* obuf)
 {
     const uint32_t lane = threadIdx.x & 63;
-    uint32_t* sums = dec_sums(ws);
     bool bad_width = false, bad_byte = false, bad_over = false;
-    DecPre pc = dec_prefetch<Pass>(a, first, sums);
+    DecPre pc = dec_prefetch<Mode>(a, first);
     if (!pc.ok)
         return;
     __builtin_amdgcn_s_waitcnt(0);
     DecLoc cc = dec_locate(a, pc, obuf, 0, bad_width);
-    DecPre pn = dec_prefetch<Pass>(a, first + stride, sums);
+    DecPre pn = dec_prefetch<Mode>(a, first + stride);
     for (uint32_t half = 0;; half ^= 1u) {
         __builtin_amdgcn_s_waitcnt(0);  // tile i's bytes in LDS, tile i+1's index entries in registers
         Block q;
@@ -1201,7 +1205,7 @@ __device__ __forceinline__ void dec_run(const Args& a, WsHeader* ws, uint64_t fi
         pnn.ok = false;
         if (pn.ok) {
             cn = dec_locate(a, pn, obuf, half ^ 1u, bad_width);
-            pnn = dec_prefetch<Pass>(a, pn.idx + stride, sums);
+            pnn = dec_prefetch<Mode>(a, pn.idx + stride);
         }
         __builtin_amdgcn_sched_barrier(0);
         const bool fast = !cc.has || cc.w == 0 || (cc.nj == L && cc.w < 16 && (cc.staged || cc.o + cc.bs + 3 <= cc.lim));
@@ -1210,7 +1214,7 @@ __device__ __forceinline__ void dec_run(const Args& a, WsHeader* ws, uint64_t fi
         bad_over |= cc.skip;
         q.w = use ? cc.w : 0u;
         const bool gen = !fast && !cc.skip;
-        if constexpr (Pass == 1) {
+        if constexpr (Mode == kCarrySums) {
             // the block's sum only (a lane on the fast path has nj = L or
             // adds zeros; the general decoder adds garbage past nj)
             uint32_t part[2] = {0u, 0u};
@@ -1229,8 +1233,11 @@ __device__ __forceinline__ void dec_run(const Args& a, WsHeader* ws, uint64_t fi
                         b += acc[j];
             }
             const uint32_t inc = wave_scan_dpp(b);
-            if (lane == 63)
-                sums[pc.idx] = inc;
+            if (lane == 63) {
+                DecJob d;
+                dec_job(a, pc.idx, d);
+                index_view(d.g, d.index).carry[d.t] = inc;
+            }
         } else {
             uint32_t acc[L];
 #pragma unroll
@@ -1249,8 +1256,7 @@ __device__ __forceinline__ void dec_run(const Args& a, WsHeader* ws, uint64_t fi
             }
             DecJob d;
             dec_job(a, pc.idx, d);
-            const Geom& g = d.g;
-            const Tile x = tile_of(g, d.tl, d.t);
+            const Tile x = tile_of(d.g, d.tl, d.t);
 #pragma unroll
             for (uint32_t j = 1; j < L; j++)
                 acc[j] += acc[j - 1];
@@ -1264,7 +1270,7 @@ __device__ __forceinline__ void dec_run(const Args& a, WsHeader* ws, uint64_t fi
             // (this tile's LDS half is free: its bytes are in registers)
             store_blocks(d.out + x.e0, vals, cc.nj, x.nblk, obuf + half * (kStageHalf / 4));
             if (lane == 0 && x.lt == 0)
-                d.out[x.seg_a] = dequant(segment_seed(g, d.bytes, d.index, x.s, ws), eb);
+                d.out[x.seg_a] = dequant(pc.carry, eb);  // the segment's first value, its seed
         }
         if (!pn.ok)
             break;
@@ -1282,20 +1288,19 @@ __device__ __forceinline__ void dec_run(const Args& a, WsHeader* ws, uint64_t fi
 
 // Scan of one segment's tile sums into carries (in place): the seed plus the
 // sums of the segment's earlier tiles, mod 2^32.  One workgroup.
-constexpr uint32_t kDecScanThreads = 1024;
+constexpr uint32_t kCarryScanThreads = 1024;
 
-__device__ __forceinline__ void decompress_scan_lane(const Geom& g, const Tiling& tl, const uint8_t* bytes,
-    const uint8_t* index, uint32_t s, uint32_t* sums, uint64_t tile0, WsHeader* ws)
+__device__ __forceinline__ void carry_scan(const Geom& g, const uint8_t* bytes, const uint8_t* index, uint32_t s,
+    WsHeader* ws)
 {
-    __shared__ uint32_t s_w[kDecScanThreads / 64];
+    __shared__ uint32_t s_w[kCarryScanThreads / 64];
     __shared__ uint32_t s_seed;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const uint32_t first = s < g.T ? s * tl.tilesT : g.T * tl.tilesT;
-    const uint32_t cnt = s < g.T ? tl.tilesT : tl.tilesR;
+    const uint32_t cnt = s < g.T ? g.cT : g.cR;
     if (tid == 0)
         s_seed = segment_seed(g, bytes, index, s, ws);
-    uint32_t* p = sums + tile0 + first;
-    const uint32_t per = (cnt + kDecScanThreads - 1) / kDecScanThreads;
+    uint32_t* p = index_view(g, index).carry + (s < g.T ? s * g.cT : g.T * g.cT);
+    const uint32_t per = (cnt + kCarryScanThreads - 1) / kCarryScanThreads;
     const uint32_t a = min(tid * per, cnt), b = min(a + per, cnt);
     uint32_t run = 0;
     for (uint32_t i = a; i < b; i++)
@@ -1370,9 +1375,10 @@ __device__ __forceinline__ void compress_tile_lane(const Geom& g, const Tiling& 
     // quantize, deltas, signs and magnitudes (values past nj are zero)
     const float* xv = reinterpret_cast<const float*>(obuf) + lane * L;
     uint32_t m[L];
-    uint32_t s = 0, s2 = 0, mx = 0;
+    uint32_t s = 0, s2 = 0, mx = 0, before;
     {
         uint32_t prev = (uint32_t) quant(xv[0], inv);
+        before = prev;
 #pragma unroll
         for (uint32_t j = 0; j < L; j++) {
             const uint32_t q = (uint32_t) quant(xv[j + 1], inv);
@@ -1431,6 +1437,9 @@ __device__ __forceinline__ void compress_tile_lane(const Geom& g, const Tiling& 
     else if (threadIdx.x == 0)
         raise_error(ws, ZK_ERR_NOSPACE);
     IndexView ox = index_view(g, oindex);
+    const uint32_t ct = (x.s < g.T ? x.s * g.cT : g.T * g.cT) + kLaneWaves * x.lt + wv;  // the wave's lane tile
+    if (lane == 0 && nbw)
+        ox.carry[ct] = before;
     if (has)
         ox.widths[x.g0 + jb] = (uint8_t) w;
     if (has && (jb % g.IG) == 0)
@@ -1440,6 +1449,8 @@ __device__ __forceinline__ void compress_tile_lane(const Geom& g, const Tiling& 
             ox.group_off[x.grp0] = P;  // a segment of its seed alone keeps one group entry
         if (x.lt == 0) {
             const uint32_t seed = (uint32_t) quant(xin[x.seg_a], inv);
+            if (x.nblk == 0)
+                ox.carry[ct] = seed;
             const uint64_t so = P - 4;
             if (so + 4 <= out_cap) {
                 store_bytes(out + so, &seed, 4);
@@ -1539,13 +1550,13 @@ __global__ void __launch_bounds__(64 * kLaneWaves, 4) k_homsum_lane_mixed(BatchA
         ldc(&job->io.size_out), t, status + tile0 * kStatusStride, b.ws, b.total_chains, zk_lds + wv * (kOutBuf / 4));
 }
 
-// The two passes: a persistent grid, wave w of workgroup b starting at launch
-// tile 4b + w and striding by the grid's waves.
-template <int Pass, typename Args>
-__device__ __forceinline__ void dec_pass(const Args& a, WsHeader* ws)
+// A persistent grid, wave w of workgroup b starting at launch tile 4b + w and
+// striding by the grid's waves.
+template <int Mode, typename Args>
+__device__ __forceinline__ void dec_grid(const Args& a, WsHeader* ws)
 {
     const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    dec_run<Pass>(a, ws, (uint64_t) blockIdx.x * kLaneWaves + wv, (uint64_t) gridDim.x * kLaneWaves,
+    dec_run<Mode>(a, ws, (uint64_t) blockIdx.x * kLaneWaves + wv, (uint64_t) gridDim.x * kLaneWaves,
         zk_lds + wv * (kOutBuf / 4));
 }
 
@@ -1553,21 +1564,25 @@ __device__ __forceinline__ void dec_pass(const Args& a, WsHeader* ws)
 constexpr uint32_t kDecGroupsPerCU = 5;
 static_assert(kDecGroupsPerCU == (uint32_t) kDecGroupsMax, "the launch bound is the grid's limit");
 
-__global__ void __launch_bounds__(64 * kLaneWaves, kDecGroupsPerCU) k_decompress_lane_sums(DecompressArgs a)
+__global__ void __launch_bounds__(64 * kLaneWaves, kDecGroupsPerCU) k_decompress_lane(DecompressArgs a)
 {
-    dec_pass<1>(a, a.ws);
+    dec_grid<kValues>(a, a.ws);
 }
-__global__ void __launch_bounds__(64 * kLaneWaves, kDecGroupsPerCU) k_decompress_lane_out(DecompressArgs a)
+__global__ void __launch_bounds__(64 * kLaneWaves, kDecGroupsPerCU) k_decompress_lane_batch(BatchArgs b)
 {
-    dec_pass<2>(a, a.ws);
+    dec_grid<kValues>(b, b.ws);
 }
-__global__ void __launch_bounds__(64 * kLaneWaves, kDecGroupsPerCU) k_decompress_lane_batch_sums(BatchArgs b)
+
+// Carries of a parsed stream (none of a corrupt one, whose size is 0).
+__global__ void __launch_bounds__(64 * kLaneWaves, kDecGroupsPerCU) k_lane_carry_sums(DecompressArgs a)
 {
-    dec_pass<1>(b, b.ws);
+    if (index_view(a.job.g, a.job.io.in[0].index).meta[0])
+        dec_grid<kCarrySums>(a, a.ws);
 }
-__global__ void __launch_bounds__(64 * kLaneWaves, kDecGroupsPerCU) k_decompress_lane_batch_out(BatchArgs b)
+__global__ void __launch_bounds__(kCarryScanThreads) k_lane_carry_scan(DecompressArgs a)
 {
-    dec_pass<2>(b, b.ws);
+    if (index_view(a.job.g, a.job.io.in[0].index).meta[0])
+        carry_scan(a.job.g, a.job.io.in[0].bytes, a.job.io.in[0].index, blockIdx.x, a.ws);
 }
 
 // Compress in the lane layout: one stream, a uniform batch (shared geometry
@@ -1630,35 +1645,6 @@ __global__ void __launch_bounds__(64 * kLaneWaves, 4) k_compress_lane_mixed(Batc
     compress_tile_lane(g, tl, ldc(&job->p.inv), ldc(&job->io.x), ldc(&job->io.out), ldc(&job->io.out_cap),
         ldc(&job->io.index), ldc(&job->io.size_out), t, status + tile0 * kStatusStride, b.ws, b.total_chains,
         zk_lds + (threadIdx.x >> 6) * (kCompBuf / 4), sh);
-}
-
-// Scans: workgroup (s, j) takes segment s of job j.
-__global__ void __launch_bounds__(kDecScanThreads) k_decompress_lane_scan(DecompressArgs a)
-{
-    if (blockIdx.x >= a.job.g.S)
-        return;
-    decompress_scan_lane(a.job.g, a.job.tl, a.job.io.in[0].bytes, a.job.io.in[0].index, blockIdx.x, dec_sums(a.ws), 0,
-        a.ws);
-}
-
-__global__ void __launch_bounds__(kDecScanThreads) k_decompress_lane_batch_scan(BatchArgs b)
-{
-    const uint32_t j = blockIdx.y;
-    if (b.uniform) {
-        if (blockIdx.x >= b.g.S)
-            return;
-        const DecompressIO* io = (const DecompressIO*) b.jobs + j;
-        decompress_scan_lane(b.g, b.tl, ldc(&io->in[0].bytes), ldc(&io->in[0].index), blockIdx.x, dec_sums(b.ws),
-            (uint64_t) j * b.tl.ntiles, b.ws);
-    } else {
-        const DecompressJob* job = (const DecompressJob*) b.jobs + j;
-        const Geom g = job->g;
-        if (blockIdx.x >= g.S)
-            return;
-        const Tiling tl = job->tl;
-        decompress_scan_lane(g, tl, ldc(&job->io.in[0].bytes), ldc(&job->io.in[0].index), blockIdx.x, dec_sums(b.ws),
-            ldc(&b.job_tile0[j]), b.ws);
-    }
 }
 
 // Single-pass sum with a lookback tile per workgroup (layout 2): the
@@ -2033,7 +2019,7 @@ uint32_t device_cu_count()
     return (uint32_t) n;
 }
 
-// Workgroups of a persistent decompress pass: the tuned number per CU (at
+// Workgroups of a persistent decompress grid: the tuned number per CU (at
 // most as many as the device holds at once), or one per four tiles when that
 // is fewer.
 static uint32_t dec_groups(uint64_t tiles)
@@ -2043,19 +2029,21 @@ static uint32_t dec_groups(uint64_t tiles)
 
 hipError_t launch_decompress_lane(const DecompressArgs& a, hipStream_t s)
 {
-    const dim3 grid(dec_groups(a.job.tl.ntiles)), block(64 * kLaneWaves);
-    hipLaunchKernelGGL(k_decompress_lane_sums, grid, block, lane_lds_bytes(), s, a);
-    hipLaunchKernelGGL(k_decompress_lane_scan, dim3(a.job.g.S), dim3(kDecScanThreads), 0, s, a);
-    hipLaunchKernelGGL(k_decompress_lane_out, grid, block, lane_lds_bytes(), s, a);
+    hipLaunchKernelGGL(k_decompress_lane, dim3(dec_groups(a.job.tl.ntiles)), dim3(64 * kLaneWaves), lane_lds_bytes(), s, a);
     return hipGetLastError();
 }
 
 hipError_t launch_decompress_lane_batch(const BatchArgs& b, hipStream_t s)
 {
-    const dim3 grid(dec_groups(b.total_tiles)), block(64 * kLaneWaves);
-    hipLaunchKernelGGL(k_decompress_lane_batch_sums, grid, block, lane_lds_bytes(), s, b);
-    hipLaunchKernelGGL(k_decompress_lane_batch_scan, dim3(b.max_segments, b.njobs), dim3(kDecScanThreads), 0, s, b);
-    hipLaunchKernelGGL(k_decompress_lane_batch_out, grid, block, lane_lds_bytes(), s, b);
+    hipLaunchKernelGGL(k_decompress_lane_batch, dim3(dec_groups(b.total_tiles)), dim3(64 * kLaneWaves), lane_lds_bytes(),
+        s, b);
+    return hipGetLastError();
+}
+
+hipError_t launch_lane_carries(const DecompressArgs& a, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_lane_carry_sums, dim3(dec_groups(a.job.tl.ntiles)), dim3(64 * kLaneWaves), lane_lds_bytes(), s, a);
+    hipLaunchKernelGGL(k_lane_carry_scan, dim3(a.job.g.S), dim3(kCarryScanThreads), 0, s, a);
     return hipGetLastError();
 }
 
