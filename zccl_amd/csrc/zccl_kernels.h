@@ -222,7 +222,8 @@ hipError_t launch_decompress_lane(const DecompressArgs& a, hipStream_t s);
 hipError_t launch_lane_carries(const DecompressArgs& a, hipStream_t s);
 hipError_t launch_decompress_lane_batch(const BatchArgs& b, hipStream_t s);
 // Workgroups per CU of the persistent lane decompress grid (1 ..
-// kDecGroupsMax; 0 restores the default, 4).
+// kDecGroupsMax, a fifth waiting for the LDS of another; 0 restores the
+// default, 4).
 constexpr int kDecGroupsMax = 5;
 bool set_decompress_groups_per_cu(int groups);
 int get_decompress_groups_per_cu();

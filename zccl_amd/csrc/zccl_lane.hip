@@ -3,13 +3,13 @@
 // jobs/*.sh): the fused homomorphic sum.
 //
 // Layout.  A wave owns one tile of 64 consecutive blocks of one segment and
-// every lane owns one whole block.  For each operand a lane reads its block's
-// bytes straight from HBM into registers with range-checked buffer loads (a
-// read past the operand's stream returns zeros, so no read ever leaves the
-// stream), decodes its 36 deltas and adds them in int32.  No LDS staging and
-// no workgroup barrier sit on this path: the only per-operand cross-lane step
-// is one DPP scan of block sizes that places each lane's block.  The next
-// operand's loads are in flight while the current one is decoded.
+// every lane owns one whole block.  An operand's tile bytes move into the
+// wave's LDS buffer with range-checked direct-to-LDS loads (a read past the
+// operand's stream returns zeros, so no read ever leaves the stream) and each
+// lane reads its block with aligned dword reads, decodes its 36 deltas and adds
+// them in int32.  No workgroup barrier sits on this path: the only per-operand
+// cross-lane step is one DPP scan of block sizes that places each lane's block.
+// The next operand's loads are in flight while the current one is decoded.
 //
 // Each wave is a tile of the decoupled lookback; a workgroup of four waves
 // takes one ticket for four consecutive tiles.  The summed block is
@@ -18,8 +18,15 @@
 // neighbour's bytes, so overlapping writes need no ordering) and leaves with
 // 16-byte stores.
 //
-// Blocks of width 16 and more, and a segment's last (short) block, take a
-// per-unit path with the same arithmetic.
+// A segment's short last block takes the same path as a whole one (its fields
+// are placed by its length).  Blocks of width 16 and more, and tiles larger
+// than half the buffer, take passes of their own through the whole buffer.
+// Measured against one decoder for whole blocks below width 16 with the others
+// read value by value from memory, and an FP64 quantizer: two 1 MB operands
+// 15.8 -> 13.8 us, sixteen 8 MB ones 60 -> 31 us, 8 sums of 8 x 2^24 values
+// 458 -> 421 us, the allreduce of velocities (widths 15 to 17) 383 -> 241 us,
+// compress of 2^24 values 50.6 -> 48.2 us, decompress of 16411 values (a short
+// block in every tile) 11.4 -> 8.7 us.
 //
 // Wire format and arithmetic (reference):
 //   block      width byte, sign bitmap MSB first, (w>>3) high bytes per
@@ -45,16 +52,19 @@ namespace {
 
 constexpr uint32_t L = kLaneL;          // values per block
 constexpr uint32_t SB = (L + 7) / 8;    // sign bytes of a whole block
-constexpr uint32_t HEADW = 11;          // dwords of bytes [0, 44): width, signs, 36 high bytes
+constexpr uint32_t NHI = L / 4;         // dwords of one high byte per value
 constexpr uint32_t NGRP = (L + 7) / 8;  // groups of (up to) 8 values in the low bits
 constexpr uint32_t kWorstBlock = 1 + SB + 4 * L;   // 150 bytes at width 32
-// Output buffer of one wave: 8 KB, so that five workgroups of four waves
-// share a CU's 160 KB of LDS.  A tile's bytes plus the reach of the
-// OR-writes past a block's end (at most 48 bytes) fit unless the tile is
-// wide (the worst tile is 64 blocks of kWorstBlock bytes); such a tile is
-// encoded half a wave at a time, and a half always fits.
-constexpr uint32_t kOutBuf = 8192;
-static_assert(kLaneTileBlocks / 2 * kWorstBlock + 64 <= kOutBuf, "half a worst-case tile fits a wave buffer");
+// Output buffer of one wave: 10 KB, so that four workgroups of four waves
+// share a CU's 160 KB of LDS (the sum's loop holds 108 registers, more than the
+// 96 that five would leave a wave).  The worst tile's bytes (64 blocks of
+// kWorstBlock) fit, with the reach of the block reads and OR-writes past them.
+constexpr uint32_t kOutBuf = 10240;
+// Block reads and writes cover 36 values whatever the block holds: a short
+// last block's reach at most 6 + 4 * 37 bytes past its first byte.
+constexpr uint32_t kReach = 160;
+static_assert(kReach >= 1 + SB + 4 * (L + 1), "the reach of a short block's reads and writes");
+static_assert(kLaneTileBlocks * kWorstBlock + 16 + kReach <= kOutBuf, "a worst-case tile fits a wave buffer");
 static_assert(kOutBuf % 16 == 0, "wave buffers stay 16-byte aligned");
 
 static_assert(L % 4 == 0 && L > 32 && L <= 40, "the lane decoder is laid out for 36-value blocks");
@@ -78,9 +88,6 @@ __device__ __forceinline__ uint32_t lane_block_bytes(uint32_t w, uint32_t n)
     return w ? 1u + ((n + 7u) >> 3) + mad_u24(w >> 3, n, (mad_u24(w & 7u, n, 7u) >> 3)) : 1u;
 }
 
-// (w >> 3) * L, the high bytes of a block, for w <= 32.
-__device__ __forceinline__ uint32_t high_bytes(uint32_t w) { return mad_u24(w >> 3, L, 0u); }
-
 using View = __amdgpu_buffer_rsrc_t;
 // Four floats at 4-byte alignment (one 16-byte store where the address is
 // only dword aligned).
@@ -97,38 +104,18 @@ __device__ __forceinline__ View make_view(const uint8_t* base, uint64_t bytes)
     return __builtin_amdgcn_make_buffer_rsrc((void*) base, (short) 0, (int) n, 0x00020000);
 }
 
-__device__ __forceinline__ uint32_t bl4(View v, uint32_t off) { return __builtin_amdgcn_raw_buffer_load_b32(v, off, 0, 0); }
-
-__device__ __forceinline__ uint2 bl8(View v, uint32_t off)
-{
-    const auto x = __builtin_amdgcn_raw_buffer_load_b64(v, off, 0, 0);
-    return make_uint2(x[0], x[1]);
-}
-
-__device__ __forceinline__ uint3 bl12(View v, uint32_t off)
-{
-    const auto x = __builtin_amdgcn_raw_buffer_load_b96(v, off, 0, 0);
-    return make_uint3(x[0], x[1], x[2]);
-}
-
 __device__ __forceinline__ uint4 bl16(View v, uint32_t off)
 {
     const auto x = __builtin_amdgcn_raw_buffer_load_b128(v, off, 0, 0);
     return make_uint4(x[0], x[1], x[2], x[3]);
 }
 
-// 4 / 8 bytes from any offset through aligned dword loads only, so every
-// byte inside the view reads as itself (up to its very end).
-__device__ __forceinline__ uint32_t bl4a(View v, uint32_t off)
+// A value that every lane holds, in scalar registers.
+__device__ __forceinline__ uint64_t uniform64(uint64_t v)
 {
-    const uint2 x = bl8(v, off & ~3u);
-    return __builtin_amdgcn_alignbyte(x.y, x.x, off);  // uses off & 3
-}
-
-__device__ __forceinline__ uint2 bl8a(View v, uint32_t off)
-{
-    const uint3 x = bl12(v, off & ~3u);
-    return make_uint2(__builtin_amdgcn_alignbyte(x.y, x.x, off), __builtin_amdgcn_alignbyte(x.z, x.y, off));
+    const uint32_t hi = (uint32_t) __builtin_amdgcn_readfirstlane((uint32_t) (v >> 32));
+    const uint32_t lo = (uint32_t) __builtin_amdgcn_readfirstlane((uint32_t) v);
+    return ((uint64_t) hi << 32) | lo;
 }
 
 // Read-only data of the launch (descriptors, input indices) through the
@@ -142,111 +129,243 @@ __device__ __forceinline__ T ldc(const T* p)
 // |d| of an int32 delta as unsigned (|INT_MIN| = 2^31).
 __device__ __forceinline__ uint32_t mag(uint32_t d) { return (uint32_t) max((int32_t) d, (int32_t) (0u - d)); }
 
-// One operand's block of this lane, loaded: bytes [0, 44) of the block (width
-// byte, sign bytes, the high bytes of a width below 16) and, for each group
-// of 8 values, the 8 bytes from the group's first byte of low bits as two
-// big-endian words.
-struct Block {
-    uint32_t h[HEADW];
-    uint32_t ge[2 * NGRP];
-    uint32_t w;   // index width (0..32)
-    uint32_t o;   // offset of the block in the operand's view
-    uint32_t lim; // length of the operand's view (the same for the wave)
-    bool fast;    // decode_fast serves this lane (else the general decoder, if w > 0)
-};
+// Integers below 2^24 as FP32 bit patterns: a denormal's bits are its integer
+// (in units of 2^-149), and the next binade's still are, so FP32 differences
+// and fused multiply-adds of such patterns are exact integer arithmetic on
+// sign-and-magnitude numbers.  They take half the time of the integer
+// instructions that would do the same (measured on the MI355X, cycles per
+// wave instruction and SIMD: add, subtract, multiply and fma FP32, and, or,
+// xor, v_bitop3, right shifts 2; bit-field extracts, left shifts, 24-bit
+// multiplies, v_perm, v_alignbit, min and max, conversions, FP64 4).
+__device__ __forceinline__ float as_f(uint32_t v) { return __uint_as_float(v); }
+__device__ __forceinline__ uint32_t as_u(float v) { return __float_as_uint(v); }
 
-// Add a whole block of width w < 16 to acc: magnitude = (high byte << r) |
-// low r bits, times the value's sign as +1 or -1.  A zero width adds zeros
-// whatever the bytes.  wide: some lane of the wave has w >= 8 (otherwise no
-// lane has high bytes and they are not extracted).
-// ZCCL/src/ZCCL_TypeManager.c:423-517 (extract), :906-950 (signs).
+// v, computed here: without this the compiler moves what a group of values
+// gives behind the branches of the groups after it (or what only a block's
+// width gives ahead of a loop), and holds registers for all 36 values.
+template <typename T>
+__device__ __forceinline__ T stay(T v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
 // a * b + c for a, b of 24 bits (signed) and any c, in one instruction.
 __device__ __forceinline__ uint32_t mad_i24(uint32_t a, uint32_t b, uint32_t c)
 {
     uint32_t d;
-    asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
+    asm volatile("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
     return d;
 }
 
-// N < L: only the sum of the block's values is wanted; value j is added to
-// acc[j % N] (N short chains of adds instead of L values to add up).
-template <bool wide, uint32_t N = L>
-__device__ __forceinline__ void decode_fast(const Block& q, uint32_t (&acc)[N])
+// Four bytes from any byte offset o of LDS words st (aligned dword reads: a
+// misaligned LDS read takes 30 times as long), in memory order and as a
+// big-endian word.
+__device__ __forceinline__ uint32_t lds_at(const uint32_t* st, uint32_t o)
 {
-    const uint32_t r = q.w & 7, hb = q.w & 8;  // hb: bits per high byte (0 or 8)
-    const uint32_t s0 = __builtin_amdgcn_alignbyte(q.h[1], q.h[0], 1);  // sign bytes 0..3, memory order
-    const uint32_t s1 = q.h[1] >> 8;                                   // sign byte 4 in bits 7..0
+    const uint32_t* p = st + (o >> 2);
+    return __builtin_amdgcn_alignbyte(p[1], p[0], o);  // uses o & 3
+}
+
+// A lane's block in registers: the sign words (value j at bit 31 - j, value
+// 32 + j of s2 likewise), the big-endian dwords at the first byte of each
+// group of 8 values' low bits, and, where some lane of the wave has a width
+// in [8, 16), one high byte per value.
+struct Block {
+    uint32_t s, s2;
+    uint32_t ge[2 * NGRP];
+    uint32_t hi[NHI];
+};
+
+// Read a block of nj <= L values and width w < 16 from tile bytes in LDS (the
+// block at byte o of st): a short block's fields are placed by nj like a
+// whole one's, so both take this path; values past nj read what follows.
+// wide: some lane of the wave has w >= 8 (uniform).
+__device__ __forceinline__ void read_block(const uint32_t* st, uint32_t o, uint32_t w, uint32_t nj, bool wide, Block& q)
+{
+    const uint32_t* p = st + (o >> 2);
+    const uint32_t x0 = __builtin_amdgcn_alignbyte(p[1], p[0], o), x1 = __builtin_amdgcn_alignbyte(p[2], p[1], o);
+    q.s = __builtin_amdgcn_perm(x1, x0, 0x01020304u);  // sign bytes 0..3 big-endian
+    q.s2 = x1 << 16;                                   // sign byte 4 on top
+    const uint32_t hp = o + 1 + ((nj + 7) >> 3);
+    uint32_t a = hp, r = w;
+    if (wide) {
+        const uint32_t* ph = st + (hp >> 2);
+        uint32_t d = ph[0];
+#pragma unroll
+        for (uint32_t i = 0; i < NHI; i++) {
+            const uint32_t e = ph[i + 1];
+            q.hi[i] = __builtin_amdgcn_alignbyte(e, d, hp);
+            d = e;
+        }
+        a += w & 8 ? nj : 0u;
+        r = w & 7;
+    }
+#pragma unroll
+    for (uint32_t g = 0; g < NGRP; g++, a += r) {
+        const uint32_t* pg = st + (a >> 2);
+        const uint32_t E0 = pg[0], E1 = pg[1], E2 = pg[2];
+        q.ge[2 * g] = __builtin_bswap32(__builtin_amdgcn_alignbyte(E1, E0, a));
+        q.ge[2 * g + 1] = __builtin_bswap32(__builtin_amdgcn_alignbyte(E2, E1, a));
+    }
+}
+
+// The values of a block of width w < 16: f(j, magnitude, +1 or -1).  A zero
+// width gives zeros whatever was read.  wide (uniform): the high bytes were
+// read; they join the low bits group by group behind a branch of their own, so
+// tiles without any skip them and the decoder stays one piece of code (two
+// whole decoders behind one branch cost the sum 10 to 36 spilled registers per
+// operand).  Three instructions per value and the sum's multiply-add: a
+// bit-field extract at one of four places of the half group's window, another
+// for the sign.  (Shifts, masks and FP32 adds that take 2 cycles each in their
+// place were five instructions and slower: the sum issues, it does not wait for
+// the units.)
+// ZCCL/src/ZCCL_TypeManager.c:423-517 (extract), :906-950 (signs).
+template <typename F>
+__device__ __forceinline__ void each_value(const Block& q, uint32_t w, bool wide, F f)
+{
+    const uint32_t r = w & 7, hb = w & 8;  // hb: bits per high byte (0 or 8)
+    const uint32_t sh[4] = {32 - r, 32 - 2 * r, 32 - 3 * r, 32 - 4 * r};
     // Sign words: a value's sign bit moved to an odd bit with a one below it,
-    // so the 2-bit field there reads -1 (sign set) or +1 as a signed number.
-    // so0/so1 hold the values whose bit is odd in s0/s1, se0/se1 (shifted up
-    // one) the values whose bit is even.
-    uint32_t so0 = (s0 & 0xAAAAAAAAu) | 0x55555555u, se0 = ((s0 << 1) & 0xAAAAAAAAu) | 0x55555555u;
-    uint32_t so1 = (s1 & 0xAAu) | 0x55u, se1 = ((s1 << 1) & 0xAAu) | 0x55u;
+    // so the 2-bit field there reads -1 (sign set) or +1 as a signed number:
+    // so the even values, se (shifted up one) the odd ones.
+    uint32_t so = (q.s & 0xAAAAAAAAu) | 0x55555555u, se = ((q.s << 1) & 0xAAAAAAAAu) | 0x55555555u;
+    uint32_t so2 = (q.s2 & 0xAAAAAAAAu) | 0x55555555u, se2 = ((q.s2 << 1) & 0xAAAAAAAAu) | 0x55555555u;
     // (opaque to the optimiser, which would otherwise extract the sign bit
     // alone and OR in the one: two instructions per value instead of one)
-    asm volatile("" : "+v"(so0), "+v"(se0), "+v"(so1), "+v"(se1));
+    asm volatile("" : "+v"(so), "+v"(se), "+v"(so2), "+v"(se2));
 #pragma unroll
-    for (uint32_t p = 0; p < NGRP; p++) {
-        // the group's low bits big-endian: value 8p+c's field is r bits from bit 64 - (c+1) r
-        const uint32_t e0 = q.ge[2 * p], e1 = q.ge[2 * p + 1];
-        uint32_t gh = e0;
+    for (uint32_t g = 0; g < NGRP; g++) {
+        __builtin_amdgcn_sched_barrier(0);  // group by group: few registers live
+        const uint32_t n = 8 * g + 8 <= L ? 8u : L - 8 * g;
+        // the group's low bits big-endian: value 8g + c's field is r bits from
+        // bit 64 - (c+1) r; value 4's window is bits 4r.. of the two dwords
+        // (any value when r = 0)
+        uint32_t m[8];
 #pragma unroll
-        for (uint32_t c = 0; c < 8; c++) {
-            const uint32_t j = 8 * p + c;
-            if (j >= L)
-                break;
-            if (c == 4)  // the window of value 4: bits 4r.. of e0:e1 (any value when r = 0)
-                gh = __builtin_amdgcn_alignbit(e0, e1, 32 - 4 * r);
-            const uint32_t hbyte = wide ? __builtin_amdgcn_ubfe(q.h[(6 + j) >> 2], 8 * ((6 + j) & 3), hb) : 0u;
-            // {high byte, window} << r: the magnitude (< 2^15) in the upper
-            // dword, the next value's window in the lower one
-            const uint64_t v = (((uint64_t) hbyte << 32) | gh) << r;
-            const uint32_t m = (uint32_t) (v >> 32);
-            gh = (uint32_t) v;
-            const uint32_t bit = j < 32 ? 8 * (j >> 3) + 7 - (j & 7) : 7 - (j - 32);
-            const uint32_t sw = j < 32 ? ((bit & 1) ? so0 : se0) : ((bit & 1) ? so1 : se1);
-            const int32_t f = __builtin_amdgcn_sbfe((int32_t) sw, bit & ~1u, 2);
-            acc[j % N] = mad_i24(m, (uint32_t) f, acc[j % N]);
+        for (uint32_t c = 0; c < n; c++) {
+            const uint32_t win =
+                c < 4 ? q.ge[2 * g] : __builtin_amdgcn_alignbit(q.ge[2 * g], q.ge[2 * g + 1], sh[3]);
+            m[c] = __builtin_amdgcn_ubfe(win, sh[c & 3], r);
+        }
+        if (wide) {
+#pragma unroll
+            for (uint32_t c = 0; c < n; c++)
+                m[c] |= __builtin_amdgcn_ubfe(q.hi[2 * g + (c >> 2)], 8 * (c & 3), hb) << r;
+        }
+#pragma unroll
+        for (uint32_t c = 0; c < n; c++) {
+            const uint32_t j = 8 * g + c, i = j & 31;
+            const uint32_t sw = j < 32 ? ((i & 1) ? se : so) : ((i & 1) ? se2 : so2);
+            f(j, m[c], (uint32_t) __builtin_amdgcn_sbfe((int32_t) sw, (31 - i) & ~1u, 2));
         }
     }
 }
 
-// Add a block of any width (nj values, nj <= L) unit by unit; values past nj
-// add garbage that the caller clears.  Same fields as decode_fast; aligned
-// loads only (this path also serves blocks that end in the view's last
-// dword), each value's high bytes with a load of their own.  Branch-free and
-// one unit's loads at a time: this path is rare and must not raise the
-// kernel's register count.  Returns whether the block's width byte differs
-// from w.
-__device__ __forceinline__ bool decode_general(View v, uint32_t o, uint32_t w, uint32_t nj, uint32_t (&acc)[L])
+// The same for widths with B = w >> 3 = 2, 3 or 4 high bytes per value (lanes
+// of that class only), straight from LDS: f(j, magnitude, sign word whose bit
+// 31 is the value's sign).
+template <uint32_t B, typename F>
+__device__ __forceinline__ void each_value_high(const uint32_t* st, uint32_t o, uint32_t w, uint32_t nj, F f)
 {
-    const uint32_t B = w >> 3, r = w & 7, nsb = (nj + 7) >> 3;
+    static_assert(B >= 2 && B <= 4, "high bytes of a width from 16");
+    const uint32_t r = w & 7, mask = (1u << r) - 1u;
+    const uint32_t hp = o + 1 + ((nj + 7) >> 3);
+    const uint32_t sh[4] = {32 - r, 32 - 2 * r, 32 - 3 * r, 32 - 4 * r};
+    uint32_t s = __builtin_bswap32(lds_at(st, o + 1)), s2 = lds_at(st, o + 5) << 24;
+    const uint32_t* ph = st + (hp >> 2);
+    uint32_t a = hp + B * nj;
+#pragma unroll
+    for (uint32_t g = 0; g < NGRP; g++, a += r) {
+        __builtin_amdgcn_sched_barrier(0);  // group by group: few registers live
+        const uint32_t n = 8 * g + 8 <= L ? 8u : L - 8 * g;
+        const uint32_t* pg = st + (a >> 2);
+        const uint32_t E0 = pg[0], E1 = pg[1], E2 = pg[2];
+        const uint32_t e0 = __builtin_bswap32(__builtin_amdgcn_alignbyte(E1, E0, a));
+        const uint32_t e1 = __builtin_bswap32(__builtin_amdgcn_alignbyte(E2, E1, a));
+        uint32_t h[2 * B + 1];  // the group's high bytes in memory order
+        uint32_t d = ph[2 * B * g];
+#pragma unroll
+        for (uint32_t i = 0; i < n * B / 4; i++) {
+            const uint32_t e = ph[2 * B * g + i + 1];
+            h[i] = __builtin_amdgcn_alignbyte(e, d, hp);
+            d = e;
+        }
+        h[n * B / 4] = 0;
+        uint32_t win = e0;
+#pragma unroll
+        for (uint32_t c = 0; c < n; c++) {
+            const uint32_t j = 8 * g + c;
+            if (c == 4)
+                win = __builtin_amdgcn_alignbit(e0, e1, sh[3]);
+            const uint32_t m = (win >> (sh[c & 3] & 31)) & mask;
+            uint32_t v;
+            if constexpr (B == 2)
+                v = (c & 1) ? h[c >> 1] >> 16 : h[c >> 1] & 0xFFFFu;
+            else if constexpr (B == 3)
+                v = __builtin_amdgcn_alignbyte(h[(3 * c) / 4 + 1], h[(3 * c) / 4], (3 * c) & 3) & 0xFFFFFFu;
+            else
+                v = h[c];
+            // (two high bytes and r bits are below 2^24: the denormal product)
+            const uint32_t mag = B == 2 ? as_u(__builtin_fmaf(as_f(v), as_f((127u + r) << 23), as_f(m))) : (v << r) | m;
+            if (j < 32) {
+                f(j, mag, s);
+                s += s;
+            } else {
+                f(j, mag, s2);
+                s2 += s2;
+            }
+        }
+    }
+}
+
+// Two's complement of a magnitude and a sign word (its bit 31).
+__device__ __forceinline__ uint32_t signed_of(uint32_t m, uint32_t s)
+{
+    const uint32_t t = (uint32_t) ((int32_t) s >> 31);
+    return (m ^ t) - t;
+}
+
+// Lanes of the wave whose block takes each_value_high (w >= 16, `on`), by
+// class.
+template <typename F>
+__device__ __forceinline__ void each_high_lane(const uint32_t* st, uint32_t o, uint32_t w, uint32_t nj, bool on, F f)
+{
+    if (on && (w >> 3) == 2)
+        each_value_high<2>(st, o, w, nj, f);
+    if (on && (w >> 3) == 3)
+        each_value_high<3>(st, o, w, nj, f);
+    if (on && w == 32)
+        each_value_high<4>(st, o, w, nj, f);
+}
+
+// Add a block of any width (nj values, nj <= L) from LDS to acc, four values at
+// a time; values past nj add garbage that the caller clears.  Each value's
+// high bytes are read on their own: few registers, for the sum's rare tiles.
+__device__ __forceinline__ void decode_any(const uint32_t* st, uint32_t o, uint32_t w, uint32_t nj, uint32_t (&acc)[L])
+{
+    w = stay(w);  // (or the loop around this would keep 45 offsets made from it)
+    const uint32_t B = w >> 3, r = w & 7;
     const uint32_t hmask = B >= 4 ? ~0u : (1u << (8 * B)) - 1u;
-    const uint32_t hp = o + 1 + nsb, lp = hp + B * nj;
-    const bool bad = (bl4a(v, o) & 0xFFu) != w;
-    const uint2 sg = bl8a(v, o + 1);
+    const uint32_t hp = o + 1 + ((nj + 7) >> 3), lp = hp + B * nj;
+    uint32_t s = __builtin_bswap32(lds_at(st, o + 1)), s2 = lds_at(st, o + 5) << 24;
 #pragma unroll
     for (uint32_t u = 0; u < L / 4; u++) {
         __builtin_amdgcn_sched_barrier(0);
         uint32_t H[4];
 #pragma unroll
         for (uint32_t c = 0; c < 4; c++)
-            H[c] = bl4a(v, hp + (4 * u + c) * B);
-        const uint32_t X = bl4a(v, lp + ((4 * u * r) >> 3));
-        const uint32_t sw = (u >> 1) < 4 ? sg.x : sg.y;
-        const uint32_t nib = __builtin_amdgcn_ubfe(sw, 8 * ((u >> 1) & 3) + ((u & 1) ? 0 : 4), 4);
-        uint32_t lo = __builtin_bswap32(X) << ((4 * u * r) & 4u);
+            H[c] = lds_at(st, hp + (4 * u + c) * B) & hmask;
+        uint32_t lo = __builtin_bswap32(lds_at(st, lp + ((4 * u * r) >> 3))) << ((4 * u * r) & 4u);
+        uint32_t& sw = u < 8 ? s : s2;
 #pragma unroll
         for (uint32_t c = 0; c < 4; c++) {
-            const uint32_t hs = H[c] & hmask;
-            const uint64_t x = (((uint64_t) hs << 32) | lo) << r;
-            const uint32_t m = (uint32_t) (x >> 32);
+            const uint64_t x = (((uint64_t) H[c] << 32) | lo) << r;
             lo = (uint32_t) x;
-            const uint32_t sm = (uint32_t) __builtin_amdgcn_sbfe((int32_t) nib, 3 - c, 1);
-            acc[4 * u + c] += (m ^ sm) - sm;
+            acc[4 * u + c] += signed_of((uint32_t) (x >> 32), sw);
+            sw += sw;
         }
     }
-    return bad;
 }
 
 // OR bytes into the wave's zeroed LDS buffer.
@@ -259,110 +378,110 @@ __device__ __forceinline__ void lds_or(uint32_t* p, uint32_t v)
 // 4i of a byte array placed sh bytes into the aligned grid.
 __device__ __forceinline__ uint32_t shift_sel(uint32_t sh) { return 0x07060504u - sh * 0x01010101u; }
 
-// Encode a whole block of width 0 < w < 16 at byte o of the buffer: width
-// byte, sign bitmap MSB first, one high byte per value when w >= 8, then the
-// low r bits of every magnitude as an MSB-first stream (groups of 8 values
-// fill r whole bytes).  wide: some lane of the wave has w >= 8 (otherwise
-// the high bytes are known to be absent).
-// ZCCL/src/ZCCL_TypeManager.c:12-91 (fixed-length bits), :824-848 (signs).
-// s: signs of values 0..31 (value j at bit 31 - j), s2: signs of values
-// 32..35 (value 32 at bit 3); m: magnitudes.
-__device__ __forceinline__ void encode_fast(uint32_t* ob, uint32_t o, uint32_t w, uint32_t s, uint32_t s2,
-    const uint32_t (&m)[L], bool wide)
+// OR the N dwords x (a byte array) at byte a of the buffer.
+template <uint32_t N>
+__device__ __forceinline__ void or_words(uint32_t* ob, uint32_t a, const uint32_t (&x)[N])
 {
-    const uint32_t r = w & 7, B = w >> 3;
-    const uint32_t sb = __builtin_bswap32(s);  // sign bytes 0..3 in memory order
-    // high bytes (zero when w < 8: then m < 2^r)
-    uint32_t H[L];
-#pragma unroll
-    for (uint32_t j = 0; j < L; j++)
-        H[j] = m[j] >> r;
-    uint32_t x[HEADW + 1];
-    x[0] = w | (sb << 8);
-    x[1] = (sb >> 24) | (s2 << (8 + 40 - L)) | (H[0] << 16) | (H[1] << 24);  // sign byte 4: value 32 at bit 7
-#pragma unroll
-    for (uint32_t i = 2; i < HEADW; i++) {
-        const uint32_t j = 4 * i - 6;
-        x[i] = H[j] | (j + 1 < L ? H[j + 1] << 8 : 0u) | (j + 2 < L ? H[j + 2] << 16 : 0u) |
-               (j + 3 < L ? H[j + 3] << 24 : 0u);
-    }
-    x[HEADW] = 0;
-    const uint32_t sel = shift_sel(o & 3);
-    uint32_t* p = ob + (o >> 2);
+    const uint32_t sel = shift_sel(a & 3);
+    uint32_t* p = ob + (a >> 2);
     uint32_t prev = 0;
-    const uint32_t nd = wide ? HEADW + 1 : 3;
 #pragma unroll
-    for (uint32_t i = 0; i < HEADW + 1; i++) {
-        if (i < nd)
-            lds_or(p + i, __builtin_amdgcn_perm(x[i], prev, sel));
+    for (uint32_t i = 0; i < N; i++) {
+        lds_or(p + i, __builtin_amdgcn_perm(x[i], prev, sel));
         prev = x[i];
     }
-    if (r) {
-        const uint32_t mask = (1u << r) - 1, lo0 = o + 1 + SB + B * L;
+    lds_or(p + N, __builtin_amdgcn_perm(0u, prev, sel));
+}
+
+// The high bytes (B per value) of a block of width w >= 8 at byte a.  For
+// B = 1 and 2 the bytes are put together by exact FP32 multiply-adds.
+template <uint32_t B>
+__device__ __forceinline__ void encode_high(uint32_t* ob, uint32_t a, uint32_t w, const uint32_t (&m)[L])
+{
+    const uint32_t r = w & 7;
+    uint32_t x[B * NHI];
 #pragma unroll
-        for (uint32_t g = 0; g < NGRP; g++) {
-            uint32_t ua = 0, ub = 0;
+    for (uint32_t i = 0; i < NHI; i++) {
+        uint32_t h[4];
 #pragma unroll
-            for (uint32_t c = 0; c < 4; c++) {
-                const uint32_t j = 8 * g + c;
-                ua = (ua << r) | (m[j] & mask);
-                if (j + 4 < L)
-                    ub = (ub << r) | (m[j + 4] & mask);
-            }
-            // 8 fields (the last group: 4 and zeros) = r bytes, top-aligned in Y
-            const uint64_t G = ((uint64_t) ua << (4 * r)) | ub;
-            const uint64_t Y = G << (64 - 8 * r);
-            const uint32_t z0 = __builtin_bswap32((uint32_t) (Y >> 32)), z1 = __builtin_bswap32((uint32_t) Y);
-            const uint32_t a = lo0 + g * r;
-            const uint32_t gs = shift_sel(a & 3);
-            uint32_t* q = ob + (a >> 2);
-            lds_or(q, __builtin_amdgcn_perm(z0, 0u, gs));
-            lds_or(q + 1, __builtin_amdgcn_perm(z1, z0, gs));
-            lds_or(q + 2, __builtin_amdgcn_perm(0u, z1, gs));
+        for (uint32_t c = 0; c < 4; c++)
+            h[c] = m[4 * i + c] >> r;
+        if constexpr (B == 1) {
+            const uint32_t lo = as_u(__builtin_fmaf(as_f(h[1]), 256.0f, as_f(h[0])));
+            const uint32_t hi = as_u(__builtin_fmaf(as_f(h[3]), 256.0f, as_f(h[2])));
+            x[i] = lo | (hi << 16);
+        } else if constexpr (B == 2) {
+            x[2 * i] = h[0] | (h[1] << 16);
+            x[2 * i + 1] = h[2] | (h[3] << 16);
+        } else if constexpr (B == 3) {
+            x[3 * i] = h[0] | (h[1] << 24);
+            x[3 * i + 1] = (h[1] >> 8) | (h[2] << 16);
+            x[3 * i + 2] = (h[2] >> 16) | (h[3] << 8);
+        } else {
+#pragma unroll
+            for (uint32_t c = 0; c < 4; c++)
+                x[4 * i + c] = h[c];
         }
     }
+    or_words(ob, a, x);
 }
 
-// OR the n <= 4 little-endian bytes of v at LDS byte address a (two dwords).
-__device__ __forceinline__ void or_bytes(uint32_t* ob, uint32_t a, uint32_t v)
+// Encode the blocks of the lanes with w > 0 (nj <= L values; those past nj are
+// zero) at byte o of the wave's zeroed buffer: width byte, sign bitmap MSB
+// first, (w >> 3) high bytes per value, then the low r bits of every
+// magnitude as an MSB-first stream (groups of 8 values fill r whole bytes).
+// s: signs of values 0..31 (value j at bit 31 - j), s2: signs of values
+// 32..35 (value 32 at bit 3); m: magnitudes.  The zeros past a short block's
+// values land at most kReach bytes past its start.
+// ZCCL/src/ZCCL_TypeManager.c:12-91 (fixed-length bits), :824-848 (signs).
+__device__ __forceinline__ void encode_blocks(uint32_t* ob, uint32_t o, uint32_t w, uint32_t nj, uint32_t s, uint32_t s2,
+    const uint32_t (&m)[L])
 {
-    const uint64_t x = (uint64_t) v << (8 * (a & 3));
-    uint32_t* q = ob + (a >> 2);
-    lds_or(q, (uint32_t) x);
-    lds_or(q + 1, (uint32_t) (x >> 32));
-}
-
-// Encode a block of any width w > 0 with 0 < nj <= L values (values past nj
-// are zero) by OR-writes, value by value and without branches, for the rare
-// blocks encode_fast does not take (widths from 16, a segment's short last
-// block).  Writes of the zero values past nj go to the last value's bytes
-// or at most 30 bytes past the block.  Same format and arguments as
-// encode_fast.
-__device__ __forceinline__ void encode_general(uint32_t* ob, uint32_t o, uint32_t w, uint32_t nj, uint32_t s,
-    uint32_t s2, const uint32_t (&m)[L])
-{
-    const uint32_t B = w >> 3, r = w & 7, nsb = (nj + 7) >> 3;
-    const uint32_t hmask = B >= 4 ? ~0u : (1u << (8 * B)) - 1u;
-    const uint32_t fmask = (1u << r) - 1u;
-    const uint32_t hp = o + 1 + nsb, lo0 = hp + B * nj;
-    // width byte and sign bytes (the bits of values past nj are zero, and so
-    // are the sign bytes past nsb that these dwords also cover)
-    const uint32_t sb = __builtin_bswap32(s);
-    const uint32_t x0 = w | (sb << 8), x1 = (sb >> 24) | (s2 << (8 + 40 - L));
-    const uint32_t sel = shift_sel(o & 3);
-    uint32_t* p = ob + (o >> 2);
-    lds_or(p, __builtin_amdgcn_perm(x0, 0u, sel));
-    lds_or(p + 1, __builtin_amdgcn_perm(x1, x0, sel));
-    lds_or(p + 2, __builtin_amdgcn_perm(0u, x1, sel));
+    const uint32_t hp = o + 1 + ((nj + 7) >> 3);
+    const bool wide = __any(w >= 8);
+    if (w) {
+        const uint32_t sb = __builtin_bswap32(s);  // sign bytes 0..3 in memory order
+        const uint32_t x[2] = {w | (sb << 8), (sb >> 24) | (s2 << (8 + 40 - L))};
+        or_words(ob, o, x);
+    }
+    // (the classes as separate branches: one with all of them would keep what
+    // they share live)
+    if (wide) {
+        if ((w >> 3) == 1)
+            encode_high<1>(ob, hp, w, m);
+        if (__any(w >= 16)) {
+            if ((w >> 3) == 2)
+                encode_high<2>(ob, hp, w, m);
+            if ((w >> 3) == 3)
+                encode_high<3>(ob, hp, w, m);
+            if (w == 32)
+                encode_high<4>(ob, hp, w, m);
+        }
+    }
+    const uint32_t r = w & 7;
+    if (r) {
+        const uint32_t mask = (1u << r) - 1u;
+        const float scale = as_f((127u + r) << 23);  // 2^r
+        uint32_t a = hp + (w >> 3) * nj;
 #pragma unroll
-    for (uint32_t j = 0; j < L; j++) {
-        __builtin_amdgcn_sched_barrier(0);  // value by value: few registers live
-        // high bytes: B bytes of m >> r at hp + j B (m >> r < 2^32, so width 32 has 4)
-        or_bytes(ob, hp + min(j, nj - 1) * B, (m[j] >> r) & hmask);
-        // low bits: r bits at bit j r of the MSB-first stream (a 16-bit window)
-        const uint32_t bit = j * r;
-        const uint32_t be = (m[j] & fmask) << (16 - r - (bit & 7));
-        or_bytes(ob, lo0 + (bit >> 3), ((be >> 8) & 0xFFu) | ((be & 0xFFu) << 8));
+        for (uint32_t g = 0; g < NGRP; g++, a += r) {
+            // four fields: two pairs by exact FP32 multiply-adds (14 bits at most each)
+            uint32_t u[2] = {0, 0};
+#pragma unroll
+            for (uint32_t h = 0; h < 2; h++) {
+                const uint32_t j = 8 * g + 4 * h;
+                if (j < L) {
+                    const uint32_t f0 = m[j] & mask, f1 = m[j + 1] & mask, f2 = m[j + 2] & mask, f3 = m[j + 3] & mask;
+                    u[h] = (as_u(__builtin_fmaf(as_f(f0), scale, as_f(f1))) << (2 * r)) |
+                           as_u(__builtin_fmaf(as_f(f2), scale, as_f(f3)));
+                }
+            }
+            // 8 fields (the last group: 4 and zeros) = r bytes, top-aligned in Y
+            const uint64_t G = ((uint64_t) u[0] << (4 * r)) | u[1];
+            const uint64_t Y = G << (64 - 8 * r);
+            const uint32_t z[2] = {__builtin_bswap32((uint32_t) (Y >> 32)), __builtin_bswap32((uint32_t) Y)};
+            or_words(ob, a, z);
+        }
     }
 }
 
@@ -406,51 +525,27 @@ struct ArgIO {
 
 // Staging area of one operand's tile bytes: half of the wave's output buffer
 // (the buffer is free until the encode), less the reach of the block reads
-// past the staged bytes (up to 47 bytes).
+// past the staged bytes; the whole buffer for a tile that fits no half.
 constexpr uint32_t kStageHalf = kOutBuf / 2;
-constexpr uint32_t kStageCap = kStageHalf - 64;
+constexpr uint32_t kStageCap = kStageHalf - kReach;
 static_assert(kStageHalf % 16 == 0, "stage halves stay 16-byte aligned");
 
-// A lane's block from tile bytes staged in LDS at st (offset o, index width
-// w): aligned dword reads (a misaligned LDS read is legal but slow).
-__device__ __forceinline__ void read_block_staged(const uint32_t* st, uint32_t o, uint32_t w, Block& q)
+// Move the first tot bytes of view v into LDS at st with 16-byte
+// direct-to-LDS buffer loads, 64 lanes per instruction; the view's range
+// check zero-fills past the stream.
+__device__ __forceinline__ void stage_bytes(View v, uint32_t tot, uint32_t* st)
 {
-    const uint32_t* p = st + (o >> 2);
-    uint32_t D[HEADW + 1];
-#pragma unroll
-    for (uint32_t i = 0; i < HEADW + 1; i++)
-        D[i] = p[i];
-#pragma unroll
-    for (uint32_t i = 0; i < HEADW; i++)
-        q.h[i] = __builtin_amdgcn_alignbyte(D[i + 1], D[i], o);  // uses o & 3
-    const uint32_t r = w & 7, lo = o + 1 + SB + high_bytes(w);
-    uint32_t a = lo;
-#pragma unroll
-    for (uint32_t gp = 0; gp < NGRP; gp++, a += r) {
-        const uint32_t* pg = st + (a >> 2);
-        const uint32_t E0 = pg[0], E1 = pg[1], E2 = pg[2];
-        // the big-endian dwords at byte a & 3 (alignbyte uses a & 3)
-        q.ge[2 * gp] = __builtin_bswap32(__builtin_amdgcn_alignbyte(E1, E0, a));
-        q.ge[2 * gp + 1] = __builtin_bswap32(__builtin_amdgcn_alignbyte(E2, E1, a));
+    const uint32_t lane = threadIdx.x & 63, nch = (tot + 15) >> 4;
+#pragma unroll 1
+    for (uint32_t run = 0; run * 64 < nch; run++) {
+        const uint32_t ch = run * 64 + lane;
+        if (ch < nch)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(v,
+                (__attribute__((address_space(3))) void*) ((uint8_t*) st + run * 1024), 16, 16 * ch, 0, 0, 0);
     }
 }
 
-// The same straight from a view, per lane (tiles too large to stage).
-__device__ __forceinline__ void read_block_direct(View v, uint32_t o, uint32_t w, Block& q)
-{
-    const uint4 h0 = bl16(v, o), h1 = bl16(v, o + 16);
-    const uint3 h2 = bl12(v, o + 32);
-    q.h[0] = h0.x; q.h[1] = h0.y; q.h[2] = h0.z; q.h[3] = h0.w;
-    q.h[4] = h1.x; q.h[5] = h1.y; q.h[6] = h1.z; q.h[7] = h1.w;
-    q.h[8] = h2.x; q.h[9] = h2.y; q.h[10] = h2.z;
-    const uint32_t r = w & 7, lo = o + 1 + SB + high_bytes(w);
-#pragma unroll
-    for (uint32_t gp = 0; gp < NGRP; gp++) {
-        const uint2 e = bl8(v, lo + gp * r);
-        q.ge[2 * gp] = __builtin_bswap32(e.x);
-        q.ge[2 * gp + 1] = __builtin_bswap32(e.y);
-    }
-}
+__device__ __forceinline__ uint32_t staged_len(uint32_t tot) { return 16 * ((tot + 15) >> 4); }
 
 // Shared state of a workgroup of lane waves that owns one lookback tile:
 // each wave's bytes, and the tile's stream offset.
@@ -552,42 +647,29 @@ __device__ __forceinline__ void homsum_tile_lane(const Geom& g, const Tiling& tl
         c.tot += delta;  // bytes of the view that hold the tile
         return c;
     };
-    // move an operand's tile bytes (view bytes [0, tot)) into LDS half `half`
-    // with 16-byte direct-to-LDS buffer loads, 64 lanes per instruction; the
-    // view's range check zero-fills past the stream.  False when they do not
-    // fit (then the blocks are read with per-lane loads).
+    // stage an operand's tile bytes into LDS half `half`; false when they do
+    // not fit there
     auto stage = [&](const Loc& c, uint32_t half) -> bool {
-        const uint32_t nch = (c.tot + 15) >> 4;
-        if (c.skip || 16 * nch > kStageCap)
+        if (c.skip || staged_len(c.tot) > kStageCap)
             return false;
-        uint8_t* st = (uint8_t*) obuf + half * kStageHalf;
-        for (uint32_t run = 0; run * 64 < nch; run++) {
-            const uint32_t ch = run * 64 + lane;
-            if (ch < nch)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(c.v, (__attribute__((address_space(3))) void*) (st + run * 1024),
-                    16, 16 * ch, 0, 0, 0);
-        }
+        stage_bytes(c.v, c.tot, obuf + half * (kStageHalf / 4));
         return true;
     };
-    auto read_staged = [&](const Loc& c, uint32_t half, Block& q) {
-        read_block_staged(obuf + half * (kStageHalf / 4), c.o, c.w, q);
-    };
-    auto read_direct = [&](const Loc& c, Block& q) { read_block_direct(c.v, c.o, c.w, q); };
 
     uint32_t acc[L];
 #pragma unroll
     for (uint32_t j = 0; j < L; j++)
         acc[j] = 0;
-    // bit r: this lane's block of operand r needs the general decoder, which
-    // runs after the pipelined loop (fewer registers live there)
-    uint32_t gen = 0;
+    // bit r (uniform): operand r's tile does not fit a half, or has a block of
+    // width 16 or more: (the rest of) it is left to the pass below
+    uint32_t whole = 0, high = 0;
 
     // ---- operand pipeline: operand r+1's tile bytes move into the other LDS
     // half while operand r is decoded, operand r+2's widths are on their way
     {
         Op on = op_of(0);
         Loc cn = locate(on, widths(on));
-        bool sn = stage(cn, 0);
+        bool hn = stage(cn, 0);
         uint32_t wq2 = 0;
         Op o2;
         if (k > 1) {
@@ -599,59 +681,80 @@ __device__ __forceinline__ void homsum_tile_lane(const Geom& g, const Tiling& tl
         carry = wave_scan_dpp(carry);
         if (lane == 63 && x.ngrp)
             index_view(g, oindex).carry[t] = carry;
-        for (int r = 0; r < k; r++) {
+        // (a loop that runs at least once: its sums then have no second life
+        // as the zeros of an empty one)
+        int r = 0;
+        do {
             const Loc c = cn;
-            const bool staged = sn;
+            const bool half = hn;
             __builtin_amdgcn_s_waitcnt(0);  // operand r's bytes are in LDS, operand r+1's widths in registers
+            // a lane of a wider block, or of a tile that is not here, decodes
+            // zeros (without a branch: one would copy the sums)
+            const uint32_t w = half && c.w < 16 ? c.w : 0u, o = half ? c.o : 0u;
+            const bool wide = __any(w >= 8);
+            const uint32_t* st = obuf + ((uint32_t) r & 1u) * (kStageHalf / 4);
+            bad_byte |= (has && half) & (((const uint8_t*) st)[o] != c.w);
             Block q;
-            q.w = c.w;
-            q.o = c.o;
-            q.lim = c.lim;
-            if (staged)
-                read_staged(c, (uint32_t) r & 1u, q);
-            else
-                read_direct(c, q);
+            read_block(st, o, w, nj, wide, q);
             // (phase fences keep the scheduler from interleaving the block
             // reads, the next operand's staging and the decode, which would
             // hold all their values at once)
             __builtin_amdgcn_sched_barrier(0);
             if (r + 1 < k) {
                 cn = locate(o2, wq2);
-                sn = stage(cn, (uint32_t) (r + 1) & 1u);
+                hn = stage(cn, (uint32_t) (r + 1) & 1u);
             }
             if (r + 2 < k) {
                 o2 = op_of(r + 2);
                 wq2 = widths(o2);
             }
             __builtin_amdgcn_sched_barrier(0);
-            // decode_fast reads a block correctly unless the per-lane loads
-            // read it and it ends in the view's last three bytes (a dword
-            // straddling the end reads as zero); such a block, a wide one or
-            // a short one goes to the general decoder.  Zero-width and empty
-            // lanes add nothing either way.  Branch-free: a lane that does
-            // not use the fast decoder runs it at width 0, which adds zeros.
             bad_over |= c.skip;
-            const bool fast = !has || q.w == 0 || (nj == L && q.w < 16 && (staged || q.o + c.bs + 3 <= q.lim));
-            const bool use = fast && !c.skip;
-            if (!fast && !c.skip)
-                gen |= 1u << r;
-            // (a zero-width block in the view's last three bytes is not
-            // checked when read per lane: its first dword reads as zero)
-            bad_byte |= use && has && (q.w || staged || q.o + 4 <= q.lim) && (q.h[0] & 0xFFu) != q.w;
-            q.w = use ? q.w : 0u;
-            decode_fast<true>(q, acc);
-        }
+            whole |= !half && !c.skip ? 1u << r : 0u;
+            high |= half && __any(c.w >= 16) ? 1u << r : 0u;
+            each_value(q, w, wide, [&](uint32_t j, uint32_t v, uint32_t sign) { acc[j] = mad_i24(v, sign, acc[j]); });
+        } while (++r < k);
     }
-    if (__any(gen)) {
-        for (int r = 0; r < k; r++) {
-            if (!__any((gen >> r) & 1u))
-                continue;
-            const Op o = op_of(r);
-            const Loc c = locate(o, widths(o));
-            if ((gen >> r) & 1u)
-                bad_byte |= decode_general(c.v, c.o, c.w, nj, acc);
-        }
+    // the operands left over, one at a time through the whole buffer
+    for (uint32_t left = whole | high; __builtin_expect(left != 0, 0); left &= left - 1) {
+        const int r = __builtin_ctz(left);
+        const Op op = op_of(r);
+        const Loc c = locate(op, widths(op));
+        const bool all = (whole >> r) & 1u;
+        stage_bytes(c.v, c.tot, obuf);
+        __builtin_amdgcn_s_waitcnt(0);
+        const bool mine = has && (all || c.w >= 16);
+        bad_byte |= mine & (((const uint8_t*) obuf)[c.o] != c.w);
+        if (mine && c.w)
+            decode_any(obuf, c.o, c.w, nj, acc);
     }
+    if (__any(nj < L)) {
+        // values past a short block's end decoded what follows it
+#pragma unroll
+        for (uint32_t j = 0; j < L; j++)
+            if (j >= nj)
+                acc[j] = 0;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // signs (s: value j at bit 31 - j; s2: value 35 at bit 0), then the
+    // magnitudes in place of the sums
+    uint32_t s = 0, s2 = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < L; j++) {
+        if (j < 32)
+            s = __builtin_amdgcn_alignbit(s, acc[j], 31);  // (s << 1) | sign of value j
+        else
+            s2 = __builtin_amdgcn_alignbit(s2, acc[j], 31);
+    }
+    // (phase fence: without it the scheduler computes the magnitudes before
+    // the sign words and keeps both arrays live)
+    __builtin_amdgcn_sched_barrier(0);
+    uint32_t (&m)[L] = acc;
+#pragma unroll
+    for (uint32_t j = 0; j < L; j++)
+        m[j] = mag(m[j]);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_sched_barrier(0);
     if (__any(bad_width) && lane == 0)
         raise_error(ws, ZK_ERR_WIDTH);
     if (__any(bad_byte) && lane == 0)
@@ -674,31 +777,11 @@ __device__ __forceinline__ void homsum_tile_lane(const Geom& g, const Tiling& tl
         seed = (uint32_t) wave_sum64(sv);
     }
 
-    // ---- output: widths, sizes, offsets
-    if (nj < L) {
-#pragma unroll
-        for (uint32_t j = 0; j < L; j++)
-            if (j >= nj)
-                acc[j] = 0;
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    // signs, then the magnitudes in place of the deltas
-    uint32_t s = 0, s2 = 0;
-#pragma unroll
-    for (uint32_t j = 0; j < 32; j++)
-        s = __builtin_amdgcn_alignbit(s, acc[j], 31);  // (s << 1) | sign of value j
-#pragma unroll
-    for (uint32_t j = 32; j < L; j++)
-        s2 = __builtin_amdgcn_alignbit(s2, acc[j], 31);
-    // (phase fences: without them the scheduler computes the magnitudes
-    // before the sign words and keeps both arrays live)
-    __builtin_amdgcn_sched_barrier(0);
+    // ---- widths, sizes, offsets
     uint32_t mx = 0;
 #pragma unroll
-    for (uint32_t j = 0; j < L; j++) {
-        acc[j] = mag(acc[j]);
-        mx = max(mx, acc[j]);
-    }
+    for (uint32_t j = 0; j < L; j++)
+        mx = max(mx, m[j]);
     __builtin_amdgcn_sched_barrier(0);
     const uint32_t w = has ? dwidth(mx) : 0u;
     const uint32_t bs = has ? (nj == L ? full_block_bytes(w) : lane_block_bytes(w, nj)) : 0u;
@@ -707,8 +790,6 @@ __device__ __forceinline__ void homsum_tile_lane(const Geom& g, const Tiling& tl
     const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
     if (Mode == kSumWave && lane == 0)
         lookback_publish(status, t, 0, total, 0);  // successors see the aggregate now
-    const bool fast = nj == L && w < 16;
-    const bool wide = __any(has && w >= 8);
 
     if constexpr (Mode == kSumWg) {
         // the workgroup's tile: its waves' bytes in wave order, one lookback
@@ -725,16 +806,10 @@ __device__ __forceinline__ void homsum_tile_lane(const Geom& g, const Tiling& tl
         }
         if (threadIdx.x == 0)
             lookback_publish(status, t_wg, 0, gtot, 0);  // successors see the aggregate now
-        const bool split = total + 64 > kOutBuf;
-        if (!split) {
-            const uint32_t nz = (total + 64 + 15) / 16;
-            for (uint32_t i = lane; i < nz; i += 64)
-                reinterpret_cast<uint4*>(obuf)[i] = make_uint4(0, 0, 0, 0);
-            if (has && w && fast)
-                encode_fast(obuf, excl, w, s, s2, acc, wide);
-            if (has && w && !fast)
-                encode_general(obuf, excl, w, nj, s, s2, acc);
-        }
+        const uint32_t nz = (total + 64 + 15) / 16;
+        for (uint32_t i = lane; i < nz; i += 64)
+            reinterpret_cast<uint4*>(obuf)[i] = make_uint4(0, 0, 0, 0);
+        encode_blocks(obuf, excl, w, nj, s, s2, m);
         if (wv == 0) {
             const unsigned long long ex = lookback(status, t_wg, 0, gtot, 0, ws, true);
             if (lane == 0)
@@ -745,25 +820,8 @@ __device__ __forceinline__ void homsum_tile_lane(const Geom& g, const Tiling& tl
         const uint64_t P0 = hdr + wsh->ex;  // the workgroup tile's stream offset
         const uint64_t P = P0 + woff;       // this wave's
         const bool fits = P0 + gtot <= out_cap;
-        if (!split) {
-            if (fits)
-                store_wave(obuf, out + P, total);
-        } else {
-            // a wave too wide for the buffer: half a wave at a time, value by value
-            const uint32_t mid = __builtin_amdgcn_readlane(excl, 32);
-            for (uint32_t i = lane; i < (mid + 64 + 15) / 16; i += 64)
-                reinterpret_cast<uint4*>(obuf)[i] = make_uint4(0, 0, 0, 0);
-            if (lane < 32 && has && w)
-                encode_general(obuf, excl, w, nj, s, s2, acc);
-            if (fits)
-                store_wave(obuf, out + P, mid);
-            for (uint32_t i = lane; i < (total - mid + 64 + 15) / 16; i += 64)
-                reinterpret_cast<uint4*>(obuf)[i] = make_uint4(0, 0, 0, 0);
-            if (lane >= 32 && has && w)
-                encode_general(obuf, excl - mid, w, nj, s, s2, acc);
-            if (fits)
-                store_wave(obuf, out + P + mid, total - mid);
-        }
+        if (fits)
+            store_wave(obuf, out + P, total);
         if (!fits && threadIdx.x == 0)
             raise_error(ws, ZK_ERR_NOSPACE);
         IndexView ox = index_view(g, oindex);
@@ -795,31 +853,13 @@ __device__ __forceinline__ void homsum_tile_lane(const Geom& g, const Tiling& tl
 
     if constexpr (Mode == kSumStaged) {
         uint8_t* slot = area + (8 + sizeof(StageRec)) * R + kStageSlot * sidx;
-        if (total + 64 <= kOutBuf) {
-            const uint32_t nz = (total + 64 + 15) / 16;
-            for (uint32_t i = lane; i < nz; i += 64)
-                reinterpret_cast<uint4*>(obuf)[i] = make_uint4(0, 0, 0, 0);
-            if (has && w && fast)
-                encode_fast(obuf, excl, w, s, s2, acc, wide);
-            if (has && w && !fast)
-                encode_general(obuf, excl, w, nj, s, s2, acc);
-            // whole 16-byte chunks: the slot is the tile's own (total <= kStageSlot, a multiple of 16)
-            for (uint32_t i = lane; i < (total + 15) / 16; i += 64)
-                reinterpret_cast<uint4*>(slot)[i] = reinterpret_cast<const uint4*>(obuf)[i];
-        } else {
-            // too wide for the buffer: half a wave at a time, value by value
-            const uint32_t mid = __builtin_amdgcn_readlane(excl, 32);
-            for (uint32_t i = lane; i < (mid + 64 + 15) / 16; i += 64)
-                reinterpret_cast<uint4*>(obuf)[i] = make_uint4(0, 0, 0, 0);
-            if (lane < 32 && has && w)
-                encode_general(obuf, excl, w, nj, s, s2, acc);
-            store_wave(obuf, slot, mid);
-            for (uint32_t i = lane; i < (total - mid + 64 + 15) / 16; i += 64)
-                reinterpret_cast<uint4*>(obuf)[i] = make_uint4(0, 0, 0, 0);
-            if (lane >= 32 && has && w)
-                encode_general(obuf, excl - mid, w, nj, s, s2, acc);
-            store_wave(obuf, slot + mid, total - mid);
-        }
+        const uint32_t nz = (total + 64 + 15) / 16;
+        for (uint32_t i = lane; i < nz; i += 64)
+            reinterpret_cast<uint4*>(obuf)[i] = make_uint4(0, 0, 0, 0);
+        encode_blocks(obuf, excl, w, nj, s, s2, m);
+        // whole 16-byte chunks: the slot is the tile's own (total <= kStageSlot, a multiple of 16)
+        for (uint32_t i = lane; i < (total + 15) / 16; i += 64)
+            reinterpret_cast<uint4*>(slot)[i] = reinterpret_cast<const uint4*>(obuf)[i];
         if (has)
             index_view(g, oindex).widths[x.g0 + lane] = (uint8_t) w;
         const uint32_t e16 = __builtin_amdgcn_readlane(excl, 16), e32 = __builtin_amdgcn_readlane(excl, 32),
@@ -839,42 +879,14 @@ __device__ __forceinline__ void homsum_tile_lane(const Geom& g, const Tiling& tl
 
     // ---- encode into the LDS buffer and store
     const uint64_t hdr = 8ull * g.T + 4ull * (x.s + 1);
-    unsigned long long ex;
-    if (total + 64 <= kOutBuf) {
-        const uint32_t nz = (total + 64 + 15) / 16;
-        for (uint32_t i = lane; i < nz; i += 64)
-            reinterpret_cast<uint4*>(obuf)[i] = make_uint4(0, 0, 0, 0);
-        // (two separate branches rather than if/else: the compiler would hoist
-        // what the two encoders share above an if/else and keep it live)
-        if (has && w && fast)
-            encode_fast(obuf, excl, w, s, s2, acc, wide);
-        if (has && w && !fast)
-            encode_general(obuf, excl, w, nj, s, s2, acc);
-        // the tile's stream offset: after its encoding, so predecessors had longer to publish
-        ex = lookback(status, t, 0, total, 0, ws, true);
-        if (hdr + ex + total <= out_cap)
-            store_wave(obuf, out + hdr + ex, total);
-    } else {
-        // a tile too wide for the buffer (its blocks average over 127 bytes):
-        // half a wave at a time, each half encoded value by value after the
-        // offset is known.  Straight-line: a loop here would keep the
-        // accumulators in scratch memory.
-        ex = lookback(status, t, 0, total, 0, ws, true);
-        const uint32_t mid = __builtin_amdgcn_readlane(excl, 32);  // lane 32's block offset
-        const bool ok = hdr + ex + total <= out_cap;
-        for (uint32_t i = lane; i < (mid + 64 + 15) / 16; i += 64)
-            reinterpret_cast<uint4*>(obuf)[i] = make_uint4(0, 0, 0, 0);
-        if (lane < 32 && has && w)
-            encode_general(obuf, excl, w, nj, s, s2, acc);
-        if (ok)
-            store_wave(obuf, out + hdr + ex, mid);
-        for (uint32_t i = lane; i < (total - mid + 64 + 15) / 16; i += 64)
-            reinterpret_cast<uint4*>(obuf)[i] = make_uint4(0, 0, 0, 0);
-        if (lane >= 32 && has && w)
-            encode_general(obuf, excl - mid, w, nj, s, s2, acc);
-        if (ok)
-            store_wave(obuf, out + hdr + ex + mid, total - mid);
-    }
+    const uint32_t nz = (total + 64 + 15) / 16;
+    for (uint32_t i = lane; i < nz; i += 64)
+        reinterpret_cast<uint4*>(obuf)[i] = make_uint4(0, 0, 0, 0);
+    encode_blocks(obuf, excl, w, nj, s, s2, m);
+    // the tile's stream offset: after its encoding, so predecessors had longer to publish
+    const unsigned long long ex = lookback(status, t, 0, total, 0, ws, true);
+    if (hdr + ex + total <= out_cap)
+        store_wave(obuf, out + hdr + ex, total);
     const uint64_t P = hdr + ex;
     const bool fits = P + total <= out_cap;
     if (!fits && lane == 0)
@@ -1019,8 +1031,8 @@ struct DecPre {
 
 struct DecLoc {
     View v;
-    uint32_t w, bs, o, lim, nj;
-    bool has, skip, staged;
+    uint32_t w, o, tot, nj;
+    bool has, skip, half;
 };
 
 // What a run over the tiles writes: their values, or (single streams) their
@@ -1049,9 +1061,7 @@ __device__ __forceinline__ DecPre dec_prefetch(const Args& a, uint64_t tg)
 }
 
 // Locate the lane's block of tile p (one scan of the block sizes) and stage
-// the tile's bytes into LDS half `half` of the wave buffer (16-byte
-// direct-to-LDS loads, zeros past the stream); tiles too large to stage are
-// read per lane.
+// the tile's bytes into LDS half `half` of the wave buffer, if they fit there.
 template <typename Args>
 __device__ __forceinline__ DecLoc dec_locate(const Args& a, const DecPre& p, uint32_t* obuf, uint32_t half,
     bool& bad_width)
@@ -1069,27 +1079,21 @@ __device__ __forceinline__ DecLoc dec_locate(const Args& a, const DecPre& p, uin
         bad_width = true;
         c.w = 0;
     }
-    c.bs = c.has ? (c.nj == L ? full_block_bytes(c.w) : lane_block_bytes(c.w, c.nj)) : 0u;
-    const uint32_t binc = wave_scan_dpp(c.bs);
+    const uint32_t bs = c.has ? (c.nj == L ? full_block_bytes(c.w) : lane_block_bytes(c.w, c.nj)) : 0u;
+    const uint32_t binc = wave_scan_dpp(bs);
     const uint32_t tot0 = __builtin_amdgcn_readlane(binc, 63);
-    c.skip = p.goff > p.size || tot0 > p.size - p.goff;
-    const uint8_t* base = d.bytes + p.goff;
+    // (the same in every lane: scalar, so that what depends on them branches)
+    const uint64_t goff = uniform64(p.goff), size = uniform64(p.size);
+    c.skip = goff > size || tot0 > size - goff;
+    const uint8_t* base = d.bytes + goff;
     const uint32_t delta = (uint32_t) ((uintptr_t) base & 3u);
-    const uint64_t vlen = c.skip ? 0ull : align_up(delta + (p.size - p.goff), 4);
-    c.lim = vlen > 0xFFFFFFFCull ? 0xFFFFFFFCu : (uint32_t) vlen;
+    const uint64_t vlen = c.skip ? 0ull : align_up(delta + (size - goff), 4);
     c.v = make_view(base - delta, vlen);
-    c.o = delta + binc - c.bs;
-    const uint32_t nch = (tot0 + delta + 15) >> 4;
-    c.staged = !c.skip && 16 * nch <= kStageCap;
-    if (c.staged) {
-        uint8_t* st = (uint8_t*) obuf + half * kStageHalf;
-        for (uint32_t run = 0; run * 64 < nch; run++) {
-            const uint32_t ch = run * 64 + lane;
-            if (ch < nch)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(c.v, (__attribute__((address_space(3))) void*) (st + run * 1024),
-                    16, 16 * ch, 0, 0, 0);
-        }
-    }
+    c.o = delta + binc - bs;
+    c.tot = tot0 + delta;
+    c.half = !c.skip && staged_len(c.tot) <= kStageCap;
+    if (c.half)
+        stage_bytes(c.v, c.tot, obuf + half * (kStageHalf / 4));
     return c;
 }
 
@@ -1174,10 +1178,8 @@ __device__ __forceinline__ void store_blocks(float* base, const float (&v)[L], u
 
 // A run over launch tiles first, first + stride, ... of one wave.  Per step,
 // tile i is decoded while tile i+1's bytes move into the other LDS half and
-// tile i+2's index entries are on their way.  The lane decoders are the sum's
-// (whole blocks below width 16 that the reads covered take the fast one, the
-// rest the general one; a lane that does not use the fast decoder runs it at
-// width 0, which adds zeros).
+// tile i+2's index entries are on their way (a tile too large for a half is
+// staged alone).  The lane decoders are the sum's.
 template <int Mode, typename Args>
 __device__ __forceinline__ void dec_run(const Args& a, WsHeader* ws, uint64_t first, uint64_t stride, uint32_t* obuf)
 {
@@ -1190,48 +1192,50 @@ __device__ __forceinline__ void dec_run(const Args& a, WsHeader* ws, uint64_t fi
     DecLoc cc = dec_locate(a, pc, obuf, 0, bad_width);
     DecPre pn = dec_prefetch<Mode>(a, first + stride);
     for (uint32_t half = 0;; half ^= 1u) {
+        const uint32_t* st = obuf + (cc.half ? half * (kStageHalf / 4) : 0u);
+        if (!cc.half && !cc.skip)  // (the other half's tile is decoded)
+            stage_bytes(cc.v, cc.tot, obuf);
         __builtin_amdgcn_s_waitcnt(0);  // tile i's bytes in LDS, tile i+1's index entries in registers
-        Block q;
-        q.w = cc.w;
-        q.o = cc.o;
-        q.lim = cc.lim;
-        if (cc.staged)
-            read_block_staged(obuf + half * (kStageHalf / 4), cc.o, cc.w, q);
-        else
-            read_block_direct(cc.v, cc.o, cc.w, q);
-        __builtin_amdgcn_sched_barrier(0);
         DecLoc cn;
         DecPre pnn;
         pnn.ok = false;
-        if (pn.ok) {
-            cn = dec_locate(a, pn, obuf, half ^ 1u, bad_width);
-            pnn = dec_prefetch<Mode>(a, pn.idx + stride);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        const bool fast = !cc.has || cc.w == 0 || (cc.nj == L && cc.w < 16 && (cc.staged || cc.o + cc.bs + 3 <= cc.lim));
-        const bool use = fast && !cc.skip;
-        bad_byte |= use && cc.has && (cc.w || cc.staged || cc.o + 4 <= cc.lim) && (q.h[0] & 0xFFu) != cc.w;
-        bad_over |= cc.skip;
-        q.w = use ? cc.w : 0u;
-        const bool gen = !fast && !cc.skip;
-        if constexpr (Mode == kCarrySums) {
-            // the block's sum only (a lane on the fast path has nj = L or
-            // adds zeros; the general decoder adds garbage past nj)
-            uint32_t part[2] = {0u, 0u};
-            decode_fast<true>(q, part);
-            uint32_t b = part[0] + part[1];
-            if (__any(gen)) {
-                uint32_t acc[L];
-#pragma unroll
-                for (uint32_t j = 0; j < L; j++)
-                    acc[j] = 0;
-                if (gen)
-                    bad_byte |= decode_general(cc.v, cc.o, cc.w, cc.nj, acc);
-#pragma unroll
-                for (uint32_t j = 0; j < L; j++)
-                    if (j < cc.nj)
-                        b += acc[j];
+        auto next = [&] {
+            if (pn.ok) {
+                cn = dec_locate(a, pn, obuf, half ^ 1u, bad_width);
+                pnn = dec_prefetch<Mode>(a, pn.idx + stride);
             }
+        };
+        // f(j, magnitude, +1 or -1) over the lane's values (zeros for a lane
+        // without a block), f_high(j, magnitude, sign word) over those of a block
+        // from width 16, and next() where it overlaps best
+        auto values = [&](auto f, auto f_high) {
+            if (!cc.skip) {
+                bad_byte |= cc.has & (((const uint8_t*) st)[cc.o] != cc.w);
+                const bool wide = __any(cc.w >= 8);
+                const uint32_t w = cc.w < 16 ? cc.w : 0u;
+                Block q;
+                read_block(st, cc.o, w, cc.nj, wide, q);
+                __builtin_amdgcn_sched_barrier(0);
+                const bool high = wide && __any(cc.w >= 16);
+                if (cc.half && !high)
+                    next();
+                __builtin_amdgcn_sched_barrier(0);
+                each_value(q, w, wide, f);
+                if (high)
+                    each_high_lane(st, cc.o, cc.w, cc.nj, cc.w >= 16, f_high);
+                return cc.half && !high;
+            }
+            return false;
+        };
+        bad_over |= cc.skip;
+        if constexpr (Mode == kCarrySums) {
+            // the block's sum only, of its nj values
+            uint32_t b = 0;
+            const bool ahead = values(
+                [&](uint32_t j, uint32_t m, uint32_t sign) { b = mad_i24(j < cc.nj ? m : 0u, sign, b); },
+                [&](uint32_t j, uint32_t m, uint32_t sw) { b += j < cc.nj ? signed_of(m, sw) : 0u; });
+            if (!ahead)
+                next();
             const uint32_t inc = wave_scan_dpp(b);
             if (lane == 63) {
                 DecJob d;
@@ -1239,35 +1243,32 @@ __device__ __forceinline__ void dec_run(const Args& a, WsHeader* ws, uint64_t fi
                 index_view(d.g, d.index).carry[d.t] = inc;
             }
         } else {
+            // the deltas, then their running sums (past a short block's
+            // values: whatever follows it, never stored)
             uint32_t acc[L];
 #pragma unroll
             for (uint32_t j = 0; j < L; j++)
                 acc[j] = 0;
-            decode_fast<true>(q, acc);
-            if (__any(gen)) {
-                if (gen)
-                    bad_byte |= decode_general(cc.v, cc.o, cc.w, cc.nj, acc);
-            }
-            if (cc.nj < L) {
-#pragma unroll
-                for (uint32_t j = 0; j < L; j++)
-                    if (j >= cc.nj)
-                        acc[j] = 0;
-            }
-            DecJob d;
-            dec_job(a, pc.idx, d);
-            const Tile x = tile_of(d.g, d.tl, d.t);
+            const bool ahead =
+                values([&](uint32_t j, uint32_t m, uint32_t sign) { acc[j] = mad_i24(m, sign, 0u); },
+                    [&](uint32_t j, uint32_t m, uint32_t sw) { acc[j] = stay(signed_of(m, sw)); });
+            if (!ahead)
+                next();
 #pragma unroll
             for (uint32_t j = 1; j < L; j++)
                 acc[j] += acc[j - 1];
-            const uint32_t bsum = acc[L - 1];
-            const uint32_t carry = pc.carry + wave_scan_dpp(bsum) - bsum;
+            const uint32_t run = acc[L - 1];
+            DecJob d;
+            dec_job(a, pc.idx, d);
+            const Tile x = tile_of(d.g, d.tl, d.t);
+            const uint32_t carry = pc.carry + wave_scan_dpp(run) - run;
             const float eb = d.eb;
             float vals[L];
 #pragma unroll
             for (uint32_t jj = 0; jj < L; jj++)
                 vals[jj] = dequant(carry + acc[jj], eb);
-            // (this tile's LDS half is free: its bytes are in registers)
+            // (this tile's LDS half is free: its bytes are in registers; the
+            // other half may hold the next tile's)
             store_blocks(d.out + x.e0, vals, cc.nj, x.nblk, obuf + half * (kStageHalf / 4));
             if (lane == 0 && x.lt == 0)
                 d.out[x.seg_a] = dequant(pc.carry, eb);  // the segment's first value, its seed
@@ -1334,8 +1335,41 @@ __device__ __forceinline__ void carry_scan(const Geom& g, const uint8_t* bytes, 
 // (one chain per stream, as the slot kernel), and each wave stores its bytes.
 // Arithmetic: ZCCL/src/ZCCL_float.c:563,577-606 (quantize, delta, width),
 // ZCCL/src/ZCCL_TypeManager.c:12-91, 824-848 (packing, signs).
+
+// Quantize by FP32: x / bound is exact in 48 bits, and FP32 rounding toward
+// zero keeps its integer part below 2^24; a second product with 2^-149,
+// rounded toward zero too, drops the fraction and leaves the integer as a
+// denormal's bits, so deltas are FP32 differences (exact below 2^23).  Two
+// 2-cycle instructions and one to turn -0 into +0 in place of an FP64 product
+// with its conversions and range checks (22 cycles).  `far` collects the
+// largest magnitude, or NaN: the wave takes the FP64 form unless it is below
+// kQuantSmall.  The products are volatile so that none moves above
+// round_toward_zero(); nothing else in the kernel rounds FP32.
+constexpr float kQuantSmall = 8388608.0f;  // 2^23
+
+__device__ __forceinline__ void round_toward_zero()
+{
+    asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 3");
+}
+
+__device__ __forceinline__ void quant_small(float x, float inv, float& q, float& far)
+{
+    float p, t;
+    asm volatile("v_mul_f32 %0, %1, %2" : "=v"(p) : "v"(x), "v"(inv));
+    asm volatile("v_mul_f32 %0, %1, %2" : "=v"(t) : "s"(1u), "v"(p));
+    q = t + 0.0f;
+    asm("v_maximum3_f32 %0, |%1|, %2, %2" : "=v"(far) : "v"(p), "v"(far));
+}
+
+// v of the lane below; lane 0: first.
+__device__ __forceinline__ float from_lane_below(float v, float first)
+{
+    return as_f((uint32_t) __builtin_amdgcn_update_dpp((int) as_u(first), (int) as_u(v), 0x138, 0xF, 0xF, false));  // wave_shr:1
+}
+
 constexpr uint32_t kCompBuf = 9728;  // a wave's values (<= 2305 floats) or a worst-case 64-block encode + reach
-static_assert(kCompBuf >= kLaneTileBlocks * kWorstBlock + 64 && kCompBuf >= 4 * (kLaneTileBlocks * L + 1) + 16,
+static_assert(kCompBuf >= kLaneTileBlocks * kWorstBlock + 64 && kCompBuf >= (kLaneTileBlocks - 1) * kWorstBlock + kReach &&
+        kCompBuf >= 4 * kLaneTileBlocks * L,
     "a compress wave buffer holds the staged values and the worst-case encode");
 static_assert(kCompBuf % 16 == 0, "compress wave buffers stay 16-byte aligned");
 
@@ -1348,49 +1382,93 @@ __device__ __forceinline__ void compress_tile_lane(const Geom& g, const Tiling& 
     uint8_t* out, uint64_t out_cap, uint8_t* oindex, unsigned long long* size_out, uint64_t t,
     unsigned long long* status, WsHeader* ws, uint32_t nchains, uint32_t* obuf, CompShared& sh)
 {
+    round_toward_zero();
     const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const Tile x = tile_of(g, tl, (uint32_t) t);
     const uint32_t jb = kLaneTileBlocks * wv + lane;  // block of the tile
     const bool has = jb < x.nblk;
     const uint32_t nj = has ? min(tile_block_len(g, x, jb), L) : 0u;
-    // the wave's values and the one before them (the segment's first value,
-    // the seed, before its first block)
+    // the wave's values
     const uint32_t nbw = x.nblk > kLaneTileBlocks * wv ? min(x.nblk - kLaneTileBlocks * wv, kLaneTileBlocks) : 0u;
     const uint32_t nvals = nbw ? (nbw - 1) * L + min(tile_block_len(g, x, kLaneTileBlocks * wv + nbw - 1), L) : 0u;
-    const uint32_t v0 = x.e0 + kLaneTileBlocks * L * wv - 1;  // input index of LDS float 0
+    const uint32_t v0 = x.e0 + kLaneTileBlocks * L * wv;  // input index of the wave's first value
+    float xb = 0.0f;                                      // lane 0: the value before it
     if (nbw) {
-        // (a view of the wave's values alone: its range check ends them)
-        const View vx = make_view((const uint8_t*) (xin + v0), 4ull * (nvals + 1));
-        const uint32_t nch = (4 * (nvals + 1) + 15) >> 4;
-        for (uint32_t run = 0; run * 64 < nch; run++) {
-            const uint32_t ch = run * 64 + lane;
-            if (ch < nch)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(vx,
-                    (__attribute__((address_space(3))) void*) ((uint8_t*) obuf + run * 1024), 16, 16 * ch, 0, 0, 0);
-        }
+        // (a view of the wave's values alone: its range check ends them with
+        // zeros)
+        const View vx = make_view((const uint8_t*) (xin + v0), 4ull * nvals);
+#pragma unroll
+        for (uint32_t run = 0; run < kLaneTileBlocks * L / 256; run++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(vx,
+                (__attribute__((address_space(3))) void*) ((uint8_t*) obuf + run * 1024), 16, 1024 * run + 16 * lane, 0,
+                0, 0);
+        if (lane == 0)
+            xb = xin[v0 - 1];
     }
     __builtin_amdgcn_s_waitcnt(0);
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     // quantize, deltas, signs and magnitudes (values past nj are zero)
-    const float* xv = reinterpret_cast<const float*>(obuf) + lane * L;
+    const float4* xv = reinterpret_cast<const float4*>(obuf) + lane * (L / 4);
     uint32_t m[L];
-    uint32_t s = 0, s2 = 0, mx = 0, before;
+    uint32_t s = 0, s2 = 0, mx = 0;
+    uint32_t before = 0;  // lane 0: the quantized value before the wave's first
     {
-        uint32_t prev = (uint32_t) quant(xv[0], inv);
-        before = prev;
+        const float finv = (float) inv;
+        float q[L];
+        float far = 0.0f;
 #pragma unroll
-        for (uint32_t j = 0; j < L; j++) {
-            const uint32_t q = (uint32_t) quant(xv[j + 1], inv);
-            const uint32_t d = j < nj ? q - prev : 0u;
-            prev = q;
-            if (j < 32)
-                s = __builtin_amdgcn_alignbit(s, d, 31);  // (s << 1) | sign of value j
-            else
-                s2 = __builtin_amdgcn_alignbit(s2, d, 31);
-            m[j] = mag(d);
-            mx = max(mx, m[j]);
+        for (uint32_t i = 0; i < L / 4; i++) {
+            const float4 v = xv[i];
+            quant_small(v.x, finv, q[4 * i], far);
+            quant_small(v.y, finv, q[4 * i + 1], far);
+            quant_small(v.z, finv, q[4 * i + 2], far);
+            quant_small(v.w, finv, q[4 * i + 3], far);
         }
+        float qb;
+        quant_small(xb, finv, qb, far);
+        if (!__any(!(far < kQuantSmall))) {
+            before = signed_of(as_u(qb) & 0x7FFFFFFFu, as_u(qb));
+            float prev = from_lane_below(q[L - 1], qb);
+#pragma unroll
+            for (uint32_t j = 0; j < L; j++) {
+                m[j] = as_u(q[j] - prev);
+                prev = q[j];
+            }
+            if (__any(nj < L)) {
+#pragma unroll
+                for (uint32_t j = 0; j < L; j++)
+                    if (j >= nj)
+                        m[j] = 0;
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < L; j++) {
+                if (j < 32)
+                    s = __builtin_amdgcn_alignbit(s, m[j], 31);  // (s << 1) | sign of value j
+                else
+                    s2 = __builtin_amdgcn_alignbit(s2, m[j], 31);
+                m[j] &= 0x7FFFFFFFu;
+            }
+        } else {
+            // some value of the wave is 2^23 bounds from zero, or not a number
+            before = (uint32_t) quant(xb, inv);
+            uint32_t prev =
+                as_u(from_lane_below(as_f((uint32_t) quant(reinterpret_cast<const float*>(xv)[L - 1], inv)), as_f(before)));
+#pragma unroll
+            for (uint32_t j = 0; j < L; j++) {
+                const uint32_t qj = (uint32_t) quant(reinterpret_cast<const float*>(xv)[j], inv);
+                const uint32_t d = j < nj ? qj - prev : 0u;
+                prev = qj;
+                if (j < 32)
+                    s = __builtin_amdgcn_alignbit(s, d, 31);
+                else
+                    s2 = __builtin_amdgcn_alignbit(s2, d, 31);
+                m[j] = mag(d);
+            }
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < L; j++)
+            mx = max(mx, m[j]);
     }
     const uint32_t w = has ? dwidth(mx) : 0u;
     const uint32_t bs = has ? (nj == L ? full_block_bytes(w) : lane_block_bytes(w, nj)) : 0u;
@@ -1409,19 +1487,12 @@ __device__ __forceinline__ void compress_tile_lane(const Geom& g, const Tiling& 
     }
     if (threadIdx.x == 0)
         lookback_publish(status, t, 0, total, 0);  // successors see the aggregate now
-    const bool fast = nj == L && w < 16;
-    const bool wide = __any(has && w >= 8);
     const uint32_t nz = (wtot + 64 + 15) / 16;
     for (uint32_t i = lane; i < nz; i += 64)
         reinterpret_cast<uint4*>(obuf)[i] = make_uint4(0, 0, 0, 0);
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    // (two separate branches rather than if/else: the compiler would hoist
-    // what the two encoders share above an if/else and keep it live)
-    if (has && w && fast)
-        encode_fast(obuf, excl, w, s, s2, m, wide);
-    if (has && w && !fast)
-        encode_general(obuf, excl, w, nj, s, s2, m);
+    encode_blocks(obuf, excl, w, nj, s, s2, m);
     if (wv == 0) {
         const unsigned long long ex = lookback(status, t, 0, total, 0, ws, true);
         if (lane == 0)
@@ -1492,7 +1563,7 @@ __global__ void __launch_bounds__(64 * kLaneWaves, 4) k_homsum_lane(HomsumArgs a
 
 // Uniform batch: shared geometry, per-job pointers in device memory; tiles of
 // the jobs interleave (tile b is tile b / njobs of job b % njobs).
-__global__ void __launch_bounds__(64 * kLaneWaves, 5) k_homsum_lane_batch(BatchArgs b)
+__global__ void __launch_bounds__(64 * kLaneWaves, 4) k_homsum_lane_batch(BatchArgs b)
 {
     uint64_t t0;
     unsigned long long* status;
@@ -1560,21 +1631,17 @@ __device__ __forceinline__ void dec_grid(const Args& a, WsHeader* ws)
         zk_lds + wv * (kOutBuf / 4));
 }
 
-// five workgroups per CU: the LDS buffers' limit
-constexpr uint32_t kDecGroupsPerCU = 5;
-static_assert(kDecGroupsPerCU == (uint32_t) kDecGroupsMax, "the launch bound is the grid's limit");
-
-__global__ void __launch_bounds__(64 * kLaneWaves, kDecGroupsPerCU) k_decompress_lane(DecompressArgs a)
+__global__ void __launch_bounds__(64 * kLaneWaves, 4) k_decompress_lane(DecompressArgs a)
 {
     dec_grid<kValues>(a, a.ws);
 }
-__global__ void __launch_bounds__(64 * kLaneWaves, kDecGroupsPerCU) k_decompress_lane_batch(BatchArgs b)
+__global__ void __launch_bounds__(64 * kLaneWaves, 4) k_decompress_lane_batch(BatchArgs b)
 {
     dec_grid<kValues>(b, b.ws);
 }
 
 // Carries of a parsed stream (none of a corrupt one, whose size is 0).
-__global__ void __launch_bounds__(64 * kLaneWaves, kDecGroupsPerCU) k_lane_carry_sums(DecompressArgs a)
+__global__ void __launch_bounds__(64 * kLaneWaves, 4) k_lane_carry_sums(DecompressArgs a)
 {
     if (index_view(a.job.g, a.job.io.in[0].index).meta[0])
         dec_grid<kCarrySums>(a, a.ws);
@@ -1773,7 +1840,7 @@ __global__ void __launch_bounds__(64 * kLaneWaves, 4) k_homsum_lane_staged(Homsu
 // Pass one of a uniform batch: a workgroup takes kLaneWaves consecutive
 // tiles of one job (ceil(ntiles / kLaneWaves) workgroups per job, jobs in
 // order of the XCD-contiguous index), slot job * ntiles + tile.
-__global__ void __launch_bounds__(64 * kLaneWaves, 5) k_homsum_lane_batch_staged(BatchArgs b, uint8_t* stage)
+__global__ void __launch_bounds__(64 * kLaneWaves, 4) k_homsum_lane_batch_staged(BatchArgs b, uint8_t* stage)
 {
     const uint32_t wv = threadIdx.x >> 6;
     const uint32_t wpj = (uint32_t) ceil_div(b.tl.ntiles, kLaneWaves);
@@ -1988,7 +2055,7 @@ hipError_t launch_homsum_lane_batch(const BatchArgs& b, hipStream_t s)
     return hipGetLastError();
 }
 
-// (four measured fastest on the 8 x 2^24 batch, the grid's limit being five)
+// (four: what the LDS buffers let a CU hold)
 constexpr int kDecGroupsDefault = 4;
 static std::atomic<int> g_dec_groups{kDecGroupsDefault};
 
