@@ -1260,7 +1260,9 @@ static int sz3_args(size_t d1, size_t d2, size_t d3, int Bs, int T, void* ws, si
     a->offs = (unsigned long long*) (w + L.offs);
     a->part_sums = (unsigned long long*) (w + L.sums);
     a->parts = (const Part3*) (w + L.parts);
-    HIP_TRY(launch_sz3_table(a->g, (Part3*) a->parts, a->status, s));
+    // (the tile words of a compress by lanes lie where other paths keep the
+    // block offsets: at most a tile per block)
+    HIP_TRY(launch_sz3_table(a->g, (Part3*) a->parts, a->status, a->offs, a->g.nlane, s));
     return ZCCL_OK;
 }
 

@@ -251,7 +251,9 @@ hipError_t launch_homsum_lane_batch_staged(const BatchArgs& b, uint8_t* stage, h
 hipError_t launch_case_count(const uint8_t* w1, const uint8_t* w2, uint64_t nblocks,
     unsigned long long* counts, hipStream_t s);
 hipError_t launch_ws_init(WsHeader* ws, uint64_t capacity, hipStream_t s);
-hipError_t launch_sz3_table(const Geom3& g, Part3* parts, unsigned long long* status, hipStream_t s);
+// (clear: the tiles' words to zero)
+hipError_t launch_sz3_table(const Geom3& g, Part3* parts, unsigned long long* status, unsigned long long* clear,
+    uint32_t nclear, hipStream_t s);
 hipError_t launch_sz3_compress(const Sz3Args& a, hipStream_t s);
 hipError_t launch_sz3_decompress(const Sz3Args& a, hipStream_t s);
 

@@ -35,8 +35,9 @@ struct Part3 {
     uint32_t zr0;          // first z-row (x, y pair) of the sub-volume in the z pass
     uint32_t yc0;          // first y-column (x, z pair) in the y pass
     uint32_t xc0;          // first x-column (y, z pair) in the x pass
-    uint32_t u0;           // first chunk of the tiled compress (block sides 4, 8)
+    uint32_t u0;           // first chunk of the tiled compress (block side 8)
     uint32_t c0;           // first block column (bx, by) of the tiled decoder
+    uint32_t l0;           // first workgroup tile of the lane compress (block side 4)
 };
 
 struct Geom3 {
@@ -46,12 +47,25 @@ struct Geom3 {
     uint32_t zrows, ycols, xcols;
     uint32_t nunits;       // chunks of the tiled compress (0: no tiled path)
     uint32_t ncols;        // block columns of the tiled decoder
+    uint32_t nlane;        // workgroup tiles of the lane compress (0: not that path)
+    uint32_t wlane;        // waves of such a tile
 };
 
 // Blocks per chunk along z of the tiled kernels: a chunk is one (bx, by)
 // column of blocks cut to tile_nz3 blocks, whose quantized values with a
 // one-value halo fit in LDS.  0 where the tiled path has no instance.
 ZK_HD constexpr uint32_t tile_nz3(uint32_t Bs) { return Bs == 4 ? 64u : Bs == 8 ? 8u : 0u; }
+
+// Lane compress (block side 4): one lane per block, a wave per run of
+// kLaneRun3 blocks of a sub-volume in stream order (lane 0 holds the block
+// before the run), kLaneWide3 waves per workgroup tile, or kLaneSlim3 below
+// kLaneFew3 values, where wide tiles leave compute units idle.  Rows are
+// addressed by 32-bit offsets, so longer ones than kLaneMaxRow3 take the
+// generic kernels.
+constexpr uint32_t kLaneRun3 = 63;
+constexpr uint32_t kLaneSlim3 = 4, kLaneWide3 = 12;
+constexpr uint64_t kLaneFew3 = 64ull * kLaneRun3 * kLaneWide3 * 256;
+constexpr uint32_t kLaneMaxRow3 = 1u << 27;
 
 // Factorise T over three dims as My_Dims_create (ZCCL/src/ZCCL_multidim.c:
 // 100-140): prime factors of T, largest first, each multiplied into the
@@ -111,7 +125,10 @@ ZK_HD bool make_geom3(uint64_t d1, uint64_t d2, uint64_t d3, int Bs, int T, Geom
     const uint32_t bx = g->d1 / td[0], rx = g->d1 % td[0], by = g->d2 / td[1], ry = g->d2 % td[1];
     const uint32_t bz = g->d3 / td[2], rz = g->d3 % td[2];
     const uint32_t nz = tile_nz3((uint32_t) Bs);
-    uint32_t r = 0, ox = 0, nb = 0, zr = 0, yc = 0, xc = 0, nu = 0, nc = 0;
+    const bool lane = Bs == 4 && g->d3 < kLaneMaxRow3;
+    g->wlane = (uint64_t) g->d1 * g->d2 * g->d3 < kLaneFew3 ? kLaneSlim3 : kLaneWide3;
+    const uint32_t lane_tile = g->wlane * kLaneRun3;
+    uint32_t r = 0, ox = 0, nb = 0, zr = 0, yc = 0, xc = 0, nu = 0, nc = 0, nl = 0;
     for (int px = 0; px < td[0]; px++) {
         const uint32_t sx = bx + ((uint32_t) px < rx ? 1u : 0u);
         uint32_t oy = 0;
@@ -131,6 +148,8 @@ ZK_HD bool make_geom3(uint64_t d1, uint64_t d2, uint64_t d3, int Bs, int T, Geom
                 p.xc0 = xc;
                 p.u0 = nu;
                 p.c0 = nc;
+                p.l0 = nl;
+                nl += lane ? (p.b1 * p.b2 * p.b3 + lane_tile - 1) / lane_tile : 0u;
                 nu += nz ? p.b1 * p.b2 * ((p.b3 + nz - 1) / nz) : 0u;
                 nc += p.b1 * p.b2;
                 nb += p.b1 * p.b2 * p.b3;
@@ -149,6 +168,7 @@ ZK_HD bool make_geom3(uint64_t d1, uint64_t d2, uint64_t d3, int Bs, int T, Geom
     g->xcols = xc;
     g->nunits = nu;
     g->ncols = nc;
+    g->nlane = nl;
     return true;
 }
 
@@ -174,6 +194,20 @@ ZK_HD uint32_t part_of_block(const Part3* parts, uint32_t T, uint32_t gb)
     while (hi - lo > 1) {
         const uint32_t mid = (lo + hi) / 2;
         if (parts[mid].g0 <= gb)
+            lo = mid;
+        else
+            hi = mid;
+    }
+    return lo;
+}
+
+// Sub-volume of workgroup tile v of the lane compress, by binary search.
+ZK_HD uint32_t part_of_lane_tile(const Part3* parts, uint32_t T, uint32_t v)
+{
+    uint32_t lo = 0, hi = T;
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) / 2;
+        if (parts[mid].l0 <= v)
             lo = mid;
         else
             hi = mid;
@@ -225,7 +259,7 @@ ZK_HD Chunk3 chunk_of3(const Part3& p, uint32_t rel, uint32_t Bs)
 }
 
 // Device workspace of one 3-D call, in order: 256 bytes of status words
-// (status[0] stream size, status[1] error bits), the per-block size words,
+// (status[0] stream size, status[1] error bits, status[2] the next tile ticket), the per-block size words,
 // their exclusive scan (u64), the scan's per-group sums (+ the total) and the
 // sub-volume table.
 constexpr uint32_t kScan3Group = 1024;  // entries per scan group

@@ -6,7 +6,8 @@
 // buffers; its residual is the exact 3-D difference dx dy dz q (zero outside
 // the sub-volume) and its decoder the exact 3-D prefix sum, so both are done
 // here with full parallelism:
-//   compress   k3_table (sub-volume table) -> k3_widths (one wave per block:
+//   compress   k3_table (sub-volume table) -> for block side 4 k3l_compress (one
+//              lane per block, one pass); others k3_widths (one wave per block:
 //              residuals from x, block max, width, payload size) -> scan of the
 //              payload sizes -> k3_encode (one wave per block: width header
 //              byte, sub-volume offset, sign bitmap and fixed-length bits with
@@ -20,8 +21,12 @@
 // built with -ffp-contract=off); residuals and sums wrap in 32 bits.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
+#include "zccl_device.h"
 #include "zccl_internal.h"
 #include "zccl_kernels.h"
+#include "zccl_pack.h"
 #include "zccl_sz3d.h"
 #include "zccl_unit.h"
 
@@ -137,16 +142,20 @@ __device__ __forceinline__ uint32_t wave_incl_scan32(uint32_t v)
 constexpr uint32_t kSizeMask = (1u << 26) - 1;
 
 // Sub-volume table, built on the device by one thread (no host copy on the
-// stream the caller passes), and the status words cleared.
-__global__ void k3_table(uint32_t d1, uint32_t d2, uint32_t d3, int Bs, int T, Part3* parts,
-    unsigned long long* status)
+// stream the caller passes), and the status words and `nclear` lookback words
+// cleared.
+__global__ void __launch_bounds__(256) k3_table(uint32_t d1, uint32_t d2, uint32_t d3, int Bs, int T, Part3* parts,
+    unsigned long long* status, unsigned long long* clear, uint32_t nclear)
 {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
         Geom3 g;
         make_geom3(d1, d2, d3, Bs, T, &g, parts);
         status[0] = 0;
         status[1] = 0;
+        status[2] = 0;
     }
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < nclear; i += gridDim.x * 256)
+        clear[i] = 0;
 }
 
 // Width and payload size of every block: one wave per block.
@@ -860,6 +869,306 @@ __global__ void __launch_bounds__(256) k3t_decode(Sz3Args a)
     }
 }
 
+// ------------------------------------------------------------ lane compress
+// Block side 4.  One lane per block: the lane reads its block's 16 rows of four
+// values and the rows one y and one x before them (16-byte loads, consecutive
+// blocks of a row in consecutive lanes), quantizes, and takes the differences
+// in registers: along z from its own values and the last of the lane below
+// (lane 0 of a wave holds the block before the wave's run for that alone),
+// along y from the row before, along x from the plane before.  The 64 residuals
+// stay in the lane for the width, the wave scans the sizes, the lane encoders
+// pack the payload in LDS, and the sizes of all tiles before it in stream
+// order give its place: every value is read once (its halo rows come from the
+// caches) and quantized 25/16 times.
+//
+// Two chunk kernels with the quantized values in LDS, a scan of the block sizes
+// between them, read and quantized everything twice and took 617 us for a
+// 512^3 volume (relative bound 1e-3); this takes 323.  250 without the wait for
+// the tiles before one, with four waves a tile: the workgroups that wait finish
+// together and the next ones load together.  Twelve waves a tile leave a third
+// of the tickets (12 ns each: adds to one address follow one another) and of
+// the lookback words: 323 us against 384 with four; 256^3: 58 against 64; but
+// 128^3: 28 against 16 (half the compute units idle), hence the line at a wide
+// tile for each of 256 units.  Not faster: sums over groups of 64 tiles (326 to
+// 690), a workgroup that places a tile after the next one's differences (426).
+
+// Payload bytes of the tiles before tile t, and of those before tile p0 <= t
+// (a sub-volume's first), by one wave once t's own `agg` bytes are published:
+// the decoupled lookback with four tiles a lane, 256 in a window (512 tiles
+// are in flight).  Tiles are numbered by tickets, so those before one have all
+// started; the wait is bounded.
+__device__ __forceinline__ void places3(unsigned long long* status, uint32_t t, uint32_t p0, unsigned long long agg,
+    unsigned long long* err, unsigned long long& at, unsigned long long& part)
+{
+    const uint32_t lane = threadIdx.x & 63;
+    unsigned long long excl = 0, sp = kFlagInc;
+    uint32_t spins = 0;
+    for (int64_t end = t; end > 0; end -= 256) {
+        unsigned long long sum = 0;
+        bool inc = false;
+        while (true) {
+            sum = 0;
+            inc = false;
+            bool miss = false;
+            if (p0)
+                sp = st_poll(&status[p0 - 1]);
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const int64_t i = end - 1 - (int64_t) (4 * lane + c);
+                const unsigned long long st = i >= 0 ? st_poll(&status[i]) : kFlagInc;
+                // up to the nearest inclusive value, or the first missing one
+                const bool use = !inc && !miss;
+                miss |= use && (st >> 62) == 0;
+                sum += use ? st & kValMask : 0ull;
+                inc |= use && (st >> 62) == 2;
+            }
+            const unsigned long long mm = __ballot(miss), im = __ballot(inc);
+            const unsigned long long need = im ? ((im & (~im + 1)) << 1) - 1 : ~0ull;
+            if (!(mm & need))
+                break;
+            if (++spins > kSpinLimit) {
+                if (lane == 0)
+                    raise3(err, ZK_ERR_SPIN);
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+        const unsigned long long im = __ballot(inc);
+        if (im && lane > (uint32_t) __builtin_ctzll(im))
+            sum = 0;
+        excl += wave_sum64(sum);
+        if (im)
+            break;
+    }
+    if (lane == 0)
+        st_publish(&status[t], kFlagInc | ((excl + agg) & kValMask));
+    while ((sp >> 62) != 2 && t != p0) {
+        if (++spins > kSpinLimit) {
+            if (lane == 0)
+                raise3(err, ZK_ERR_SPIN);
+            break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+        sp = st_poll(&status[p0 - 1]);
+    }
+    at = excl;
+    part = t == p0 ? excl : sp & kValMask;
+}
+
+// A wave's payloads (wider runs: a third of the lanes at a time), with the
+// reach of the writes past a block of few values.
+constexpr uint32_t kLaneBuf3 = 8192, kLaneReach3 = 8 + 4 * 64 + 16;
+static_assert(22 * 264 + kLaneReach3 <= kLaneBuf3, "a third of the widest payloads fits");
+
+template <uint32_t W>
+__global__ void __launch_bounds__(64 * W, 3) k3l_compress(Sz3Args a)
+{
+    __shared__ __attribute__((aligned(16))) uint32_t s_buf[W][kLaneBuf3 / 4];
+    __shared__ uint32_t s_tot[W], s_ticket;
+    __shared__ unsigned long long s_ex, s_part;
+    const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    if (threadIdx.x == 0)
+        s_ticket = (uint32_t) atomicAdd(&a.status[2], 1ull);
+    __syncthreads();
+    const uint32_t t = __builtin_amdgcn_readfirstlane(s_ticket);
+    const uint32_t pi = __builtin_amdgcn_readfirstlane(part_of_lane_tile(a.parts, a.g.T, t));
+    const Part3 p = a.parts[pi];
+    const uint32_t nbp = p.b1 * p.b2 * p.b3;
+    // this lane's block; the run's own blocks are those of lanes 1..63
+    const int32_t lbs = (int32_t) (kLaneRun3 * (W * (t - p.l0) + wv) + lane) - 1;
+    const bool own = lane > 0 && lbs < (int32_t) nbp;
+    const uint32_t lb = (uint32_t) min(max(lbs, 0), (int32_t) nbp - 1);
+    const uint32_t yz = p.b2 * p.b3;
+    const uint32_t bx = lb / yz, rest = lb - bx * yz, by = rest / p.b3, bz = rest - by * p.b3;
+    const uint32_t ex = min(4u, p.sx - 4 * bx), ey = min(4u, p.sy - 4 * by), ez = min(4u, p.sz - 4 * bz);
+    const bool hx = bx > 0, hy = by > 0, hz = bz > 0;
+    const bool edge = ex * ey * ez < 64;
+    const bool any_edge = __any(edge), any_z = __any(ez < 4);
+    // element offsets of rows -1..3 and values 1..3, clamped into the block and
+    // its halo (what a clamped load returns is masked)
+    const int32_t d3 = (int32_t) a.g.d3;
+    int32_t ro[5];
+#pragma unroll
+    for (int32_t j = 0; j < 5; j++)
+        ro[j] = min(max(j - 1, hy ? -1 : 0), (int32_t) ey - 1) * d3;
+    const uint32_t z1 = min(1u, ez - 1), z2 = min(2u, ez - 1), z3 = ez - 1;
+    const int64_t sx = (int64_t) a.g.d2 * d3;
+    const float* base = a.x + ((int64_t) (p.ox + 4 * bx) * a.g.d2 + (p.oy + 4 * by)) * (int64_t) d3 + p.oz + 4 * bz;
+    uint32_t m[64];
+    uint32_t ep[16];  // the plane before's differences along z and y
+#pragma unroll
+    for (uint32_t v = 0; v < 16; v++)
+        ep[v] = 0;
+    // (the next plane's rows are on their way while one is differenced)
+    float4 nx[5];
+    auto load = [&](int32_t i) {
+        const float* pl = base + min(max(i - 1, hx ? -1 : 0), (int32_t) ex - 1) * sx;
+#pragma unroll
+        for (uint32_t j = 0; j < 5; j++) {
+            const float* q = pl + ro[j];
+            if (any_z)
+                nx[j] = make_float4(q[0], q[z1], q[z2], q[z3]);
+            else
+                nx[j] = ldf4(q);
+        }
+    };
+    load(0);
+#pragma unroll
+    for (int32_t i = 0; i < 5; i++) {
+        float4 x[5];
+#pragma unroll
+        for (uint32_t j = 0; j < 5; j++)
+            x[j] = nx[j];
+        if (i < 4)
+            load(i + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        uint32_t dp[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (uint32_t j = 0; j < 5; j++) {
+            uint32_t q[4] = {(uint32_t) quant3(x[j].x, a.inv), (uint32_t) quant3(x[j].y, a.inv),
+                (uint32_t) quant3(x[j].z, a.inv), (uint32_t) quant3(x[j].w, a.inv)};
+            // the last value of the lane below (wave_shr:1), zero at z = 0
+            uint32_t qb = (uint32_t) __builtin_amdgcn_update_dpp(0, (int) q[3], 0x138, 0xF, 0xF, false);
+            qb = hz ? qb : 0u;
+            const bool out = (i == 0 && !hx) || (j == 0 && !hy);
+            uint32_t d[4];
+#pragma unroll
+            for (uint32_t k = 0; k < 4; k++)
+                d[k] = q[k] - (k ? q[k - 1] : qb);
+            if (i == 0 || j == 0) {
+#pragma unroll
+                for (uint32_t k = 0; k < 4; k++)
+                    d[k] = out ? 0u : d[k];
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < 4; k++) {
+                if (j > 0) {
+                    const uint32_t e = d[k] - dp[k];
+                    if (i > 0)
+                        m[16 * (i - 1) + 4 * (j - 1) + k] = e - ep[4 * (j - 1) + k];
+                    ep[4 * (j - 1) + k] = e;
+                }
+                dp[k] = d[k];
+            }
+        }
+    }
+    uint32_t* buf = s_buf[wv];
+    const uint32_t cnt = ex * ey * ez;
+    if (any_edge) {
+        // blocks at a far edge: their values closed up in order (through LDS,
+        // half the lanes at a time), zeros behind them
+        for (uint32_t h = 0; h < 2; h++) {
+            const bool mine = (lane >> 5) == h;
+            if (mine) {
+#pragma unroll
+                for (uint32_t v = 0; v < 64; v++)
+                    buf[32 * v + (lane & 31)] = m[v];
+            }
+            wave_sync_lds();
+            if (mine && edge) {
+                uint32_t at = lane & 31, j = 0, k = 0;  // at: of value (i, j, k)
+                const uint32_t ey1 = stay(ey), ez1 = stay(ez);
+#pragma unroll
+                for (uint32_t e = 0; e < 64; e++) {
+                    const uint32_t v = buf[min(at, 32u * 63 + 31)];
+                    m[e] = e < cnt ? v : 0u;
+                    k++;
+                    at += 32;
+                    const bool row = k == ez1;
+                    at += row ? 32 * (4 - ez1) : 0u;
+                    j += row ? 1u : 0u;
+                    k = row ? 0u : k;
+                    const bool plane = j == ey1;
+                    at += plane ? 128 * (4 - ey1) : 0u;
+                    j = plane ? 0u : j;
+                }
+            }
+            wave_sync_lds();
+        }
+    }
+    // signs, magnitudes, width and size
+    uint32_t s0 = 0, s1 = 0, mx = 0;
+#pragma unroll
+    for (uint32_t v = 0; v < 64; v++) {
+        if (v < 32)
+            s0 = __builtin_amdgcn_alignbit(s0, m[v], 31);  // (s0 << 1) | sign of value v
+        else
+            s1 = __builtin_amdgcn_alignbit(s1, m[v], 31);
+        m[v] = mag(m[v]);
+        mx = max(mx, m[v]);
+    }
+    const uint32_t w = own && mx ? 32u - (uint32_t) __clz((int) mx) : 0u;
+    const uint32_t size = payload3(w, cnt);
+    const uint32_t incl = wave_scan_dpp(size), excl = incl - size;
+    const uint32_t wtot = __builtin_amdgcn_readlane(incl, 63);
+    if (lane == 0)
+        s_tot[wv] = wtot;
+    __syncthreads();
+    uint32_t woff = 0, total = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < W; i++) {
+        const uint32_t v = s_tot[i];
+        woff += i < wv ? v : 0u;
+        total += v;
+    }
+    if (threadIdx.x == 0)
+        st_publish(&a.offs[t], (t ? kFlagAgg : kFlagInc) | total);
+    const bool one = wtot + kLaneReach3 <= kLaneBuf3;
+    uint8_t* dst = nullptr;
+    bool fits = false;
+    for (uint32_t q = 0; q < (one ? 1u : 3u); q++) {
+        // the lanes of this round, their bytes [b0, b1) of the wave's
+        const uint32_t b0 = q ? __builtin_amdgcn_readlane(excl, 22 * q) : 0u;
+        const uint32_t b1 = one || q == 2 ? wtot : __builtin_amdgcn_readlane(excl, 22 * (q + 1));
+        const uint32_t wq = one || lane / 22 == q ? w : 0u, o = excl - b0;
+        for (uint32_t i = lane; i < (b1 - b0 + 32 + 15) / 16; i += 64)
+            reinterpret_cast<uint4*>(buf)[i] = make_uint4(0, 0, 0, 0);
+        wave_sync_lds();
+        if (wq) {
+            const uint32_t sb[2] = {__builtin_bswap32(s0), __builtin_bswap32(s1)};
+            or_words(buf, o, sb);
+        }
+        const uint32_t hp = o + ((cnt + 7) >> 3);
+        if (__any(wq >= 8))
+            encode_high_class(buf, hp, wq, m);
+        encode_low(buf, hp + cnt * (wq >> 3), wq, m);
+        if (q == 0) {
+            if (wv == 0) {
+                unsigned long long at, part;
+                places3(a.offs, t, p.l0, total, a.status, at, part);
+                if (lane == 0) {
+                    s_ex = at;
+                    s_part = part;
+                }
+            }
+            __syncthreads();
+            const uint64_t P = 8ull * a.g.T + p.nbc + nbp + s_ex;  // the tile's first payload byte
+            fits = P + total <= a.out_cap;
+            dst = a.out + P + woff;
+        }
+        wave_sync_lds();
+        if (fits)
+            store_wave(buf, dst + b0, b1 - b0);
+        wave_sync_lds();
+    }
+    const uint64_t sub = (uint64_t) p.nbc + s_part;  // sub-volume start after the header
+    if (!fits && threadIdx.x == 0)
+        raise3(a.status, ZK_ERR_NOSPACE);
+    if (own && 8ull * a.g.T + sub + nbp <= a.out_cap)
+        a.out[8ull * a.g.T + sub + lb] = (uint8_t) w;
+    if (threadIdx.x == 0) {
+        if (t == p.l0 && 8ull * (pi + 1) <= a.out_cap)
+            __builtin_memcpy(a.out + 8ull * pi, &sub, 8);
+        if (t == a.g.nlane - 1) {
+            // the last tile ends the stream: if it fits, every tile fits
+            const unsigned long long all = 8ull * a.g.T + a.g.nblocks + s_ex + total;
+            a.status[0] = all;
+            if (a.size_out)
+                *a.size_out = all > a.out_cap ? 0ull : all;
+        }
+    }
+}
+
 }  // namespace
 
 static hipError_t scan3(const Sz3Args& a, int check_cap, hipStream_t s)
@@ -871,9 +1180,11 @@ static hipError_t scan3(const Sz3Args& a, int check_cap, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_sz3_table(const Geom3& g, Part3* parts, unsigned long long* status, hipStream_t s)
+hipError_t launch_sz3_table(const Geom3& g, Part3* parts, unsigned long long* status, unsigned long long* clear,
+    uint32_t nclear, hipStream_t s)
 {
-    hipLaunchKernelGGL(k3_table, dim3(1), dim3(64), 0, s, g.d1, g.d2, g.d3, (int) g.Bs, (int) g.T, parts, status);
+    hipLaunchKernelGGL(k3_table, dim3(1 + std::min(nclear / 256, 255u)), dim3(256), 0, s, g.d1, g.d2, g.d3, (int) g.Bs,
+        (int) g.T, parts, status, clear, nclear);
     return hipGetLastError();
 }
 
@@ -903,8 +1214,13 @@ static hipError_t decompress_tiled(const Sz3Args& a, hipStream_t s)
 
 hipError_t launch_sz3_compress(const Sz3Args& a, hipStream_t s)
 {
-    if (a.g.nunits && a.g.Bs == 4)
-        return compress_tiled<4>(a, s);
+    if (a.g.nlane) {
+        if (a.g.wlane == kLaneSlim3)
+            hipLaunchKernelGGL(k3l_compress<kLaneSlim3>, dim3(a.g.nlane), dim3(64 * kLaneSlim3), 0, s, a);
+        else
+            hipLaunchKernelGGL(k3l_compress<kLaneWide3>, dim3(a.g.nlane), dim3(64 * kLaneWide3), 0, s, a);
+        return hipGetLastError();
+    }
     if (a.g.nunits && a.g.Bs == 8)
         return compress_tiled<8>(a, s);
     const uint32_t waves = (uint32_t) ceil_div(a.g.nblocks, 4);
