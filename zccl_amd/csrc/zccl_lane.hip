@@ -1217,6 +1217,14 @@ static_assert(kCompBuf >= kLaneTileBlocks * kWorstBlock + 64 && kCompBuf >= (kLa
     "a compress wave buffer holds the staged values and the worst-case encode");
 static_assert(kCompBuf % 16 == 0, "compress wave buffers stay 16-byte aligned");
 
+// Tiles a workgroup takes with one ticket.  Tickets are adds to one address, 12
+// ns each: the 1820 of a 2^24-value stream took 22 us of the kernel's 47; two
+// tiles a ticket: 37 us (four: 34, but 136 us against 116 for the 8 streams of a
+// staged allreduce, whose tiles then end together).  Up to kCompFew tiles, one
+// for each compute unit, a tile has a workgroup of its own (7 tiles: 9.4 us
+// against 10.1).
+constexpr uint32_t kCompPair = 2, kCompFew = 256;
+
 struct CompShared {
     uint32_t wtot[kLaneWaves];
     unsigned long long ex;
@@ -1224,16 +1232,16 @@ struct CompShared {
 
 __device__ __forceinline__ void compress_tile_lane(const Geom& g, const Tiling& tl, double inv, const float* xin,
     uint8_t* out, uint64_t out_cap, uint8_t* oindex, unsigned long long* size_out, uint64_t t,
-    unsigned long long* status, WsHeader* ws, uint32_t nchains, uint32_t* obuf, CompShared& sh)
+    unsigned long long* status, WsHeader* ws, uint32_t nchains, uint32_t* obuf, CompShared& sh, bool live)
 {
     round_toward_zero();
-    const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const uint32_t lane = threadIdx.x & 63, wv = (threadIdx.x >> 6) % kLaneWaves;  // wave of the tile
     const Tile x = tile_of(g, tl, (uint32_t) t);
     const uint32_t jb = kLaneTileBlocks * wv + lane;  // block of the tile
-    const bool has = jb < x.nblk;
+    const bool has = live & (jb < x.nblk);
     const uint32_t nj = has ? min(tile_block_len(g, x, jb), L) : 0u;
     // the wave's values
-    const uint32_t nbw = x.nblk > kLaneTileBlocks * wv ? min(x.nblk - kLaneTileBlocks * wv, kLaneTileBlocks) : 0u;
+    const uint32_t nbw = (live & (x.nblk > kLaneTileBlocks * wv)) ? min(x.nblk - kLaneTileBlocks * wv, kLaneTileBlocks) : 0u;
     const uint32_t nvals = nbw ? (nbw - 1) * L + min(tile_block_len(g, x, kLaneTileBlocks * wv + nbw - 1), L) : 0u;
     const uint32_t v0 = x.e0 + kLaneTileBlocks * L * wv;  // input index of the wave's first value
     float xb = 0.0f;                                      // lane 0: the value before it
@@ -1329,7 +1337,7 @@ __device__ __forceinline__ void compress_tile_lane(const Geom& g, const Tiling& 
         woff += i < wv ? v : 0u;
         total += v;
     }
-    if (threadIdx.x == 0)
+    if (live & ((wv | lane) == 0))
         lookback_publish(status, t, 0, total, 0);  // successors see the aggregate now
     const uint32_t nz = (wtot + 64 + 15) / 16;
     for (uint32_t i = lane; i < nz; i += 64)
@@ -1337,19 +1345,21 @@ __device__ __forceinline__ void compress_tile_lane(const Geom& g, const Tiling& 
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     encode_blocks(obuf, excl, w, nj, s, s2, m);
-    if (wv == 0) {
+    if (live & (wv == 0)) {
         const unsigned long long ex = lookback(status, t, 0, total, 0, ws, true);
         if (lane == 0)
             sh.ex = ex;
     }
     __syncthreads();
+    if (!live)
+        return;
     const uint64_t P = 8ull * g.T + 4ull * (x.s + 1) + sh.ex;
     const bool fits = P + total <= out_cap;
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     if (fits)
         store_wave(obuf, out + P + woff, wtot);
-    else if (threadIdx.x == 0)
+    else if ((wv | lane) == 0)
         raise_error(ws, ZK_ERR_NOSPACE);
     IndexView ox = index_view(g, oindex);
     const uint32_t ct = (x.s < g.T ? x.s * g.cT : g.T * g.cT) + kLaneWaves * x.lt + wv;  // the wave's lane tile
@@ -1359,7 +1369,7 @@ __device__ __forceinline__ void compress_tile_lane(const Geom& g, const Tiling& 
         ox.widths[x.g0 + jb] = (uint8_t) w;
     if (has && (jb % g.IG) == 0)
         ox.group_off[x.grp0 + jb / g.IG] = P + woff + excl;
-    if (threadIdx.x == 0) {
+    if ((wv | lane) == 0) {
         if (x.nblk == 0 && x.ngrp)
             ox.group_off[x.grp0] = P;  // a segment of its seed alone keeps one group entry
         if (x.lt == 0) {
@@ -1498,24 +1508,34 @@ __global__ void __launch_bounds__(kCarryScanThreads) k_lane_carry_scan(Decompres
 
 // Compress in the lane layout: one stream, a uniform batch (shared geometry
 // and bound, per-job pointers, tiles of the jobs interleaved) or a mixed one.
-__global__ void __launch_bounds__(64 * kLaneWaves, 4) k_compress_lane(CompressArgs a)
+template <uint32_t N>
+__global__ void __launch_bounds__(64 * kLaneWaves * N, 4) k_compress_lane(CompressArgs a)
 {
-    __shared__ CompShared sh;
+    __shared__ CompShared sh[N];
+    const uint32_t part = __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * kLaneWaves));
     uint64_t t;
     unsigned long long* status;
-    if (!launch_status(a.ws, a.job.tl.ntiles, t, status))
+    if (!launch_status(a.ws, a.job.tl.ntiles, t, status, N))
         return;
+    t += part;
+    const bool live = t < a.job.tl.ntiles;
     compress_tile_lane(a.job.g, a.job.tl, a.job.p.inv, a.job.io.x, a.job.io.out, a.job.io.out_cap, a.job.io.index,
-        a.job.io.size_out, t, status, a.ws, 1, zk_lds + (threadIdx.x >> 6) * (kCompBuf / 4), sh);
+        a.job.io.size_out, live ? t : 0, status, a.ws, 1, zk_lds + (threadIdx.x >> 6) * (kCompBuf / 4), sh[part], live);
 }
 
-__global__ void __launch_bounds__(64 * kLaneWaves, 4) k_compress_lane_batch(BatchArgs b)
+template <uint32_t N>
+__global__ void __launch_bounds__(64 * kLaneWaves * N, 4) k_compress_lane_batch(BatchArgs b)
 {
-    __shared__ CompShared sh;
+    __shared__ CompShared sh[N];
+    const uint32_t part = __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * kLaneWaves));
     uint64_t tg;
     unsigned long long* status;
-    if (!launch_status(b.ws, b.total_tiles, tg, status))
+    if (!launch_status(b.ws, b.total_tiles, tg, status, N))
         return;
+    tg += part;
+    const bool live = tg < b.total_tiles;
+    if (!live)
+        tg = b.total_tiles - 1;
     uint32_t jidx, t;
     if (b.interleave) {
         jidx = (uint32_t) tg % b.njobs;
@@ -1529,16 +1549,22 @@ __global__ void __launch_bounds__(64 * kLaneWaves, 4) k_compress_lane_batch(Batc
     const CompressIO* io = (const CompressIO*) b.jobs + jidx;
     compress_tile_lane(b.g, b.tl, b.p.inv, ldc(&io->x), ldc(&io->out), ldc(&io->out_cap), ldc(&io->index),
         ldc(&io->size_out), t, status + (uint64_t) jidx * b.tl.ntiles * kStatusStride, b.ws, b.total_chains,
-        zk_lds + (threadIdx.x >> 6) * (kCompBuf / 4), sh);
+        zk_lds + (threadIdx.x >> 6) * (kCompBuf / 4), sh[part], live);
 }
 
-__global__ void __launch_bounds__(64 * kLaneWaves, 4) k_compress_lane_mixed(BatchArgs b)
+template <uint32_t N>
+__global__ void __launch_bounds__(64 * kLaneWaves * N, 4) k_compress_lane_mixed(BatchArgs b)
 {
-    __shared__ CompShared sh;
+    __shared__ CompShared sh[N];
+    const uint32_t part = __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * kLaneWaves));
     uint64_t tg;
     unsigned long long* status;
-    if (!launch_status(b.ws, b.total_tiles, tg, status))
+    if (!launch_status(b.ws, b.total_tiles, tg, status, N))
         return;
+    tg += part;
+    const bool live = tg < b.total_tiles;
+    if (!live)
+        tg = b.total_tiles - 1;
     uint32_t lo = 0, hi = b.njobs;
     while (hi - lo > 1) {
         const uint32_t mid = (lo + hi) / 2;
@@ -1555,7 +1581,7 @@ __global__ void __launch_bounds__(64 * kLaneWaves, 4) k_compress_lane_mixed(Batc
     const Tiling tl = job->tl;
     compress_tile_lane(g, tl, ldc(&job->p.inv), ldc(&job->io.x), ldc(&job->io.out), ldc(&job->io.out_cap),
         ldc(&job->io.index), ldc(&job->io.size_out), t, status + tile0 * kStatusStride, b.ws, b.total_chains,
-        zk_lds + (threadIdx.x >> 6) * (kCompBuf / 4), sh);
+        zk_lds + (threadIdx.x >> 6) * (kCompBuf / 4), sh[part], live);
 }
 
 // Single-pass sum with a lookback tile per workgroup (layout 2): the
@@ -1976,24 +2002,30 @@ hipError_t launch_homsum_lane_wg_batch(const BatchArgs& b, hipStream_t s)
     return hipGetLastError();
 }
 
-size_t compress_lane_lds_bytes() { return (size_t) kLaneWaves * kCompBuf; }
+// Workgroups of N tiles each (kCompFew: where the line lies).
+template <uint32_t N, typename K, typename A>
+static hipError_t launch_comp(K kernel, uint64_t ntiles, const A& args, hipStream_t s)
+{
+    hipLaunchKernelGGL(kernel, dim3((uint32_t) ceil_div(ntiles, N)), dim3(64 * kLaneWaves * N), N * kLaneWaves * kCompBuf,
+        s, args);
+    return hipGetLastError();
+}
 
 hipError_t launch_compress_lane(const CompressArgs& a, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_compress_lane, dim3((uint32_t) a.job.tl.ntiles), dim3(64 * kLaneWaves),
-        compress_lane_lds_bytes(), s, a);
-    return hipGetLastError();
+    const uint64_t n = a.job.tl.ntiles;
+    return n > kCompFew ? launch_comp<kCompPair>(k_compress_lane<kCompPair>, n, a, s) :
+                          launch_comp<1>(k_compress_lane<1>, n, a, s);
 }
 
 hipError_t launch_compress_lane_batch(const BatchArgs& b, hipStream_t s)
 {
+    const uint64_t n = b.total_tiles;
     if (b.uniform)
-        hipLaunchKernelGGL(k_compress_lane_batch, dim3((uint32_t) b.total_tiles), dim3(64 * kLaneWaves),
-            compress_lane_lds_bytes(), s, b);
-    else
-        hipLaunchKernelGGL(k_compress_lane_mixed, dim3((uint32_t) b.total_tiles), dim3(64 * kLaneWaves),
-            compress_lane_lds_bytes(), s, b);
-    return hipGetLastError();
+        return n > kCompFew ? launch_comp<kCompPair>(k_compress_lane_batch<kCompPair>, n, b, s) :
+                              launch_comp<1>(k_compress_lane_batch<1>, n, b, s);
+    return n > kCompFew ? launch_comp<kCompPair>(k_compress_lane_mixed<kCompPair>, n, b, s) :
+                          launch_comp<1>(k_compress_lane_mixed<1>, n, b, s);
 }
 
 hipError_t launch_homsum_lane_staged(const HomsumArgs& a, uint8_t* stage, hipStream_t s)
