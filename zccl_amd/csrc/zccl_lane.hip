@@ -1399,12 +1399,20 @@ __device__ __forceinline__ void compress_tile_lane(const Geom& g, const Tiling& 
 
 }  // namespace
 
+// Waves (tiles) that share a ticket of a sum: tickets are adds to one address,
+// 12 ns each, so beyond kSumFew tiles, which fill the chip's 1024 SIMDs with four
+// waves each, they bound the kernel and eight waves share one (32 mixed buckets:
+// 88.6 -> 79.2 us); below, smaller workgroups start sooner (868 tiles of 4
+// operands: 34.0 us, with eight 38.4).
+constexpr uint32_t kSumMany = 8, kSumFew = 4096;
+
 // One fused sum (kernel arguments hold its geometry and pointers).
-__global__ void __launch_bounds__(64 * kLaneWaves, 4) k_homsum_lane(HomsumArgs a)
+template <uint32_t W>
+__global__ void __launch_bounds__(64 * W, 4) k_homsum_lane(HomsumArgs a)
 {
     uint64_t t0;
     unsigned long long* status;
-    if (!launch_status(a.ws, a.job.tl.ntiles, t0, status, kLaneWaves))
+    if (!launch_status(a.ws, a.job.tl.ntiles, t0, status, W))
         return;
     const uint32_t wv = threadIdx.x >> 6;
     const uint64_t t = t0 + wv;
@@ -1417,11 +1425,12 @@ __global__ void __launch_bounds__(64 * kLaneWaves, 4) k_homsum_lane(HomsumArgs a
 
 // Uniform batch: shared geometry, per-job pointers in device memory; tiles of
 // the jobs interleave (tile b is tile b / njobs of job b % njobs).
-__global__ void __launch_bounds__(64 * kLaneWaves, 4) k_homsum_lane_batch(BatchArgs b)
+template <uint32_t W>
+__global__ void __launch_bounds__(64 * W, 4) k_homsum_lane_batch(BatchArgs b)
 {
     uint64_t t0;
     unsigned long long* status;
-    if (!launch_status(b.ws, b.total_tiles, t0, status, kLaneWaves))
+    if (!launch_status(b.ws, b.total_tiles, t0, status, W))
         return;
     const uint32_t wv = threadIdx.x >> 6;
     const uint64_t tg = t0 + wv;
@@ -1446,11 +1455,12 @@ __global__ void __launch_bounds__(64 * kLaneWaves, 4) k_homsum_lane_batch(BatchA
 
 // Mixed batch: every job carries its own geometry; job j owns launch tiles
 // [job_tile0[j], job_tile0[j+1]).
-__global__ void __launch_bounds__(64 * kLaneWaves, 4) k_homsum_lane_mixed(BatchArgs b)
+template <uint32_t W>
+__global__ void __launch_bounds__(64 * W, 4) k_homsum_lane_mixed(BatchArgs b)
 {
     uint64_t t0;
     unsigned long long* status;
-    if (!launch_status(b.ws, b.total_tiles, t0, status, kLaneWaves))
+    if (!launch_status(b.ws, b.total_tiles, t0, status, W))
         return;
     const uint32_t wv = threadIdx.x >> 6;
     const uint64_t tg = t0 + wv;
@@ -1908,21 +1918,29 @@ __global__ void __launch_bounds__(64 * kLaneWaves) k_place_lane_batch(BatchArgs 
 
 size_t lane_lds_bytes() { return (size_t) kLaneWaves * kOutBuf; }
 
+// Workgroups of W waves, one ticket each.
+template <uint32_t W, typename K, typename A>
+static hipError_t launch_sum(K kernel, uint64_t ntiles, const A& args, hipStream_t s)
+{
+    hipLaunchKernelGGL(kernel, dim3((uint32_t) ceil_div(ntiles, W)), dim3(64 * W), W * kOutBuf, s, args);
+    return hipGetLastError();
+}
+
 hipError_t launch_homsum_lane(const HomsumArgs& a, hipStream_t s)
 {
-    const uint32_t groups = (uint32_t) ceil_div(a.job.tl.ntiles, kLaneWaves);
-    hipLaunchKernelGGL(k_homsum_lane, dim3(groups), dim3(64 * kLaneWaves), lane_lds_bytes(), s, a);
-    return hipGetLastError();
+    const uint64_t n = a.job.tl.ntiles;
+    return n > kSumFew ? launch_sum<kSumMany>(k_homsum_lane<kSumMany>, n, a, s) :
+                         launch_sum<kLaneWaves>(k_homsum_lane<kLaneWaves>, n, a, s);
 }
 
 hipError_t launch_homsum_lane_batch(const BatchArgs& b, hipStream_t s)
 {
-    const uint32_t groups = (uint32_t) ceil_div(b.total_tiles, kLaneWaves);
+    const uint64_t n = b.total_tiles;
     if (b.uniform)
-        hipLaunchKernelGGL(k_homsum_lane_batch, dim3(groups), dim3(64 * kLaneWaves), lane_lds_bytes(), s, b);
-    else
-        hipLaunchKernelGGL(k_homsum_lane_mixed, dim3(groups), dim3(64 * kLaneWaves), lane_lds_bytes(), s, b);
-    return hipGetLastError();
+        return n > kSumFew ? launch_sum<kSumMany>(k_homsum_lane_batch<kSumMany>, n, b, s) :
+                             launch_sum<kLaneWaves>(k_homsum_lane_batch<kLaneWaves>, n, b, s);
+    return n > kSumFew ? launch_sum<kSumMany>(k_homsum_lane_mixed<kSumMany>, n, b, s) :
+                         launch_sum<kLaneWaves>(k_homsum_lane_mixed<kLaneWaves>, n, b, s);
 }
 
 // (four: what the LDS buffers let a CU hold)
