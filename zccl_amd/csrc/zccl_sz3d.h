@@ -38,6 +38,10 @@ struct Part3 {
     uint32_t u0;           // first chunk of the tiled compress (block side 8)
     uint32_t c0;           // first block column (bx, by) of the tiled decoder
     uint32_t l0;           // first workgroup tile of the lane compress (block side 4)
+    uint32_t v0;           // lane decoder: first run of 64 blocks along z
+    uint32_t d0;           // its first workgroup (a row of blocks along z, kLaneSeg3 of them along x)
+    uint32_t t0;           // first of its segments' last planes
+    uint32_t h0;           // first column (bx, z) of its y pass
 };
 
 struct Geom3 {
@@ -49,6 +53,12 @@ struct Geom3 {
     uint32_t ncols;        // block columns of the tiled decoder
     uint32_t nlane;        // workgroup tiles of the lane compress (0: not that path)
     uint32_t wlane;        // waves of such a tile
+    uint32_t nruns;        // runs of the lane decoder (0: not that path)
+    uint32_t nrows;        // its workgroups
+    uint32_t ntail;        // values of its segments' last planes
+    uint32_t nhcol;        // columns of its y pass
+    uint32_t wruns;        // runs (waves) to a row
+    uint32_t edges;        // some sub-volume has blocks of fewer values
 };
 
 // Blocks per chunk along z of the tiled kernels: a chunk is one (bx, by)
@@ -66,6 +76,15 @@ constexpr uint32_t kLaneRun3 = 63;
 constexpr uint32_t kLaneSlim3 = 4, kLaneWide3 = 12;
 constexpr uint64_t kLaneFew3 = 64ull * kLaneRun3 * kLaneWide3 * 256;
 constexpr uint32_t kLaneMaxRow3 = 1u << 27;
+
+// Lane decoder (block side 4): one lane per block, a wave per run of 64 blocks
+// along z (kLaneRuns3 to a row at most), a workgroup per row of blocks and
+// kLaneSeg3 blocks along x.  Rows shorter than kLaneMinB3 blocks leave most
+// lanes idle and take the tiled kernels (16 sub-volumes, us by lanes / tiled:
+// 256^3, 32 blocks a row: 111 / 143; 180^3, 23 blocks: 112 / 106; 128^3, 16: 72 /
+// 70).  The last plane of every segment but a
+// sub-volume's last is kept for the y pass: at most 8 bytes per block.
+constexpr uint32_t kLaneSeg3 = 8, kLaneMinB3 = 32, kLaneRuns3 = 4;
 
 // Factorise T over three dims as My_Dims_create (ZCCL/src/ZCCL_multidim.c:
 // 100-140): prime factors of T, largest first, each multiplied into the
@@ -128,7 +147,8 @@ ZK_HD bool make_geom3(uint64_t d1, uint64_t d2, uint64_t d3, int Bs, int T, Geom
     const bool lane = Bs == 4 && g->d3 < kLaneMaxRow3;
     g->wlane = (uint64_t) g->d1 * g->d2 * g->d3 < kLaneFew3 ? kLaneSlim3 : kLaneWide3;
     const uint32_t lane_tile = g->wlane * kLaneRun3;
-    uint32_t r = 0, ox = 0, nb = 0, zr = 0, yc = 0, xc = 0, nu = 0, nc = 0, nl = 0;
+    uint32_t r = 0, ox = 0, nb = 0, zr = 0, yc = 0, xc = 0, nu = 0, nc = 0, nl = 0, nv = 0, nd = 0, nt = 0, nh = 0;
+    uint32_t b3lo = ~0u, b3hi = 0, odd = 0;
     for (int px = 0; px < td[0]; px++) {
         const uint32_t sx = bx + ((uint32_t) px < rx ? 1u : 0u);
         uint32_t oy = 0;
@@ -149,6 +169,17 @@ ZK_HD bool make_geom3(uint64_t d1, uint64_t d2, uint64_t d3, int Bs, int T, Geom
                 p.u0 = nu;
                 p.c0 = nc;
                 p.l0 = nl;
+                p.v0 = nv;
+                p.d0 = nd;
+                p.t0 = nt;
+                p.h0 = nh;
+                nv += p.b1 * p.b2 * ((p.b3 + 63) / 64);
+                nd += p.b2 * ((p.b1 + kLaneSeg3 - 1) / kLaneSeg3);
+                nt += ((p.b1 + kLaneSeg3 - 1) / kLaneSeg3 - 1) * p.sy * p.sz;
+                nh += p.b1 * p.sz;
+                odd |= (p.sx | p.sy | p.sz) & 3;  // (block side 4)
+                b3lo = p.b3 < b3lo ? p.b3 : b3lo;
+                b3hi = p.b3 > b3hi ? p.b3 : b3hi;
                 nl += lane ? (p.b1 * p.b2 * p.b3 + lane_tile - 1) / lane_tile : 0u;
                 nu += nz ? p.b1 * p.b2 * ((p.b3 + nz - 1) / nz) : 0u;
                 nc += p.b1 * p.b2;
@@ -169,6 +200,13 @@ ZK_HD bool make_geom3(uint64_t d1, uint64_t d2, uint64_t d3, int Bs, int T, Geom
     g->nunits = nu;
     g->ncols = nc;
     g->nlane = nl;
+    const bool runs = Bs == 4 && b3lo >= kLaneMinB3 && b3hi <= 64 * kLaneRuns3;
+    g->nruns = runs ? nv : 0u;
+    g->nrows = nd;
+    g->ntail = nt;
+    g->nhcol = nh;
+    g->wruns = (b3hi + 63) / 64;
+    g->edges = odd ? 1u : 0u;
     return true;
 }
 

@@ -12,7 +12,9 @@
 //              payload sizes -> k3_encode (one wave per block: width header
 //              byte, sub-volume offset, sign bitmap and fixed-length bits with
 //              the one-writer-per-byte unit encoder of the 1-D sum)
-//   decompress k3_table -> k3_dsizes (widths read from the stream's own
+//   decompress k3_table -> for block side 4 and rows of 32 to 256 blocks
+//              k3l_sizes, k3l_decode, k3l_ypass (one lane per block, two passes
+//              over the volume); others k3_dsizes (widths read from the stream's own
 //              header) -> scan -> k3_decode (residuals into the output buffer
 //              as int32) -> k3_zpass / k3_ypass (inclusive prefix sums along z
 //              and y) -> k3_xpass (along x, then x' = (float)(q * 2 eb) in place)
@@ -1169,6 +1171,390 @@ __global__ void __launch_bounds__(64 * W, 3) k3l_compress(Sz3Args a)
     }
 }
 
+// ---------------------------------------------------------- lane decompress
+// Block side 4.  The 3-D prefix sum of the residuals, in two passes over the
+// volume: k3l_decode decodes a row of blocks along z with one lane per block,
+// sums along x in registers (kLaneSeg3 blocks one after the other, the last plane
+// of the segment kept aside) and along z by wave scans, and writes the integers;
+// k3l_ypass sums along y, adds the segments before its own and dequantizes in
+// place.  The residuals never reach memory, which the tiled decoder's chunks
+// wrote (330 us for a 512^3 volume at a relative bound of 1e-3), the y pass (248)
+// and the x pass (238) read and wrote again: 849 us with the sizes.  This takes
+// 391: decode 146 (512 MB written; four waves a SIMD, 142 us at its registers'
+// limit, 176 with three), y pass 206 (1 GB at 5.2 TB/s, a copy reaches 5.5),
+// sizes and kept planes 30.  Volumes with blocks of fewer values (Edges) need 156
+// registers to move those to their places: 510^3 962 -> 565 us; in one kernel for
+// both 512^3 took 493.
+
+// Bytes of every run of 64 blocks, one lane per run: words[] holds the exclusive
+// sums within 256 runs, part_sums[] the groups' sums (scanned by k3_scan_top).
+__global__ void __launch_bounds__(256) k3l_sizes(Sz3Args a)
+{
+    __shared__ uint32_t s_w[4];
+    const uint32_t u = blockIdx.x * 256 + threadIdx.x;
+    uint32_t sum = 0;
+    if (u < a.g.nruns) {
+        uint32_t lo = 0, hi = a.g.T;
+        while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) / 2;
+            if (a.parts[mid].v0 <= u)
+                lo = mid;
+            else
+                hi = mid;
+        }
+        const Part3 p = a.parts[lo];
+        const uint32_t nz = (p.b3 + 63) / 64, rel = u - p.v0, row = rel / nz, z0 = 64 * (rel - row * nz);
+        const uint32_t bx = row / p.b2, by = row - bx * p.b2;
+        const uint32_t face = min(4u, p.sx - 4 * bx) * min(4u, p.sy - 4 * by), n = min(64u, p.b3 - z0);
+        uint64_t h;
+        __builtin_memcpy(&h, a.in + 8ull * lo, 8);
+        const uint64_t pos = 8ull * a.g.T + h + (uint64_t) row * p.b3 + z0;
+        uint32_t far = 0;
+        bool past = false;
+#pragma unroll 8
+        for (uint32_t i = 0; i < n; i++) {
+            const bool in = pos + i < a.in_size;
+            uint32_t w = in ? a.in[pos + i] : 0u;
+            past |= !in;
+            far = max(far, w);
+            w = w > 32 ? 0u : w;
+            sum += payload3(w, face * min(4u, p.sz - 4 * (z0 + i)));
+        }
+        if (far > 32)
+            raise3(a.status, ZK_ERR_WIDTH);
+        if (past)
+            raise3(a.status, ZK_ERR_OVERRUN);
+    }
+    const uint32_t inc = wave_scan_dpp(sum);
+    if ((threadIdx.x & 63) == 63)
+        s_w[threadIdx.x >> 6] = inc;
+    __syncthreads();
+    uint32_t pre = 0, all = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < 4; w++) {
+        pre += w < (threadIdx.x >> 6) ? s_w[w] : 0u;
+        all += s_w[w];
+    }
+    if (u < a.g.nruns)
+        a.words[u] = pre + inc - sum;
+    if (threadIdx.x == 0)
+        a.part_sums[blockIdx.x] = all;
+}
+
+// Residuals of a block of width w and cnt values in stream order, its payload at
+// byte o of st; those past cnt are garbage.
+__device__ __forceinline__ void decode_block3(const uint32_t* st, uint32_t o, uint32_t w, uint32_t cnt, uint32_t (&m)[64])
+{
+    const uint32_t r = w & 7, B = w >> 3;
+    const uint32_t hp = o + ((cnt + 7) >> 3);
+    const uint32_t sh[4] = {32 - r, 32 - 2 * r, 32 - 3 * r, 32 - 4 * r};
+    uint32_t a = hp + B * cnt;
+#pragma unroll
+    for (uint32_t g = 0; g < 8; g++, a += r) {
+        __builtin_amdgcn_sched_barrier(0);  // group by group: few registers live
+        const uint32_t* pg = st + (a >> 2);
+        const uint32_t E0 = pg[0], E1 = pg[1], E2 = pg[2];
+        const uint32_t e0 = __builtin_bswap32(__builtin_amdgcn_alignbyte(E1, E0, a));
+        const uint32_t e1 = __builtin_bswap32(__builtin_amdgcn_alignbyte(E2, E1, a));
+        const uint32_t e4 = __builtin_amdgcn_alignbit(e0, e1, sh[3]);
+#pragma unroll
+        for (uint32_t c = 0; c < 8; c++)
+            m[8 * g + c] = __builtin_amdgcn_ubfe(c < 4 ? e0 : e4, sh[c & 3], r);
+    }
+    if (__any(B == 1)) {
+        const uint32_t hb = B == 1 ? 8u : 0u;
+#pragma unroll
+        for (uint32_t i = 0; i < 16; i++) {
+            const uint32_t h = lds_at(st, hp + 4 * i);
+#pragma unroll
+            for (uint32_t c = 0; c < 4; c++)
+                m[4 * i + c] |= __builtin_amdgcn_ubfe(h, 8 * c, hb) << r;
+        }
+    }
+    if (__any(B >= 2)) {
+        const uint32_t hm = B >= 4 ? ~0u : B >= 2 ? (1u << (8 * B)) - 1u : 0u;
+#pragma unroll
+        for (uint32_t e = 0; e < 64; e++) {
+            if (e % 4 == 0)
+                __builtin_amdgcn_sched_barrier(0);
+            m[e] |= (lds_at(st, hp + e * B) & hm) << r;
+        }
+    }
+    const uint32_t s0 = __builtin_bswap32(lds_at(st, o)), s1 = __builtin_bswap32(lds_at(st, o + 4));
+#pragma unroll
+    for (uint32_t e = 0; e < 64; e++) {
+        const uint32_t sg = (uint32_t) __builtin_amdgcn_sbfe((int32_t) (e < 32 ? s0 : s1), 31 - (e & 31), 1);
+        m[e] = (m[e] ^ sg) - sg;
+    }
+}
+
+// Rows of four values of blocks with N rows to a plane, from stream order to
+// their places; zeros in the rows the blocks don't have.
+template <uint32_t N>
+__device__ __forceinline__ void spread_rows3(uint32_t (&m)[64])
+{
+#pragma unroll
+    for (uint32_t v = 64; v-- > 0;) {
+        const uint32_t i = v / 16, j = (v / 4) % 4, k = v % 4;
+        m[v] = j < N ? m[4 * (i * N + j) + k] : 0u;
+    }
+}
+
+// A wave's payloads (longer runs: a third of the lanes at a time), with the
+// reach of the reads past a block of few values.
+constexpr uint32_t kRunBuf3 = 6144, kRunReach3 = 8 + 4 * 64 + 16;
+static_assert(22 * 264 + kRunReach3 <= kRunBuf3, "a third of the widest payloads fits");
+
+template <uint32_t W, bool Edges>
+__global__ void __launch_bounds__(64 * W, Edges ? 3 : 4) k3l_decode(Sz3Args a)
+{
+    __shared__ __attribute__((aligned(16))) uint32_t s_buf[W][kRunBuf3 / 4];
+    __shared__ uint32_t s_z[2][W][16];
+    const uint32_t lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    uint32_t* buf = s_buf[wv];
+    uint32_t lo = 0, hi = a.g.T;
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) / 2;
+        if (a.parts[mid].d0 <= blockIdx.x)
+            lo = mid;
+        else
+            hi = mid;
+    }
+    const uint32_t pi = __builtin_amdgcn_readfirstlane(lo);
+    const Part3 p = a.parts[pi];
+    const uint32_t nseg = (p.b1 + kLaneSeg3 - 1) / kLaneSeg3, nz = (p.b3 + 63) / 64;
+    const uint32_t by = (blockIdx.x - p.d0) / nseg, seg = blockIdx.x - p.d0 - by * nseg;
+    const uint32_t ey = Edges ? min(4u, p.sy - 4 * by) : 4u;
+    uint64_t h;
+    __builtin_memcpy(&h, a.in + 8ull * pi, 8);
+    const uint64_t wpos = 8ull * a.g.T + h, ppos = wpos + (uint64_t) p.b1 * p.b2 * p.b3;
+    const unsigned long long o0 = a.part_sums[p.v0 >> 8] + a.words[p.v0];
+    const uint32_t bz = 64 * wv + lane;
+    const bool own = bz < p.b3;
+    const uint32_t ez = Edges && own ? min(4u, p.sz - 4 * bz) : 4u;
+    const bool last_z = Edges && (p.sz & 3) && (p.b3 - 1) / 64 == wv;  // some lane's ez is below 4
+    uint32_t c[16];  // the plane before, summed along x
+#pragma unroll
+    for (uint32_t v = 0; v < 16; v++)
+        c[v] = 0;
+    uint32_t m[64];
+    const uint32_t bx1 = min(kLaneSeg3 * (seg + 1), p.b1);
+    for (uint32_t bx = kLaneSeg3 * seg; bx < bx1; bx++) {
+        const uint32_t ex = Edges ? min(4u, p.sx - 4 * bx) : 4u, cnt = ex * ey * ez;
+        const uint32_t row = bx * p.b2 + by, u = p.v0 + row * nz + min(wv, nz - 1);
+        const uint64_t wp = wpos + (uint64_t) row * p.b3 + bz;
+        uint32_t w = own && wp < a.in_size ? a.in[wp] : 0u;
+        w = w > 32 ? 0u : w;
+        const uint64_t fo = ppos + (a.part_sums[u >> 8] + a.words[u] - o0);
+        const uint32_t size = payload3(w, cnt), incl = wave_scan_dpp(size), excl = incl - size;
+        const uint32_t wtot = __builtin_amdgcn_readlane(incl, 63);
+        const uint32_t avail = fo < a.in_size ? (uint32_t) min((uint64_t) wtot, a.in_size - fo) : 0u;
+        const bool ok = w && excl + size <= avail;
+        if (w && !ok)
+            raise3(a.status, ZK_ERR_OVERRUN);
+        const uint8_t* src = a.in + (fo < a.in_size ? fo : 0);
+        const bool one = wtot + kRunReach3 <= kRunBuf3;
+#pragma unroll 1
+        for (uint32_t q = 0; q < (one ? 1u : 3u); q++) {
+            // the lanes of this round, their bytes [b0, b1) of the run's
+            const uint32_t b0 = q ? __builtin_amdgcn_readlane(excl, 22 * q) : 0u;
+            const uint32_t b1 = min(avail, one || q == 2 ? wtot : __builtin_amdgcn_readlane(excl, 22 * (q + 1)));
+            const uint32_t nb = b1 > b0 ? b1 - b0 : 0u;
+            wave_sync_lds();
+#pragma unroll 1
+            for (uint32_t i = lane; i < nb / 16; i += 64) {
+                uint4 v;
+                __builtin_memcpy(&v, src + b0 + 16 * i, 16);
+                reinterpret_cast<uint4*>(buf)[i] = v;
+            }
+            if (lane < nb % 16)
+                ((uint8_t*) buf)[nb / 16 * 16 + lane] = src[b0 + nb / 16 * 16 + lane];
+            wave_sync_lds();
+            if (one || lane / 22 == q)
+                decode_block3(buf, ok ? excl - b0 : 0u, ok ? w : 0u, cnt, m);
+        }
+        // values of the blocks at a far edge to their places, zeros in the others:
+        // the last block along z (one lane) through LDS, ...
+        if (last_z) {
+            wave_sync_lds();
+            if (ez < 4) {
+#pragma unroll
+                for (uint32_t t = 0; t < 16; t++)
+                    reinterpret_cast<uint4*>(buf)[t] = make_uint4(m[4 * t], m[4 * t + 1], m[4 * t + 2], m[4 * t + 3]);
+            }
+            wave_sync_lds();
+        }
+        // ... the last along y and x in registers (one extent for the wave)
+        if (ey == 1)
+            spread_rows3<1>(m);
+        else if (ey == 2)
+            spread_rows3<2>(m);
+        else if (ey == 3)
+            spread_rows3<3>(m);
+        if (ex < 4) {
+#pragma unroll
+            for (uint32_t v = 16; v < 64; v++)
+                m[v] = v / 16 < ex ? m[v] : 0u;
+        }
+        if (last_z && ez < 4) {
+            const uint32_t n = __builtin_amdgcn_readfirstlane(ez);
+            uint32_t e = 0;
+#pragma unroll
+            for (uint32_t t = 0; t < 16; t++) {
+                const bool in = t / 4 < ex && t % 4 < ey;
+                m[4 * t] = in ? buf[e] : 0u;
+                m[4 * t + 1] = in && n > 1 ? buf[e + 1] : 0u;
+                m[4 * t + 2] = in && n > 2 ? buf[e + 2] : 0u;
+                m[4 * t + 3] = 0;
+                e += in ? n : 0u;
+            }
+        }
+        // along x, from the plane before
+#pragma unroll
+        for (uint32_t v = 0; v < 64; v++)
+            m[v] += v < 16 ? c[v] : m[v - 16];
+#pragma unroll
+        for (uint32_t v = 0; v < 16; v++)
+            c[v] = m[48 + v];
+        // along z
+        uint32_t tot[16];
+#pragma unroll
+        for (uint32_t t = 0; t < 16; t++) {
+#pragma unroll
+            for (uint32_t k = 1; k < 4; k++)
+                m[4 * t + k] += m[4 * t + k - 1];
+            const uint32_t own_sum = m[4 * t + 3], inc = wave_scan_dpp(own_sum), ex0 = inc - own_sum;
+#pragma unroll
+            for (uint32_t k = 0; k < 4; k++)
+                m[4 * t + k] += ex0;
+            tot[t] = inc;
+        }
+        if (W > 1 && nz > 1) {
+            if (lane == 63) {
+#pragma unroll
+                for (uint32_t t = 0; t < 16; t++)
+                    s_z[bx & 1][wv][t] = tot[t];
+            }
+            __syncthreads();
+            for (uint32_t i = 0; i < wv; i++) {
+#pragma unroll
+                for (uint32_t t = 0; t < 16; t++) {
+                    const uint32_t before = s_z[bx & 1][i][t];
+#pragma unroll
+                    for (uint32_t k = 0; k < 4; k++)
+                        m[4 * t + k] += before;
+                }
+            }
+        }
+        uint32_t* q = (uint32_t*) a.y + ((uint64_t) (p.ox + 4 * bx) * a.g.d2 + (p.oy + 4 * by)) * a.g.d3 + p.oz;
+#pragma unroll
+        for (uint32_t t = 0; t < 16; t++) {
+            if (t / 4 < ex && t % 4 < ey) {
+                uint32_t* qr = q + ((uint64_t) (t / 4) * a.g.d2 + t % 4) * a.g.d3;
+                if (own && ez == 4) {
+                    const uint4 v = make_uint4(m[4 * t], m[4 * t + 1], m[4 * t + 2], m[4 * t + 3]);
+                    __builtin_memcpy(__builtin_assume_aligned(qr + 4 * bz, 4), &v, 16);
+                } else if (own) {
+#pragma unroll
+                    for (uint32_t k = 0; k < 4; k++)
+                        if (k < ez)
+                            qr[4 * bz + k] = m[4 * t + k];
+                }
+            }
+        }
+    }
+    if (seg + 1 < nseg && own) {
+        uint32_t* tail = (uint32_t*) a.offs + p.t0 + ((uint64_t) seg * p.sy + 4 * by) * p.sz + 4 * bz;
+#pragma unroll
+        for (uint32_t j = 0; j < 4; j++)
+#pragma unroll
+            for (uint32_t k = 0; k < 4; k++)
+                if (j < ey && k < ez)
+                    tail[j * p.sz + k] = m[48 + 4 * j + k];
+    }
+}
+
+// Last planes of the segments summed over the segments before: one thread per
+// (sub-volume, y, z).
+__global__ void __launch_bounds__(256) k3l_tails(Sz3Args a)
+{
+    const uint32_t col = blockIdx.x * blockDim.x + threadIdx.x;
+    if (col >= a.g.xcols)
+        return;
+    uint32_t lo = 0, hi = a.g.T;
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) / 2;
+        if (a.parts[mid].xc0 <= col)
+            lo = mid;
+        else
+            hi = mid;
+    }
+    const Part3 p = a.parts[lo];
+    const uint32_t nseg = (p.b1 + kLaneSeg3 - 1) / kLaneSeg3, face = p.sy * p.sz;
+    uint32_t* tail = (uint32_t*) a.offs + p.t0 + (col - p.xc0);
+    uint32_t run = 0;
+    for (uint32_t s = 0; s + 1 < nseg; s++) {
+        run += tail[(uint64_t) s * face];
+        tail[(uint64_t) s * face] = run;
+    }
+}
+
+// Along y, with the segments before, and dequantized in place: one thread per
+// (sub-volume, block along x, z), its four columns kRowsY3 rows at a time (all
+// their loads in flight before the first store; 512^3: 2 rows 386 us, 4 rows 261,
+// 8 rows 206, 16 rows 204 with half the waves).
+// x' = (float)((double)q * 2 eb), ZCCL/src/ZCCLd_float.c:3030.
+constexpr uint32_t kRowsY3 = 8;
+
+__global__ void __launch_bounds__(256) k3l_ypass(Sz3Args a)
+{
+    const uint32_t col = blockIdx.x * blockDim.x + threadIdx.x;
+    if (col >= a.g.nhcol)
+        return;
+    uint32_t lo = 0, hi = a.g.T;
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) / 2;
+        if (a.parts[mid].h0 <= col)
+            lo = mid;
+        else
+            hi = mid;
+    }
+    const Part3 p = a.parts[lo];
+    const uint32_t bx = (col - p.h0) / p.sz, z = (col - p.h0) - bx * p.sz, seg = bx / kLaneSeg3;
+    const uint32_t ex = min(4u, p.sx - 4 * bx);
+    const uint64_t d3 = a.g.d3, plane = (uint64_t) a.g.d2 * d3;
+    uint32_t* q = (uint32_t*) a.y + ((uint64_t) (p.ox + 4 * bx) * a.g.d2 + p.oy) * d3 + p.oz + z;
+    // (planes past the sub-volume: the last one again, not stored)
+    uint64_t po[4];
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++)
+        po[i] = min(i, ex - 1) * plane;
+    const uint32_t* tail = (const uint32_t*) a.offs + p.t0 + (uint64_t) (seg ? seg - 1 : 0u) * p.sy * p.sz + z;
+    uint32_t run[4] = {0, 0, 0, 0};
+    for (uint32_t y0 = 0; y0 < p.sy; y0 += kRowsY3) {
+        uint32_t v[kRowsY3][4], t[kRowsY3];
+#pragma unroll
+        for (uint32_t r = 0; r < kRowsY3; r++) {
+            const uint32_t y = min(y0 + r, p.sy - 1);
+            t[r] = seg ? tail[(uint64_t) y * p.sz] : 0u;
+#pragma unroll
+            for (uint32_t i = 0; i < 4; i++)
+                v[r][i] = q[y * d3 + po[i]];
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < kRowsY3; r++) {
+            if (y0 + r < p.sy) {
+#pragma unroll
+                for (uint32_t i = 0; i < 4; i++) {
+                    run[i] += v[r][i] + t[r];
+                    if (i < ex)
+                        ((float*) q)[(y0 + r) * d3 + po[i]] = (float) __dmul_rn((double) (int32_t) run[i], a.tw);
+                }
+            }
+        }
+    }
+}
+
 }  // namespace
 
 static hipError_t scan3(const Sz3Args& a, int check_cap, hipStream_t s)
@@ -1232,8 +1618,32 @@ hipError_t launch_sz3_compress(const Sz3Args& a, hipStream_t s)
     return hipGetLastError();
 }
 
+template <bool Edges>
+static hipError_t decode_rows3(const Sz3Args& a, hipStream_t s)
+{
+    if (a.g.wruns == 1)
+        hipLaunchKernelGGL((k3l_decode<1, Edges>), dim3(a.g.nrows), dim3(64), 0, s, a);
+    else if (a.g.wruns == 2)
+        hipLaunchKernelGGL((k3l_decode<2, Edges>), dim3(a.g.nrows), dim3(128), 0, s, a);
+    else
+        hipLaunchKernelGGL((k3l_decode<kLaneRuns3, Edges>), dim3(a.g.nrows), dim3(64 * kLaneRuns3), 0, s, a);
+    return hipGetLastError();
+}
+
 hipError_t launch_sz3_decompress(const Sz3Args& a, hipStream_t s)
 {
+    if (a.g.nruns) {
+        const uint32_t groups = (uint32_t) ceil_div(a.g.nruns, 256);
+        hipLaunchKernelGGL(k3l_sizes, dim3(groups), dim3(256), 0, s, a);
+        hipLaunchKernelGGL(k3_scan_top, dim3(1), dim3(256), 0, s, a, groups, 0);
+        const hipError_t e = a.g.edges ? decode_rows3<true>(a, s) : decode_rows3<false>(a, s);
+        if (e != hipSuccess)
+            return e;
+        if (a.g.ntail)
+            hipLaunchKernelGGL(k3l_tails, dim3((uint32_t) ceil_div(a.g.xcols, 256)), dim3(256), 0, s, a);
+        hipLaunchKernelGGL(k3l_ypass, dim3((uint32_t) ceil_div(a.g.nhcol, 256)), dim3(256), 0, s, a);
+        return hipGetLastError();
+    }
     if (a.g.nunits && a.g.Bs == 4)
         return decompress_tiled<4>(a, s);
     if (a.g.nunits && a.g.Bs == 8)
