@@ -38,6 +38,11 @@ def _ptr(t: torch.Tensor) -> ctypes.c_void_p:
     return ctypes.c_void_p(t.data_ptr())
 
 
+# Sizes that follow from (n, L, T) alone are kept: a call into the library for
+# each is a microsecond of the host, which sets the pace of the smallest passes
+# (64 Ki values: kernel 9.4 us).  num_tiles depends on the tunables and is not.
+
+@functools.lru_cache(maxsize=4096, typed=True)
 def worst_case_bytes(n: int, L: int, T: int) -> int:
     v = lib().zccl_worst_case_bytes(n, L, T)
     if v == 0:
@@ -45,7 +50,7 @@ def worst_case_bytes(n: int, L: int, T: int) -> int:
     return int(v)
 
 
-@functools.lru_cache(maxsize=4096)
+@functools.lru_cache(maxsize=4096, typed=True)
 def index_bytes(n: int, L: int, T: int) -> int:
     return int(lib().zccl_index_bytes(n, L, T))
 
@@ -54,8 +59,14 @@ def num_tiles(n: int, L: int, T: int) -> int:
     return int(lib().zccl_num_tiles(n, L, T))
 
 
+@functools.lru_cache(maxsize=4096, typed=True)
 def num_blocks(n: int, L: int, T: int) -> int:
     return int(lib().zccl_num_blocks(n, L, T))
+
+
+@functools.lru_cache(maxsize=4096, typed=True)
+def _index_size_offset(n: int, L: int, T: int) -> int:
+    return int(lib().zccl_index_size_offset(n, L, T))
 
 
 class Workspace:
@@ -150,7 +161,7 @@ class DeviceStream:
 
     @property
     def size_offset(self) -> int:
-        return int(lib().zccl_index_size_offset(self.n, self.L, self.T))
+        return _index_size_offset(self.n, self.L, self.T)
 
     def size_tensor(self) -> torch.Tensor:
         """Device u64 view of the stream size (no synchronisation)."""
