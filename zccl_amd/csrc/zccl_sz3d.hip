@@ -498,7 +498,11 @@ __global__ void __launch_bounds__(256) k3_zpass(Sz3Args a)
     }
 }
 
-// Along y: one thread per (sub-volume, x, z) column.
+// Along y: one thread per (sub-volume, x, z) column, kAhead3 rows of loads in
+// flight before their stores (512^3 with block side 8, us: y pass 239 without, 188
+// with 8, 213 with 16; x pass 249, 204, 230; 64^3: 11.8, 5.1, 4.6 and 7.2, 5.1, 4.7).
+constexpr uint32_t kAhead3 = 8;
+
 __global__ void __launch_bounds__(256) k3_ypass(Sz3Args a)
 {
     const uint32_t col = blockIdx.x * blockDim.x + threadIdx.x;
@@ -515,10 +519,19 @@ __global__ void __launch_bounds__(256) k3_ypass(Sz3Args a)
     const Part3 p = a.parts[lo];
     const uint32_t c = col - p.yc0, lx = c / p.sz, lz = c - lx * p.sz;
     uint32_t* q = (uint32_t*) a.y + ((uint64_t) (p.ox + lx) * a.g.d2 + p.oy) * a.g.d3 + p.oz + lz;
-    uint32_t run = q[0];
-    for (uint32_t y = 1; y < p.sy; y++) {
-        run += q[(uint64_t) y * a.g.d3];
-        q[(uint64_t) y * a.g.d3] = run;
+    uint32_t run = 0;
+    for (uint32_t y0 = 0; y0 < p.sy; y0 += kAhead3) {
+        uint32_t v[kAhead3];
+#pragma unroll
+        for (uint32_t r = 0; r < kAhead3; r++)
+            v[r] = q[(uint64_t) min(y0 + r, p.sy - 1) * a.g.d3];
+#pragma unroll
+        for (uint32_t r = 0; r < kAhead3; r++) {
+            if (y0 + r < p.sy) {
+                run += v[r];
+                q[(uint64_t) (y0 + r) * a.g.d3] = run;
+            }
+        }
     }
 }
 
@@ -541,10 +554,20 @@ __global__ void __launch_bounds__(256) k3_xpass(Sz3Args a)
     const uint32_t c = col - p.xc0, ly = c / p.sz, lz = c - ly * p.sz;
     const uint64_t sx = (uint64_t) a.g.d2 * a.g.d3;
     uint32_t* q = (uint32_t*) a.y + ((uint64_t) p.ox * a.g.d2 + (p.oy + ly)) * a.g.d3 + p.oz + lz;
+    float* y = a.y + (q - (uint32_t*) a.y);
     uint32_t run = 0;
-    for (uint32_t x = 0; x < p.sx; x++) {
-        run += q[x * sx];
-        a.y[(q - (uint32_t*) a.y) + x * sx] = (float) __dmul_rn((double) (int32_t) run, a.tw);
+    for (uint32_t x0 = 0; x0 < p.sx; x0 += kAhead3) {
+        uint32_t v[kAhead3];
+#pragma unroll
+        for (uint32_t r = 0; r < kAhead3; r++)
+            v[r] = q[min(x0 + r, p.sx - 1) * sx];
+#pragma unroll
+        for (uint32_t r = 0; r < kAhead3; r++) {
+            if (x0 + r < p.sx) {
+                run += v[r];
+                y[(x0 + r) * sx] = (float) __dmul_rn((double) (int32_t) run, a.tw);
+            }
+        }
     }
 }
 
@@ -1502,7 +1525,8 @@ __global__ void __launch_bounds__(256) k3l_tails(Sz3Args a)
 // Along y, with the segments before, and dequantized in place: one thread per
 // (sub-volume, block along x, z), its four columns kRowsY3 rows at a time (all
 // their loads in flight before the first store; 512^3: 2 rows 386 us, 4 rows 261,
-// 8 rows 206, 16 rows 204 with half the waves).
+// 8 rows 206, 16 rows 204 with half the waves;
+// 8 rows of two columns 216, of one 240, whose kept planes are read more often).
 // x' = (float)((double)q * 2 eb), ZCCL/src/ZCCLd_float.c:3030.
 constexpr uint32_t kRowsY3 = 8;
 
