@@ -11,8 +11,8 @@
 // cross-lane step is one DPP scan of block sizes that places each lane's block.
 // The next operand's loads are in flight while the current one is decoded.
 //
-// Each wave is a tile of the decoupled lookback; a workgroup of four waves
-// takes one ticket for four consecutive tiles.  The summed block is
+// Each wave is a tile of the decoupled lookback; a workgroup of four or eight
+// waves takes one ticket for as many consecutive tiles.  The summed block is
 // re-encoded into the wave's own LDS buffer with OR-writes of dwords (the
 // buffer is zeroed first, and a lane ORs zeros wherever its dwords overlap a
 // neighbour's bytes, so overlapping writes need no ordering) and leaves with
@@ -1402,7 +1402,7 @@ __device__ __forceinline__ void compress_tile_lane(const Geom& g, const Tiling& 
 // Waves (tiles) that share a ticket of a sum: tickets are adds to one address,
 // 12 ns each, so beyond kSumFew tiles, which fill the chip's 1024 SIMDs with four
 // waves each, they bound the kernel and eight waves share one (32 mixed buckets:
-// 88.6 -> 79.2 us); below, smaller workgroups start sooner (868 tiles of 4
+// 88.6 -> 79.2 us); below, smaller workgroups start sooner (868 tiles of 16
 // operands: 34.0 us, with eight 38.4).
 constexpr uint32_t kSumMany = 8, kSumFew = 4096;
 
