@@ -1708,8 +1708,13 @@ __global__ void __launch_bounds__(kParseSpecThreads) k_parse_spec(ParseArgs a, P
     __shared__ uint32_t s_cnt[64], s_ex[64];       // wave 0's walks: blocks, exit (kParseNoExit: dead)
     __shared__ uint32_t s_lo[kParseSpecWaves], s_hi[kParseSpecWaves];
     const uint32_t tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
-    const uint64_t gt = blockIdx.x;
-    const uint32_t c = (uint32_t) (gt / pl.tpc), t = (uint32_t) (gt % pl.tpc);
+    // the first tiles of all chunks, then the second ones, ...: a chunk's last
+    // tiles are mostly past its region (sized for the worst case), and their
+    // workgroups no longer stand between those with work (2^24 values in 16
+    // chunks: 65.7 -> 59.1 us; the emit, four tiles to a workgroup, in the same
+    // order: 37.3 -> 29.6)
+    const uint32_t c = blockIdx.x % a.g.T, t = blockIdx.x / a.g.T;
+    const uint64_t gt = (uint64_t) c * pl.tpc + t;
     uint64_t cs, ce;
     if (!parse_region(a, pl, c, cs, ce))
         return;  // pass two reports the chunk
@@ -1954,11 +1959,11 @@ __global__ void __launch_bounds__(256) k_parse_emit(ParseArgs a, ParseLayout pl)
     __shared__ uint32_t nzb[4][kParseNzWords];
     // (the wave index read as uniform: the walk below then runs on scalar registers)
     const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const uint64_t gt = (uint64_t) blockIdx.x * 4 + wv;
-    if (gt >= pl.ntiles)
-        return;
     const Geom& g = a.g;
-    const uint32_t c = (uint32_t) (gt / pl.tpc), t = (uint32_t) (gt % pl.tpc);
+    const uint32_t c = blockIdx.x % g.T, t = 4 * (blockIdx.x / g.T) + wv;
+    if (t >= pl.tpc)
+        return;
+    const uint64_t gt = (uint64_t) c * pl.tpc + t;
     uint64_t cs, ce;
     if (!parse_region(a, pl, c, cs, ce))
         return;
@@ -2313,7 +2318,7 @@ hipError_t launch_parse(const ParseArgs& a, hipStream_t s)
 {
     const ParseLayout pl = parse_layout(a.g);
     if (parse_parallel_ok(a.g) && a.ws_bytes >= pl.bytes) {
-        const uint32_t groups = (uint32_t) ceil_div(pl.ntiles, 4);
+        const uint32_t groups = a.g.T * (uint32_t) ceil_div(pl.tpc, 4);
         const uint64_t words = (pl.bytes - pl.flag_off) / 8;
         hipLaunchKernelGGL(k_parse_begin, dim3(1), dim3(64), 0, s, a, pl);
         hipLaunchKernelGGL(k_parse_spec, dim3((uint32_t) pl.ntiles), dim3(kParseSpecThreads), 0, s, a, pl);
