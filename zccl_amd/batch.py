@@ -19,7 +19,7 @@ import torch
 from . import _lib
 from ._lib import check, lib
 from .codec import (STAGED_L, DeviceStream, Workspace, _stream_handle, default_stage, default_workspace, indexed,
-                    staged_min_tiles)
+                    staged_min_tiles, with_room)
 
 
 class BatchPlan:
@@ -95,7 +95,7 @@ def homsum_plan(jobs: Sequence[Sequence[DeviceStream]], outs: Sequence[DeviceStr
     ixs = _ptrs([s.index for ops in jobs for s in ops])
     od = _ptrs([o.data for o in outs])
     ocap = (ctypes.c_size_t * nj)(*[o.data.numel() for o in outs])
-    oix = _ptrs([o.index for o in outs])
+    oix = _ptrs([with_room(o).index for o in outs])
     st = ctypes.c_int(0)
     h = lib().zccl_batch_homsum_plan(nj, ks, n, L, T, ins, ixs, od, ocap, oix, ctypes.byref(st))
     check(st.value, "batch homsum plan")
@@ -114,7 +114,7 @@ def compress_plan(xs: Sequence[torch.Tensor], ebs: Sequence[float], outs: Sequen
     st = ctypes.c_int(0)
     h = lib().zccl_batch_compress_plan(nj, n, eb, L, T, _ptrs(xs), _ptrs([o.data for o in outs]),
                                         (ctypes.c_size_t * nj)(*[o.data.numel() for o in outs]),
-                                        _ptrs([o.index for o in outs]), ctypes.byref(st))
+                                        _ptrs([with_room(o).index for o in outs]), ctypes.byref(st))
     check(st.value, "batch compress plan")
     return BatchPlan(h, [list(xs), list(outs)], list(outs))
 

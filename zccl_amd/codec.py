@@ -200,6 +200,15 @@ def indexed(s: DeviceStream) -> DeviceStream:
     return from_bytes(s.data, s.n, s.L, s.T)
 
 
+def with_room(s: DeviceStream) -> DeviceStream:
+    """An output stream, its index replaced where it is too short for this
+    library's (every kernel that writes a stream writes the whole index)."""
+    need = index_bytes(s.n, s.L, s.T)
+    if s.index.numel() < need:
+        s.index = torch.empty(need, dtype=torch.uint8, device=s.index.device)
+    return s
+
+
 def _ws_for(n: int, L: int, T: int, ws: Optional[Workspace]) -> Workspace:
     tiles = num_tiles(n, L, T)
     if ws is None:
@@ -219,7 +228,7 @@ def compress(x: torch.Tensor, eb: float, L: int, T: int, out: Optional[DeviceStr
     if (s.n, s.L, s.T) != (n, L, T):
         raise ValueError("output stream geometry differs")
     w = _ws_for(n, L, T, ws)
-    s.invalidate()
+    with_room(s).invalidate()
     check(lib().zccl_compress_dev(_ptr(x), n, ctypes.c_float(eb), L, T, _ptr(s.data), s.data.numel(),
                                   _ptr(s.index), None, w.ptr, w.nbytes, _stream_handle()), "compress")
     return s
@@ -271,7 +280,7 @@ def _homsum_launch(ops: Sequence[DeviceStream], out: Optional[DeviceStream], w: 
     k = len(ops)
     ins = (ctypes.c_void_p * k)(*[s.data.data_ptr() for s in ops])
     ixs = (ctypes.c_void_p * k)(*[s.index.data_ptr() for s in ops])
-    o.invalidate()
+    with_room(o).invalidate()
     if st is not None:
         check(lib().zccl_homsum_dev_staged(ins, ixs, k, n, L, T, _ptr(o.data), o.data.numel(), _ptr(o.index),
                                            None, w.ptr, w.nbytes, st.ptr, st.nbytes, _stream_handle()),
