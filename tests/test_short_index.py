@@ -99,3 +99,13 @@ def test_a_full_index_stays(lib):
     ix = out.index
     codec.compress(device(torch.zeros(N)), EB, L, T, out=out, ws=WS)
     assert out.index is ix
+
+
+def test_a_short_input_is_indexed_on_the_callers_workspace(lib):
+    """What its parse finds wrong is reported where the call's errors are."""
+    codec.decompress(stream(True), EB, out=torch.zeros(N), ws=WS)
+    codec.homsum([stream(True), stream(False)], out=stream(False), ws=WS, stage=False)
+    names = [name for name, _ in lib.calls]
+    assert names == ["zccl_parse_dev", "zccl_decompress_dev", "zccl_parse_dev", "zccl_homsum_dev"]
+    for (name, a), at in zip(lib.calls, (7, 8, 7, 10)):
+        assert a[at].value == WS.ptr.value, name

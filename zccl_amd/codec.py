@@ -192,12 +192,13 @@ def empty_stream(n: int, L: int, T: int, capacity: Optional[int] = None,
     return DeviceStream(data, index, n, L, T)
 
 
-def indexed(s: DeviceStream) -> DeviceStream:
+def indexed(s: DeviceStream, ws: Optional[Workspace] = None) -> DeviceStream:
     """s, or (its index kept from a library that wrote shorter ones) the same
-    bytes under an index of this library's size."""
+    bytes under an index of this library's size, parsed on ``ws``.  The parse
+    is made on each call: the bytes may be others by then."""
     if s.index.numel() >= index_bytes(s.n, s.L, s.T):
         return s
-    return from_bytes(s.data, s.n, s.L, s.T)
+    return from_bytes(s.data, s.n, s.L, s.T, ws=ws)
 
 
 def with_room(s: DeviceStream) -> DeviceStream:
@@ -240,7 +241,7 @@ def decompress(s: DeviceStream, eb: float, out: Optional[torch.Tensor] = None,
     if y.numel() != s.n or y.dtype != torch.float32 or not y.is_contiguous():
         raise ValueError("out must be a contiguous float32 tensor of n elements")
     w = _ws_for(s.n, s.L, s.T, ws)
-    s = indexed(s)
+    s = indexed(s, ws)
     check(lib().zccl_decompress_dev(_ptr(s.data), _ptr(s.index), s.n, ctypes.c_float(eb), s.L, s.T,
                                     _ptr(y), w.ptr, w.nbytes, _stream_handle()), "decompress")
     return y
@@ -266,7 +267,7 @@ def homsum(streams: Sequence[DeviceStream], out: Optional[DeviceStream] = None,
         st = stage if stage is not None else default_stage(tiles)
         if st.max_tiles < tiles:
             raise _lib.ZcclError(-6, f"stage area holds {st.max_tiles} tiles, sum needs {tiles}")
-    ops = [indexed(s) for s in streams]
+    ops = [indexed(s, ws) for s in streams]
     while len(ops) > MAX_OPERANDS:
         part = _homsum_launch(ops[:MAX_OPERANDS], None, w, st)
         ops = [part] + ops[MAX_OPERANDS:]
