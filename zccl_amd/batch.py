@@ -18,13 +18,13 @@ import torch
 
 from . import _lib
 from ._lib import check, lib
-from .codec import (STAGED_L, DeviceStream, Workspace, _stream_handle, default_stage, default_workspace, indexed,
-                    staged_min_tiles, with_room)
+from .codec import (STAGED_L, DeviceStream, Workspace, _stream_handle, default_stage, default_workspace, parse,
+                    parse_tiles, staged_min_tiles, with_index, with_room)
 
 
 class BatchPlan:
     def __init__(self, handle: int, keep: list, outs: Optional[List[DeviceStream]] = None,
-                 staged: bool = False):
+                 staged: bool = False, parsed: Sequence[DeviceStream] = ()):
         if not handle:
             raise _lib.ZcclError(-1, "batch plan")
         self.handle = ctypes.c_void_p(handle)
@@ -38,6 +38,9 @@ class BatchPlan:
         check(L.zccl_batch_bind(self.handle, ctypes.c_void_p(self.desc.data_ptr())), "batch bind")
         self._keep = keep
         self.outs = outs or []
+        # inputs whose own index is too short for this library: their bytes
+        # are parsed on each launch (they may be others by then)
+        self.parsed = list(parsed)
         # a homomorphic-sum batch of one geometry and operand count at
         # blockSize 36: the two-pass form applies
         self.staged = staged
@@ -45,11 +48,16 @@ class BatchPlan:
     def launch(self, ws: Optional[Workspace] = None, stage=None) -> None:
         """stage: a StageArea for the two-pass sum (None: the default one,
         False: the single-pass form); ignored by other batches."""
-        w = ws if ws is not None else default_workspace(self.tiles)
+        w = ws
+        if w is None:
+            w = default_workspace(max([self.tiles] + [parse_tiles(s.n, s.L, s.T) for s in self.parsed])
+                                  if self.parsed else self.tiles)
         if w.max_tiles < self.tiles:
             raise _lib.ZcclError(-6, f"workspace holds {w.max_tiles} tiles, batch needs {self.tiles}")
         for o in self.outs:
             o.invalidate()
+        for s in self.parsed:
+            parse(s, w)
         if self.staged and stage is not False and self.tiles >= staged_min_tiles():
             st = stage if stage is not None else default_stage(self.tiles)
             if st.max_tiles < self.tiles:
@@ -81,7 +89,7 @@ def homsum_plan(jobs: Sequence[Sequence[DeviceStream]], outs: Sequence[DeviceStr
     nj = len(jobs)
     if len(outs) != nj or nj == 0:
         raise ValueError("one output per job")
-    jobs = [[indexed(s) for s in ops] for ops in jobs]
+    given, jobs = jobs, [[with_index(s) for s in ops] for ops in jobs]
     L, T = outs[0].L, outs[0].T
     for j, ops in enumerate(jobs):
         if not 1 <= len(ops) <= 32:
@@ -100,7 +108,8 @@ def homsum_plan(jobs: Sequence[Sequence[DeviceStream]], outs: Sequence[DeviceStr
     h = lib().zccl_batch_homsum_plan(nj, ks, n, L, T, ins, ixs, od, ocap, oix, ctypes.byref(st))
     check(st.value, "batch homsum plan")
     staged = L == STAGED_L and len({(o.n, len(ops)) for o, ops in zip(outs, jobs)}) == 1
-    return BatchPlan(h, [list(jobs), list(outs)], list(outs), staged=staged)
+    return BatchPlan(h, [list(jobs), list(outs)], list(outs), staged=staged,
+                     parsed=[s for ops, old in zip(jobs, given) for s, o in zip(ops, old) if s is not o])
 
 
 def compress_plan(xs: Sequence[torch.Tensor], ebs: Sequence[float], outs: Sequence[DeviceStream]) -> BatchPlan:
@@ -120,7 +129,7 @@ def compress_plan(xs: Sequence[torch.Tensor], ebs: Sequence[float], outs: Sequen
 
 
 def decompress_plan(streams: Sequence[DeviceStream], ebs: Sequence[float], outs: Sequence[torch.Tensor]) -> BatchPlan:
-    streams = [indexed(s) for s in streams]
+    given, streams = streams, [with_index(s) for s in streams]
     nj = len(streams)
     L, T = streams[0].L, streams[0].T
     for s, y in zip(streams, outs):
@@ -132,4 +141,4 @@ def decompress_plan(streams: Sequence[DeviceStream], ebs: Sequence[float], outs:
     h = lib().zccl_batch_decompress_plan(nj, n, eb, L, T, _ptrs([s.data for s in streams]),
                                           _ptrs([s.index for s in streams]), _ptrs(outs), ctypes.byref(st))
     check(st.value, "batch decompress plan")
-    return BatchPlan(h, [list(streams), list(outs)])
+    return BatchPlan(h, [list(streams), list(outs)], parsed=[s for s, o in zip(streams, given) if s is not o])

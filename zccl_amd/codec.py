@@ -201,6 +201,14 @@ def indexed(s: DeviceStream, ws: Optional[Workspace] = None) -> DeviceStream:
     return from_bytes(s.data, s.n, s.L, s.T, ws=ws)
 
 
+def with_index(s: DeviceStream) -> DeviceStream:
+    """s, or (its index too short) the same bytes with room for an index of
+    this library's size, for parse() to write."""
+    if s.index.numel() >= index_bytes(s.n, s.L, s.T):
+        return s
+    return with_room(DeviceStream(s.data, s.index, s.n, s.L, s.T))
+
+
 def with_room(s: DeviceStream) -> DeviceStream:
     """An output stream, its index replaced where it is too short for this
     library's (every kernel that writes a stream writes the whole index)."""
@@ -297,16 +305,22 @@ def from_bytes(data: torch.Tensor, n: int, L: int, T: int, ws: Optional[Workspac
     library) and rebuild their index on the GPU."""
     if data.dtype != torch.uint8 or not data.is_cuda:
         raise ValueError("data must be a uint8 CUDA tensor")
-    index = torch.empty(index_bytes(n, L, T), dtype=torch.uint8, device=data.device)
-    if ws is None:
-        # room for the parallel parse's tables
-        need = int(lib().zccl_parse_workspace_bytes(n, L, T))
-        w = default_workspace(max(num_tiles(n, L, T), (need - 256) // 16 + 1))
-    else:
-        w = _ws_for(n, L, T, ws)
-    check(lib().zccl_parse_dev(_ptr(data), data.numel(), n, L, T, _ptr(index), None, w.ptr, w.nbytes,
+    s = DeviceStream(data, torch.empty(index_bytes(n, L, T), dtype=torch.uint8, device=data.device), n, L, T)
+    parse(s, default_workspace(parse_tiles(n, L, T)) if ws is None else _ws_for(n, L, T, ws))
+    return s
+
+
+def parse_tiles(n: int, L: int, T: int) -> int:
+    """Tiles of a workspace with room for the parallel parse's tables."""
+    need = int(lib().zccl_parse_workspace_bytes(n, L, T))
+    return max(num_tiles(n, L, T), (need - 256) // 16 + 1)
+
+
+def parse(s: DeviceStream, ws: Workspace) -> None:
+    """Rebuild s.index from s.data (asynchronous on the current stream)."""
+    s.invalidate()
+    check(lib().zccl_parse_dev(_ptr(s.data), s.data.numel(), s.n, s.L, s.T, _ptr(s.index), None, ws.ptr, ws.nbytes,
                                _stream_handle()), "parse")
-    return DeviceStream(data, index, n, L, T)
 
 
 def upload(stream: np.ndarray, n: int, L: int, T: int) -> DeviceStream:
