@@ -1,0 +1,57 @@
+// sz3d_lane_check.cpp -- host checks of the lane kernels' work split (3-D,
+// block side 4) through the functions of zccl_sz3d.h that the kernels use.
+//
+//   routes   volumes with too few rows or columns to fill the chip are left to
+//            the tiled decoder, larger ones take the lane decoder
+//
+// Built and run by tests/test_sz3d_lane.py with g++; prints "ok <cases>" or the
+// first violation.
+#include <cstdio>
+#include <cstdlib>
+#include <vector>
+
+#include "zccl_sz3d.h"
+
+using namespace zk;
+
+static long g_cases = 0;
+
+#define REQUIRE(cond, ...)                                                                         \
+    do {                                                                                           \
+        if (!(cond)) {                                                                             \
+            std::printf("FAIL %s:%d: %s | ", __FILE__, __LINE__, #cond);                           \
+            std::printf(__VA_ARGS__);                                                              \
+            std::printf("\n");                                                                     \
+            std::exit(1);                                                                          \
+        }                                                                                          \
+    } while (0)
+
+// Volumes timed by both decoders (lanes: the faster one), and those that the
+// lane decoder's GPU tests take.
+static void routes()
+{
+    struct {
+        uint32_t d1, d2, d3;
+        int T;
+        bool lanes;
+    } v[] = {{118, 27, 194, 4, false}, {77, 38, 138, 1, false}, {172, 27, 321, 8, false}, {290, 61, 367, 16, false},
+        {86, 165, 127, 1, false}, {167, 342, 264, 1, false}, {64, 336, 320, 2, false}, {160, 464, 320, 2, false},
+        {256, 256, 256, 16, true}, {300, 300, 300, 16, true}, {384, 384, 384, 8, true}, {448, 320, 176, 1, true},
+        {512, 512, 512, 16, true}, {512, 512, 512, 1, true}, {510, 510, 510, 16, true},
+        {256, 192, 256, 16, true}, {250, 190, 250, 16, true}, {200, 350, 250, 9, true}, {260, 192, 260, 4, true},
+        {131, 195, 515, 2, true}, {67, 257, 1021, 1, true}, {66, 256, 1024, 1, true}};
+    for (const auto& x : v) {
+        Geom3 g;
+        std::vector<Part3> parts(x.T);
+        REQUIRE(make_geom3(x.d1, x.d2, x.d3, 4, x.T, &g, parts.data()), "geometry");
+        REQUIRE((g.nruns > 0) == x.lanes, "%ux%ux%u T %d: runs %u", x.d1, x.d2, x.d3, x.T, g.nruns);
+        g_cases++;
+    }
+}
+
+int main()
+{
+    routes();
+    std::printf("ok %ld\n", g_cases);
+    return 0;
+}

@@ -80,11 +80,19 @@ constexpr uint32_t kLaneMaxRow3 = 1u << 27;
 // Lane decoder (block side 4): one lane per block, a wave per run of 64 blocks
 // along z (kLaneRuns3 to a row at most), a workgroup per row of blocks and
 // kLaneSeg3 blocks along x.  Rows shorter than kLaneMinB3 blocks leave most
-// lanes idle and take the tiled kernels (16 sub-volumes, us by lanes / tiled:
-// 256^3, 32 blocks a row: 111 / 143; 180^3, 23 blocks: 112 / 106; 128^3, 16: 72 /
-// 70).  The last plane of every segment but a
-// sub-volume's last is kept for the y pass: at most 8 bytes per block.
+// lanes idle and take the tiled kernels.  So do volumes that give the decoder
+// fewer than three waves for each of 256 compute units, or its y pass (a thread
+// per four columns, serial along y) less than one: what one wave waits for
+// then sets the pace, and the tiled kernels have four times the threads.  us by
+// lanes / tiled: 118 x 27 x 194 in 4 sub-volumes, 56 waves: 79 / 42; 64 x 336 x 320
+// in 2, 336 waves: 150 / 86; 167 x 342 x 264, 1032 waves and 173 in the y pass: 175 /
+// 131; 448 x 320 x 176, 1120 and 308: 156 / 179; 256^3 in 16, 1024 and 512: 100 / 117;
+// 512^3: 387 / 757.  (Of 270 volumes of 24 to 512 a side the line leaves a few with
+// long x and short y to the slower one: 502 x 40 x 130, 160 waves: 86 / 106.)  The last
+// plane of every segment but a sub-volume's last is kept for the y pass: at most
+// 8 bytes per block.
 constexpr uint32_t kLaneSeg3 = 8, kLaneMinB3 = 32, kLaneRuns3 = 4;
+constexpr uint32_t kLaneWaves3 = 3 * 256, kLaneCols3 = 64 * 256;
 
 // Factorise T over three dims as My_Dims_create (ZCCL/src/ZCCL_multidim.c:
 // 100-140): prime factors of T, largest first, each multiplied into the
@@ -200,12 +208,13 @@ ZK_HD bool make_geom3(uint64_t d1, uint64_t d2, uint64_t d3, int Bs, int T, Geom
     g->nunits = nu;
     g->ncols = nc;
     g->nlane = nl;
-    const bool runs = Bs == 4 && b3lo >= kLaneMinB3 && b3hi <= 64 * kLaneRuns3;
+    g->wruns = (b3hi + 63) / 64;
+    const bool runs = Bs == 4 && b3lo >= kLaneMinB3 && b3hi <= 64 * kLaneRuns3 &&
+                      (uint64_t) nd * g->wruns >= kLaneWaves3 && nh >= kLaneCols3;
     g->nruns = runs ? nv : 0u;
     g->nrows = nd;
     g->ntail = nt;
     g->nhcol = nh;
-    g->wruns = (b3hi + 63) / 64;
     g->edges = odd ? 1u : 0u;
     return true;
 }
