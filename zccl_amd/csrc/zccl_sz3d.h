@@ -131,6 +131,69 @@ ZK_HD void dims_create3(int T, int d[3])
 
 ZK_HD uint32_t nblk3(uint32_t s, uint32_t Bs) { return (s - 1) / Bs + 1; }
 
+// The cut of a volume along each dim: td parts of b values, the first r of them
+// of one more.
+struct Split3 {
+    uint32_t td[3], b[3], r[3];
+};
+
+ZK_HD Split3 split3(const Geom3& g)
+{
+    int td[3];
+    dims_create3((int) g.T, td);
+    const uint32_t d[3] = {g.d1, g.d2, g.d3};
+    Split3 s;
+    for (int i = 0; i < 3; i++) {
+        s.td[i] = (uint32_t) td[i];
+        s.b[i] = d[i] / s.td[i];
+        s.r[i] = d[i] % s.td[i];
+    }
+    return s;
+}
+
+// What one sub-volume adds to the table's running sums.
+constexpr uint32_t kSums3 = 11;
+struct Sums3 {
+    uint32_t v[kSums3];  // blocks, zr, yc, xc, u, c, l, v, d, t, h
+};
+
+// Sub-volume t's place and extents, and its share of the sums.
+ZK_HD Sums3 part3(const Geom3& g, const Split3& s, uint32_t t, Part3& p)
+{
+    const uint32_t yz = s.td[1] * s.td[2], px = t / yz, py = (t - px * yz) / s.td[2], pz = t - px * yz - py * s.td[2];
+    p.sx = s.b[0] + (px < s.r[0] ? 1u : 0u);
+    p.sy = s.b[1] + (py < s.r[1] ? 1u : 0u);
+    p.sz = s.b[2] + (pz < s.r[2] ? 1u : 0u);
+    p.ox = px * s.b[0] + (px < s.r[0] ? px : s.r[0]);
+    p.oy = py * s.b[1] + (py < s.r[1] ? py : s.r[1]);
+    p.oz = pz * s.b[2] + (pz < s.r[2] ? pz : s.r[2]);
+    p.b1 = nblk3(p.sx, g.Bs);
+    p.b2 = nblk3(p.sy, g.Bs);
+    p.b3 = nblk3(p.sz, g.Bs);
+    const uint32_t cols = p.b1 * p.b2, segs = (p.b1 + kLaneSeg3 - 1) / kLaneSeg3;
+    const uint32_t nz = tile_nz3(g.Bs), lane = g.Bs == 4 && g.d3 < kLaneMaxRow3 ? g.wlane * kLaneRun3 : 0u;
+    Sums3 c = {{cols * p.b3, p.sx * p.sy, p.sx * p.sz, p.sy * p.sz, nz ? cols * ((p.b3 + nz - 1) / nz) : 0u, cols,
+        lane ? (cols * p.b3 + lane - 1) / lane : 0u, cols * ((p.b3 + 63) / 64), p.b2 * segs, (segs - 1) * p.sy * p.sz,
+        p.b1 * p.sz}};
+    return c;
+}
+
+// The sums over the sub-volumes before it.
+ZK_HD void place3(Part3& p, const Sums3& c)
+{
+    p.g0 = p.nbc = c.v[0];
+    p.zr0 = c.v[1];
+    p.yc0 = c.v[2];
+    p.xc0 = c.v[3];
+    p.u0 = c.v[4];
+    p.c0 = c.v[5];
+    p.l0 = c.v[6];
+    p.v0 = c.v[7];
+    p.d0 = c.v[8];
+    p.t0 = c.v[9];
+    p.h0 = c.v[10];
+}
+
 // Fill g and parts[T] (sub-volumes in thread order, ZCCL/src/ZCCL_float.c:
 // 1901-1935); false when the geometry is out of range or a sub-volume would be
 // empty (the reference's DSize3D_init underflows then).
@@ -140,82 +203,38 @@ ZK_HD bool make_geom3(uint64_t d1, uint64_t d2, uint64_t d3, int Bs, int T, Geom
         return false;
     if (d1 * d2 * d3 > kMaxN)
         return false;
-    int td[3];
-    dims_create3(T, td);
-    if (d1 < (uint64_t) td[0] || d2 < (uint64_t) td[1] || d3 < (uint64_t) td[2])
-        return false;
     g->d1 = (uint32_t) d1;
     g->d2 = (uint32_t) d2;
     g->d3 = (uint32_t) d3;
     g->Bs = (uint32_t) Bs;
     g->T = (uint32_t) T;
-    const uint32_t bx = g->d1 / td[0], rx = g->d1 % td[0], by = g->d2 / td[1], ry = g->d2 % td[1];
-    const uint32_t bz = g->d3 / td[2], rz = g->d3 % td[2];
-    const uint32_t nz = tile_nz3((uint32_t) Bs);
-    const bool lane = Bs == 4 && g->d3 < kLaneMaxRow3;
+    const Split3 s = split3(*g);
+    if (!s.b[0] || !s.b[1] || !s.b[2])
+        return false;
     g->wlane = (uint64_t) g->d1 * g->d2 * g->d3 < kLaneFew3 ? kLaneSlim3 : kLaneWide3;
-    const uint32_t lane_tile = g->wlane * kLaneRun3;
-    uint32_t r = 0, ox = 0, nb = 0, zr = 0, yc = 0, xc = 0, nu = 0, nc = 0, nl = 0, nv = 0, nd = 0, nt = 0, nh = 0;
-    uint32_t b3lo = ~0u, b3hi = 0, odd = 0;
-    for (int px = 0; px < td[0]; px++) {
-        const uint32_t sx = bx + ((uint32_t) px < rx ? 1u : 0u);
-        uint32_t oy = 0;
-        for (int py = 0; py < td[1]; py++) {
-            const uint32_t sy = by + ((uint32_t) py < ry ? 1u : 0u);
-            uint32_t oz = 0;
-            for (int pz = 0; pz < td[2]; pz++) {
-                const uint32_t sz = bz + ((uint32_t) pz < rz ? 1u : 0u);
-                Part3& p = parts[r++];
-                p.ox = ox; p.oy = oy; p.oz = oz;
-                p.sx = sx; p.sy = sy; p.sz = sz;
-                p.b1 = nblk3(sx, Bs); p.b2 = nblk3(sy, Bs); p.b3 = nblk3(sz, Bs);
-                p.g0 = nb;
-                p.nbc = nb;
-                p.zr0 = zr;
-                p.yc0 = yc;
-                p.xc0 = xc;
-                p.u0 = nu;
-                p.c0 = nc;
-                p.l0 = nl;
-                p.v0 = nv;
-                p.d0 = nd;
-                p.t0 = nt;
-                p.h0 = nh;
-                nv += p.b1 * p.b2 * ((p.b3 + 63) / 64);
-                nd += p.b2 * ((p.b1 + kLaneSeg3 - 1) / kLaneSeg3);
-                nt += ((p.b1 + kLaneSeg3 - 1) / kLaneSeg3 - 1) * p.sy * p.sz;
-                nh += p.b1 * p.sz;
-                odd |= (p.sx | p.sy | p.sz) & 3;  // (block side 4)
-                b3lo = p.b3 < b3lo ? p.b3 : b3lo;
-                b3hi = p.b3 > b3hi ? p.b3 : b3hi;
-                nl += lane ? (p.b1 * p.b2 * p.b3 + lane_tile - 1) / lane_tile : 0u;
-                nu += nz ? p.b1 * p.b2 * ((p.b3 + nz - 1) / nz) : 0u;
-                nc += p.b1 * p.b2;
-                nb += p.b1 * p.b2 * p.b3;
-                zr += sx * sy;
-                yc += sx * sz;
-                xc += sy * sz;
-                oz += sz;
-            }
-            oy += sy;
-        }
-        ox += sx;
+    Sums3 sum = {};
+    for (uint32_t t = 0; t < g->T; t++) {
+        const Sums3 c = part3(*g, s, t, parts[t]);
+        place3(parts[t], sum);
+        for (uint32_t i = 0; i < kSums3; i++)
+            sum.v[i] += c.v[i];
     }
-    g->nblocks = nb;
-    g->zrows = zr;
-    g->ycols = yc;
-    g->xcols = xc;
-    g->nunits = nu;
-    g->ncols = nc;
-    g->nlane = nl;
+    g->nblocks = sum.v[0];
+    g->zrows = sum.v[1];
+    g->ycols = sum.v[2];
+    g->xcols = sum.v[3];
+    g->nunits = sum.v[4];
+    g->ncols = sum.v[5];
+    g->nlane = sum.v[6];
+    g->nrows = sum.v[8];
+    g->ntail = sum.v[9];
+    g->nhcol = sum.v[10];
+    const uint32_t b3lo = nblk3(s.b[2], g->Bs), b3hi = nblk3(s.b[2] + (s.r[2] ? 1u : 0u), g->Bs);
     g->wruns = (b3hi + 63) / 64;
     const bool runs = Bs == 4 && b3lo >= kLaneMinB3 && b3hi <= 64 * kLaneRuns3 &&
-                      (uint64_t) nd * g->wruns >= kLaneWaves3 && nh >= kLaneCols3;
-    g->nruns = runs ? nv : 0u;
-    g->nrows = nd;
-    g->ntail = nt;
-    g->nhcol = nh;
-    g->edges = odd ? 1u : 0u;
+                      (uint64_t) g->nrows * g->wruns >= kLaneWaves3 && g->nhcol >= kLaneCols3;
+    g->nruns = runs ? sum.v[7] : 0u;
+    g->edges = (s.b[0] | s.b[1] | s.b[2]) & 3 || s.r[0] || s.r[1] || s.r[2] ? 1u : 0u;  // (block side 4)
     return true;
 }
 

@@ -143,18 +143,33 @@ __device__ __forceinline__ uint32_t wave_incl_scan32(uint32_t v)
 
 constexpr uint32_t kSizeMask = (1u << 26) - 1;
 
-// Sub-volume table, built on the device by one thread (no host copy on the
-// stream the caller passes), and the status words and `nclear` lookback words
-// cleared.
-__global__ void __launch_bounds__(256) k3_table(uint32_t d1, uint32_t d2, uint32_t d3, int Bs, int T, Part3* parts,
-    unsigned long long* status, unsigned long long* clear, uint32_t nclear)
+// Sub-volume table, built on the device by one wave, a lane per sub-volume (no
+// host copy on the stream the caller passes), and the status words and `nclear`
+// lookback words cleared.  (One thread filling one sub-volume after the other took
+// 6.4 us, the median over tables of 16 and of 4; by lanes 2.7.)
+__global__ void __launch_bounds__(256) k3_table(Geom3 g, Split3 sp, Part3* parts, unsigned long long* status,
+    unsigned long long* clear, uint32_t nclear)
 {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        Geom3 g;
-        make_geom3(d1, d2, d3, Bs, T, &g, parts);
-        status[0] = 0;
-        status[1] = 0;
-        status[2] = 0;
+    if (threadIdx.x < 64 && blockIdx.x == 0) {
+        const uint32_t lane = threadIdx.x;
+        if (lane < 3)
+            status[lane] = 0;
+        Sums3 run = {};
+        for (uint32_t t0 = 0; t0 < g.T; t0 += 64) {
+            Part3 p;
+            const uint32_t t = t0 + lane;
+            const Sums3 c = part3(g, sp, min(t, g.T - 1), p);
+            Sums3 before;
+#pragma unroll
+            for (uint32_t i = 0; i < kSums3; i++) {
+                const uint32_t inc = wave_scan_dpp(c.v[i]);
+                before.v[i] = run.v[i] + inc - c.v[i];
+                run.v[i] += __builtin_amdgcn_readlane(inc, 63);
+            }
+            place3(p, before);
+            if (t < g.T)
+                parts[t] = p;
+        }
     }
     for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < nclear; i += gridDim.x * 256)
         clear[i] = 0;
@@ -1593,8 +1608,8 @@ static hipError_t scan3(const Sz3Args& a, int check_cap, hipStream_t s)
 hipError_t launch_sz3_table(const Geom3& g, Part3* parts, unsigned long long* status, unsigned long long* clear,
     uint32_t nclear, hipStream_t s)
 {
-    hipLaunchKernelGGL(k3_table, dim3(1 + std::min(nclear / 256, 255u)), dim3(256), 0, s, g.d1, g.d2, g.d3, (int) g.Bs,
-        (int) g.T, parts, status, clear, nclear);
+    hipLaunchKernelGGL(k3_table, dim3(1 + std::min(nclear / 256, 255u)), dim3(256), 0, s, g, split3(g), parts, status,
+        clear, nclear);
     return hipGetLastError();
 }
 
