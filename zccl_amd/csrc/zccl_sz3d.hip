@@ -1000,6 +1000,38 @@ __device__ __forceinline__ void places3(unsigned long long* status, uint32_t t, 
 constexpr uint32_t kLaneBuf3 = 8192, kLaneReach3 = 8 + 4 * 64 + 16;
 static_assert(22 * 264 + kLaneReach3 <= kLaneBuf3, "a third of the widest payloads fits");
 
+// Where on: C runs of From values each, of which the first To count, closed up.
+template <uint32_t From, uint32_t To, uint32_t C>
+__device__ __forceinline__ void close3(uint32_t (&m)[64], bool on)
+{
+#pragma unroll
+    for (uint32_t v = To; v < C * To; v++) {
+        const uint32_t there = m[v], moved = m[v / To * From + v % To];
+        m[v] = on ? moved : there;
+    }
+}
+
+// The values of blocks with rows of R values (R < 4: only those, else all) closed
+// up along z, then their n rows to a plane along y (n = 1 to 3; 0: no such blocks).
+// (The empty asm ends each branch differently: the compiler would otherwise merge
+// their last stores into one of a chosen address, and keep m in scratch memory.)
+template <uint32_t R>
+__device__ __forceinline__ void close_block3(uint32_t (&m)[64], bool rows, bool planes, uint32_t n)
+{
+    if (R < 4)
+        close3<4, R, 16>(m, rows);
+    if (n == 1) {
+        close3<4 * R, R, 4>(m, rows && planes);
+        asm volatile("; y1");
+    } else if (n == 2) {
+        close3<4 * R, 2 * R, 4>(m, rows && planes);
+        asm volatile("; y2");
+    } else if (n == 3) {
+        close3<4 * R, 3 * R, 4>(m, rows && planes);
+        asm volatile("; y3");
+    }
+}
+
 template <uint32_t W>
 __global__ void __launch_bounds__(64 * W, 3) k3l_compress(Sz3Args a)
 {
@@ -1095,36 +1127,26 @@ __global__ void __launch_bounds__(64 * W, 3) k3l_compress(Sz3Args a)
     uint32_t* buf = s_buf[wv];
     const uint32_t cnt = ex * ey * ez;
     if (any_edge) {
-        // blocks at a far edge: their values closed up in order (through LDS,
-        // half the lanes at a time), zeros behind them
-        for (uint32_t h = 0; h < 2; h++) {
-            const bool mine = (lane >> 5) == h;
-            if (mine) {
-#pragma unroll
-                for (uint32_t v = 0; v < 64; v++)
-                    buf[32 * v + (lane & 31)] = m[v];
-            }
-            wave_sync_lds();
-            if (mine && edge) {
-                uint32_t at = lane & 31, j = 0, k = 0;  // at: of value (i, j, k)
-                const uint32_t ey1 = stay(ey), ez1 = stay(ez);
-#pragma unroll
-                for (uint32_t e = 0; e < 64; e++) {
-                    const uint32_t v = buf[min(at, 32u * 63 + 31)];
-                    m[e] = e < cnt ? v : 0u;
-                    k++;
-                    at += 32;
-                    const bool row = k == ez1;
-                    at += row ? 32 * (4 - ez1) : 0u;
-                    j += row ? 1u : 0u;
-                    k = row ? 0u : k;
-                    const bool plane = j == ey1;
-                    at += plane ? 128 * (4 - ey1) : 0u;
-                    j = plane ? 0u : j;
-                }
-            }
-            wave_sync_lds();
+        // blocks at a far edge: their values closed up in order, zeros behind
+        // them.  A sub-volume's last blocks along a dim all have the same extent,
+        // so each move is one select with its place known (289 x 44 x 41: 17 us, 28 by
+        // one walk for every extent, half the lanes at a time through LDS).
+        const bool y = ey < 4, z = ez < 4;
+        const uint32_t n = __any(y) ? p.sy & 3 : 0u, k = any_z ? p.sz & 3 : 0u;
+        close_block3<4>(m, !z, y, n);
+        if (k == 1) {
+            close_block3<1>(m, z, y, n);
+            asm volatile("; z1");
+        } else if (k == 2) {
+            close_block3<2>(m, z, y, n);
+            asm volatile("; z2");
+        } else if (k == 3) {
+            close_block3<3>(m, z, y, n);
+            asm volatile("; z3");
         }
+#pragma unroll
+        for (uint32_t v = 0; v < 64; v++)
+            m[v] = v < cnt ? m[v] : 0u;
     }
     // signs, magnitudes, width and size
     uint32_t s0 = 0, s1 = 0, mx = 0;
