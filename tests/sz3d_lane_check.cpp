@@ -3,6 +3,7 @@
 //
 //   routes   volumes with too few rows or columns to fill the chip are left to
 //            the tiled decoder, larger ones take the lane decoder
+//   rows     the lane compress takes rows of any length in 32-bit offsets
 //
 // Built and run by tests/test_sz3d_lane.py with g++; prints "ok <cases>" or the
 // first violation.
@@ -49,9 +50,31 @@ static void routes()
     }
 }
 
+// Every volume of block side 4 takes the lane compress, also those with rows of
+// 2^27 values and more (the generic kernels' launch of a wave per block is too
+// large for some of them); row offsets and block numbers fit 32 signed bits.
+static void long_rows()
+{
+    const uint32_t v[][4] = {{1, 1, (1u << 27) - 1, 1}, {1, 1, 1u << 27, 1}, {2, 2, 1u << 27, 4}, {1, 3, (1u << 27) + 1001, 1},
+        {1, 4, (1u << 29) - 1, 1}, {1, 2, (1u << 30) - 1, 1}, {1, 1, 0x7FFFFFFFu, 1}, {3, 1, 715827882u, 3}};
+    for (const auto& x : v) {
+        Geom3 g;
+        std::vector<Part3> parts(x[3]);
+        REQUIRE(make_geom3(x[0], x[1], x[2], 4, (int) x[3], &g, parts.data()), "geometry");
+        REQUIRE(g.nlane > 0 && g.nlane <= g.nblocks, "%ux%ux%u: %u tiles", x[0], x[1], x[2], g.nlane);
+        REQUIRE((uint64_t) g.nlane * g.wlane * 64 < (1ull << 32), "threads of the launch");
+        const uint64_t rows = g.d2 < 4 ? g.d2 : 4;  // rows -1 .. 3 of a block, those there are
+        REQUIRE((rows - 1) * g.d3 < (1ull << 31) && g.d3 < (1ull << 31), "row offsets");
+        for (const Part3& p : parts)
+            REQUIRE((uint64_t) p.b1 * p.b2 * p.b3 + 64 * g.wlane < (1ull << 31), "block numbers");
+        g_cases++;
+    }
+}
+
 int main()
 {
     routes();
+    long_rows();
     std::printf("ok %ld\n", g_cases);
     return 0;
 }

@@ -69,13 +69,12 @@ ZK_HD constexpr uint32_t tile_nz3(uint32_t Bs) { return Bs == 4 ? 64u : Bs == 8 
 // Lane compress (block side 4): one lane per block, a wave per run of
 // kLaneRun3 blocks of a sub-volume in stream order (lane 0 holds the block
 // before the run), kLaneWide3 waves per workgroup tile, or kLaneSlim3 below
-// kLaneFew3 values, where wide tiles leave compute units idle.  Rows are
-// addressed by 32-bit offsets, so longer ones than kLaneMaxRow3 take the
-// generic kernels.
+// kLaneFew3 values, where wide tiles leave compute units idle.  A block's rows
+// are addressed by 32-bit offsets: at most 3 d3 with four of them, which is below
+// the volume's values (kMaxN).
 constexpr uint32_t kLaneRun3 = 63;
 constexpr uint32_t kLaneSlim3 = 4, kLaneWide3 = 12;
 constexpr uint64_t kLaneFew3 = 64ull * kLaneRun3 * kLaneWide3 * 256;
-constexpr uint32_t kLaneMaxRow3 = 1u << 27;
 
 // Lane decoder (block side 4): one lane per block, a wave per run of 64 blocks
 // along z (kLaneRuns3 to a row at most), a workgroup per row of blocks and
@@ -171,7 +170,7 @@ ZK_HD Sums3 part3(const Geom3& g, const Split3& s, uint32_t t, Part3& p)
     p.b2 = nblk3(p.sy, g.Bs);
     p.b3 = nblk3(p.sz, g.Bs);
     const uint32_t cols = p.b1 * p.b2, segs = (p.b1 + kLaneSeg3 - 1) / kLaneSeg3;
-    const uint32_t nz = tile_nz3(g.Bs), lane = g.Bs == 4 && g.d3 < kLaneMaxRow3 ? g.wlane * kLaneRun3 : 0u;
+    const uint32_t nz = tile_nz3(g.Bs), lane = g.Bs == 4 ? g.wlane * kLaneRun3 : 0u;
     Sums3 c = {{cols * p.b3, p.sx * p.sy, p.sx * p.sz, p.sy * p.sz, nz ? cols * ((p.b3 + nz - 1) / nz) : 0u, cols,
         lane ? (cols * p.b3 + lane - 1) / lane : 0u, cols * ((p.b3 + 63) / 64), p.b2 * segs, (segs - 1) * p.sy * p.sz,
         p.b1 * p.sz}};
