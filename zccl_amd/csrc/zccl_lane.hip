@@ -19,8 +19,9 @@
 // 16-byte stores.
 //
 // A segment's short last block takes the same path as a whole one (its fields
-// are placed by its length).  Blocks of width 16 and more, and tiles larger
-// than half the buffer, take passes of their own through the whole buffer.
+// are placed by its length).  Blocks of width 16 and more have a decoder of
+// their own, after the others of their tile; tiles larger than half the buffer
+// take a pass of their own through the whole buffer.
 // Measured against one decoder for whole blocks below width 16 with the others
 // read value by value from memory, and an FP64 quantizer: two 1 MB operands
 // 15.8 -> 13.8 us, sixteen 8 MB ones 60 -> 31 us, 8 sums of 8 x 2^24 values
@@ -504,9 +505,9 @@ __device__ __forceinline__ void homsum_tile_lane(const Geom& g, const Tiling& tl
 #pragma unroll
     for (uint32_t j = 0; j < L; j++)
         acc[j] = 0;
-    // bit r (uniform): operand r's tile does not fit a half, or has a block of
-    // width 16 or more: (the rest of) it is left to the pass below
-    uint32_t whole = 0, high = 0;
+    // bit r (uniform): operand r's tile does not fit a half and is left to the
+    // pass below
+    uint32_t whole = 0;
 
     // ---- operand pipeline: operand r+1's tile bytes move into the other LDS
     // half while operand r is decoded, operand r+2's widths are on their way
@@ -514,63 +515,88 @@ __device__ __forceinline__ void homsum_tile_lane(const Geom& g, const Tiling& tl
         Op on = op_of(0);
         Loc cn = locate(on, widths(on));
         bool hn = stage(cn, 0);
-        uint32_t wq2 = 0;
-        Op o2;
-        if (k > 1) {
-            o2 = op_of(1);
-            wq2 = widths(o2);
-        }
         // the sum's carry into the tile: the operands' carries add in int32
         // (while the first operand's bytes are on their way)
         carry = wave_scan_dpp(carry);
         if (lane == 63 && x.ngrp)
             index_view(g, oindex).carry[t] = carry;
-        // (a loop that runs at least once: its sums then have no second life
-        // as the zeros of an empty one)
-        int r = 0;
-        do {
-            const Loc c = cn;
-            const bool half = hn;
-            __builtin_amdgcn_s_waitcnt(0);  // operand r's bytes are in LDS, operand r+1's widths in registers
-            // a lane of a wider block, or of a tile that is not here, decodes
-            // zeros (without a branch: one would copy the sums)
-            const uint32_t w = half && c.w < 16 ? c.w : 0u, o = half ? c.o : 0u;
-            const bool wide = __any(w >= 8);
-            const uint32_t* st = obuf + ((uint32_t) r & 1u) * (kStageHalf / 4);
-            bad_byte |= (has && half) & (((const uint8_t*) st)[o] != c.w);
-            Block q;
-            read_block(st, o, w, nj, wide, q);
-            // (phase fences keep the scheduler from interleaving the block
-            // reads, the next operand's staging and the decode, which would
-            // hold all their values at once)
-            __builtin_amdgcn_sched_barrier(0);
-            if (r + 1 < k) {
-                cn = locate(o2, wq2);
-                hn = stage(cn, (uint32_t) (r + 1) & 1u);
-            }
-            if (r + 2 < k) {
-                o2 = op_of(r + 2);
+        if (hn || cn.skip) {
+            Op o2;
+            uint32_t wq2 = 0;
+            if (k > 1) {
+                o2 = op_of(1);
                 wq2 = widths(o2);
             }
-            __builtin_amdgcn_sched_barrier(0);
-            bad_over |= c.skip;
-            whole |= !half && !c.skip ? 1u << r : 0u;
-            high |= half && __any(c.w >= 16) ? 1u << r : 0u;
-            each_value(q, w, wide, [&](uint32_t j, uint32_t v, uint32_t sign) { acc[j] = mad_i24(v, sign, acc[j]); });
-        } while (++r < k);
+            // (a loop that runs at least once: its sums then have no second life
+            // as the zeros of an empty one)
+            int r = 0;
+            do {
+                const Loc c = cn;
+                const bool half = hn;
+                __builtin_amdgcn_s_waitcnt(0);  // operand r's bytes are in LDS, operand r+1's widths in registers
+                // a lane of a wider block, or of a tile that is not here, decodes
+                // zeros (without a branch: one would copy the sums)
+                const uint32_t w = half && c.w < 16 ? c.w : 0u, o = half ? c.o : 0u;
+                const bool wide = __any(w >= 8);
+                const uint32_t* st = obuf + ((uint32_t) r & 1u) * (kStageHalf / 4);
+                bad_byte |= (has && half) & (((const uint8_t*) st)[o] != c.w);
+                Block q;
+                read_block(st, o, w, nj, wide, q);
+                // (phase fences keep the scheduler from interleaving the block
+                // reads, the next operand's staging and the decode, which would
+                // hold all their values at once)
+                __builtin_amdgcn_sched_barrier(0);
+                if (r + 1 < k) {
+                    cn = locate(o2, wq2);
+                    hn = stage(cn, (uint32_t) (r + 1) & 1u);
+                }
+                if (r + 2 < k) {
+                    o2 = op_of(r + 2);
+                    wq2 = widths(o2);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                bad_over |= c.skip;
+                whole |= !half && !c.skip ? 1u << r : 0u;
+                each_value(q, w, wide, [&](uint32_t j, uint32_t v, uint32_t sign) { acc[j] = mad_i24(v, sign, acc[j]); });
+                // (its bytes stay until operand r+2's)
+                if (half && __builtin_expect(__any(c.w >= 16), 0)) {
+                    if (c.w >= 16)
+                        decode_any(st, c.o, c.w, nj, acc);
+                }
+            } while (++r < k);
+        } else {
+            // the first does not fit a half: nor will most of the others
+            whole = ~0u >> (32 - k);
+        }
     }
-    // the operands left over, one at a time through the whole buffer
-    for (uint32_t left = whole | high; __builtin_expect(left != 0, 0); left &= left - 1) {
-        const int r = __builtin_ctz(left);
-        const Op op = op_of(r);
-        const Loc c = locate(op, widths(op));
-        const bool all = (whole >> r) & 1u;
-        stage_bytes(c.v, c.tot, obuf);
-        __builtin_amdgcn_s_waitcnt(0);
-        const bool mine = has && (all || c.w >= 16);
-        bad_byte |= mine & (((const uint8_t*) obuf)[c.o] != c.w);
-        if (mine && c.w)
-            decode_any(obuf, c.o, c.w, nj, acc);
+    // the operands left over, one at a time through the whole buffer, the next
+    // one's widths on their way with the bytes of one.  (Twelve operands of 365 KB
+    // with widths 15 to 17: 43 us, where a second fetch for every tile with a block
+    // from width 16, and a pass of zeros for every one larger than a half, took 51;
+    // eight of 16 MB: 48 and 55.)
+    if (uint32_t left = whole; __builtin_expect(left != 0, 0)) {
+        int r = __builtin_ctz(left);
+        Op op = op_of(r);
+        uint32_t wq = widths(op);
+        while (true) {
+            const Loc c = locate(op, wq);
+            const bool mine = has && !c.skip;
+            bad_over |= c.skip;
+            if (!c.skip)
+                stage_bytes(c.v, c.tot, obuf);
+            left &= left - 1;
+            if (left) {
+                r = __builtin_ctz(left);
+                op = op_of(r);
+                wq = widths(op);
+            }
+            __builtin_amdgcn_s_waitcnt(0);
+            bad_byte |= mine & (((const uint8_t*) obuf)[c.o] != c.w);
+            if (mine && c.w)
+                decode_any(obuf, c.o, c.w, nj, acc);
+            if (!left)
+                break;
+        }
     }
     if (__any(nj < L)) {
         // values past a short block's end decoded what follows it
