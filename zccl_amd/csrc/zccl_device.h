@@ -211,10 +211,10 @@ __device__ __forceinline__ unsigned long long lookback(unsigned long long* statu
 // too small (then no workgroup of the launch takes a ticket or does anything).
 // With tiles_per_group > 1 a ticket stands for that many consecutive tiles
 // (one per wave of the workgroup) and t is the first of them.
+// s_ticket: a word of the workgroup's LDS.
 __device__ __forceinline__ bool launch_status(WsHeader* ws, uint64_t ntiles_total, uint64_t& t,
-    unsigned long long*& status, uint32_t tiles_per_group = 1)
+    unsigned long long*& status, uint32_t tiles_per_group, unsigned long long* s_ticket)
 {
-    __shared__ unsigned long long s_ticket;
     const uint64_t cap = ws->capacity;
     if (cap < ntiles_total) {
         if (threadIdx.x == 0 && blockIdx.x == 0)
@@ -222,9 +222,9 @@ __device__ __forceinline__ bool launch_status(WsHeader* ws, uint64_t ntiles_tota
         return false;
     }
     if (threadIdx.x == 0)
-        s_ticket = atomicAdd(&ws->seq, 1ull);
+        *s_ticket = atomicAdd(&ws->seq, 1ull);
     __syncthreads();
-    const unsigned long long tk = s_ticket;
+    const unsigned long long tk = *s_ticket;
     const uint32_t par = (uint32_t) (tk >> 32) & 1u;
     const uint64_t ticket = (uint32_t) tk;
     t = ticket * tiles_per_group;
@@ -236,6 +236,13 @@ __device__ __forceinline__ bool launch_status(WsHeader* ws, uint64_t ntiles_tota
     for (uint64_t i = lo + threadIdx.x; i < hi; i += blockDim.x)
         other[i * kStatusStride] = 0;
     return true;
+}
+
+__device__ __forceinline__ bool launch_status(WsHeader* ws, uint64_t ntiles_total, uint64_t& t,
+    unsigned long long*& status, uint32_t tiles_per_group = 1)
+{
+    __shared__ unsigned long long s_ticket;
+    return launch_status(ws, ntiles_total, t, status, tiles_per_group, &s_ticket);
 }
 
 // Called by one thread of the last tile of a lookback chain once that tile

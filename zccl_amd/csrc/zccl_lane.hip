@@ -57,9 +57,9 @@ constexpr uint32_t SB = (L + 7) / 8;    // sign bytes of a whole block
 constexpr uint32_t NHI = L / 4;         // dwords of one high byte per value
 constexpr uint32_t NGRP = (L + 7) / 8;  // groups of (up to) 8 values in the low bits
 constexpr uint32_t kWorstBlock = 1 + SB + 4 * L;   // 150 bytes at width 32
-// Output buffer of one wave: 10 KB, so that four workgroups of four waves
-// share a CU's 160 KB of LDS (the sum's loop holds 108 registers, more than the
-// 96 that five would leave a wave).  The worst tile's bytes (64 blocks of
+// Output buffer of one wave: 10 KB, so that a CU's 160 KB of LDS hold those of
+// sixteen waves, and nothing else (the sum's loop holds 108 to 120 registers, and
+// more than 96 leave four waves to a SIMD).  The worst tile's bytes (64 blocks of
 // kWorstBlock) fit, with the reach of the block reads and OR-writes past them.
 constexpr uint32_t kOutBuf = 10240;
 // Block reads and writes cover 36 values whatever the block holds: a short
@@ -398,6 +398,26 @@ struct WgShared {
     uint32_t wtot[kLaneWaves];
     unsigned long long ex;
 };
+
+// The state of a workgroup of a sum, in the last bytes of its last wave's buffer,
+// which neither the staging nor the encoder writes (the block reads past half
+// one's bytes take it for garbage).  As static LDS beside the buffers it left a
+// CU three workgroups of four waves for four, and one of eight for two: 8 operands
+// of 2^24 values in one pass 90.7 -> 87.5 us by four waves, 100.4 -> 80.1 by eight.
+struct SumShared {
+    unsigned long long ticket;
+    WgShared wg;
+};
+static_assert(kStageHalf + kStageCap + sizeof(SumShared) <= kOutBuf && sizeof(SumShared) % 8 == 0 &&
+        kLaneTileBlocks * kWorstBlock + 16 + kReach + sizeof(SumShared) <= kOutBuf,
+    "the workgroup's state lies behind what the waves write");
+static_assert(16 / kLaneWaves * kLaneWaves * kOutBuf <= 160 * 1024, "sixteen waves' buffers fit a CU's LDS");
+
+template <uint32_t W>
+__device__ __forceinline__ SumShared& sum_shared()
+{
+    return *reinterpret_cast<SumShared*>(zk_lds + (W * kOutBuf - sizeof(SumShared)) / 4);
+}
 
 // Forms of the lane sum's output side.
 enum SumMode : int {
@@ -1438,7 +1458,7 @@ __global__ void __launch_bounds__(64 * W, 4) k_homsum_lane(HomsumArgs a)
 {
     uint64_t t0;
     unsigned long long* status;
-    if (!launch_status(a.ws, a.job.tl.ntiles, t0, status, W))
+    if (!launch_status(a.ws, a.job.tl.ntiles, t0, status, W, &sum_shared<W>().ticket))
         return;
     const uint32_t wv = threadIdx.x >> 6;
     const uint64_t t = t0 + wv;
@@ -1456,7 +1476,7 @@ __global__ void __launch_bounds__(64 * W, 4) k_homsum_lane_batch(BatchArgs b)
 {
     uint64_t t0;
     unsigned long long* status;
-    if (!launch_status(b.ws, b.total_tiles, t0, status, W))
+    if (!launch_status(b.ws, b.total_tiles, t0, status, W, &sum_shared<W>().ticket))
         return;
     const uint32_t wv = threadIdx.x >> 6;
     const uint64_t tg = t0 + wv;
@@ -1486,7 +1506,7 @@ __global__ void __launch_bounds__(64 * W, 4) k_homsum_lane_mixed(BatchArgs b)
 {
     uint64_t t0;
     unsigned long long* status;
-    if (!launch_status(b.ws, b.total_tiles, t0, status, W))
+    if (!launch_status(b.ws, b.total_tiles, t0, status, W, &sum_shared<W>().ticket))
         return;
     const uint32_t wv = threadIdx.x >> 6;
     const uint64_t tg = t0 + wv;
@@ -1643,10 +1663,10 @@ __device__ __forceinline__ Tile wg_wave_tile(const Geom& g, const Tiling& tl, co
 
 __global__ void __launch_bounds__(64 * kLaneWaves, 4) k_homsum_lane_wg(HomsumArgs a)
 {
-    __shared__ WgShared sh;
+    SumShared& sh = sum_shared<kLaneWaves>();
     uint64_t t_wg;
     unsigned long long* status;
-    if (!launch_status(a.ws, a.job.tl.ntiles, t_wg, status))
+    if (!launch_status(a.ws, a.job.tl.ntiles, t_wg, status, 1, &sh.ticket))
         return;
     const uint32_t wv = threadIdx.x >> 6;
     const Tiling tl = make_lane_tiling(a.job.g);
@@ -1655,16 +1675,16 @@ __global__ void __launch_bounds__(64 * kLaneWaves, 4) k_homsum_lane_wg(HomsumArg
     const ArgIO src{a.job.io};
     homsum_tile_lane<kSumWg>(a.job.g, tl, a.job.p.k, src, a.job.io.out, a.job.io.out_cap, a.job.io.index,
         a.job.io.size_out, t_lane, status, a.ws, 1, zk_lds + wv * (kOutBuf / 4), nullptr, 0, 0, t_wg,
-        t_wg == a.job.tl.ntiles - 1, &sh, &x);
+        t_wg == a.job.tl.ntiles - 1, &sh.wg, &x);
 }
 
 // (four workgroups per CU: at five the workgroup state spills)
 __global__ void __launch_bounds__(64 * kLaneWaves, 4) k_homsum_lane_wg_batch(BatchArgs b)
 {
-    __shared__ WgShared sh;
+    SumShared& sh = sum_shared<kLaneWaves>();
     uint64_t tg;
     unsigned long long* status;
-    if (!launch_status(b.ws, b.total_tiles, tg, status))
+    if (!launch_status(b.ws, b.total_tiles, tg, status, 1, &sh.ticket))
         return;
     uint32_t jidx, t;
     if (b.interleave) {
@@ -1684,15 +1704,15 @@ __global__ void __launch_bounds__(64 * kLaneWaves, 4) k_homsum_lane_wg_batch(Bat
     const SumIO src{io};
     homsum_tile_lane<kSumWg>(b.g, tl, b.p.k, src, ldc(&io->out), ldc(&io->out_cap), ldc(&io->index),
         ldc(&io->size_out), t_lane, status + (uint64_t) jidx * b.tl.ntiles * kStatusStride, b.ws, b.total_chains,
-        zk_lds + wv * (kOutBuf / 4), nullptr, 0, 0, t, t == b.tl.ntiles - 1, &sh, &x);
+        zk_lds + wv * (kOutBuf / 4), nullptr, 0, 0, t, t == b.tl.ntiles - 1, &sh.wg, &x);
 }
 
 __global__ void __launch_bounds__(64 * kLaneWaves, 4) k_homsum_lane_wg_mixed(BatchArgs b)
 {
-    __shared__ WgShared sh;
+    SumShared& sh = sum_shared<kLaneWaves>();
     uint64_t tg;
     unsigned long long* status;
-    if (!launch_status(b.ws, b.total_tiles, tg, status))
+    if (!launch_status(b.ws, b.total_tiles, tg, status, 1, &sh.ticket))
         return;
     uint32_t lo = 0, hi = b.njobs;
     while (hi - lo > 1) {
@@ -1715,7 +1735,7 @@ __global__ void __launch_bounds__(64 * kLaneWaves, 4) k_homsum_lane_wg_mixed(Bat
     const SumIO src{&job->io};
     homsum_tile_lane<kSumWg>(g, tl, ldc(&job->p.k), src, ldc(&job->io.out), ldc(&job->io.out_cap),
         ldc(&job->io.index), ldc(&job->io.size_out), t_lane, status + tile0 * kStatusStride, b.ws, b.total_chains,
-        zk_lds + wv * (kOutBuf / 4), nullptr, 0, 0, t, t == tw.ntiles - 1, &sh, &x);
+        zk_lds + wv * (kOutBuf / 4), nullptr, 0, 0, t, t == tw.ntiles - 1, &sh.wg, &x);
 }
 
 // ---------------------------------------------------------------- two-pass sum
