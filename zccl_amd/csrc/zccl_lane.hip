@@ -1446,11 +1446,13 @@ __device__ __forceinline__ void compress_tile_lane(const Geom& g, const Tiling& 
 }  // namespace
 
 // Waves (tiles) that share a ticket of a sum: tickets are adds to one address,
-// 12 ns each, so beyond kSumFew tiles, which fill the chip's 1024 SIMDs with four
-// waves each, they bound the kernel and eight waves share one (32 mixed buckets:
-// 88.6 -> 79.2 us); below, smaller workgroups start sooner (868 tiles of 16
-// operands: 34.0 us, with eight 38.4).
-constexpr uint32_t kSumMany = 8, kSumFew = 4096;
+// 12 ns each, so beyond kSumFew tiles, one for each of the chip's 1024 SIMDs, eight
+// waves share one; below, smaller workgroups start sooner and spread over more
+// compute units.  us by four / eight waves: 343 tiles of 16 operands 29.6 / 36.5, 881
+// 32.1 / 39.7, 912 of 8 23.9 / 28.2; 1824 34.2 / 31.3, 2168 (mixed batch) 38.5 / 38.7,
+// 3727 (mixed, 16 operands) 69.0 / 64.5, 8656 (mixed, 4) 76.1 / 70.7, 7296 of 8 87.5 /
+// 80.1.
+constexpr uint32_t kSumMany = 8, kSumFew = 1024;
 
 // One fused sum (kernel arguments hold its geometry and pointers).
 template <uint32_t W>
