@@ -91,9 +91,6 @@ __device__ __forceinline__ uint32_t lane_block_bytes(uint32_t w, uint32_t n)
 }
 
 using View = __amdgpu_buffer_rsrc_t;
-// Four floats at 4-byte alignment (one 16-byte store where the address is
-// only dword aligned).
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 // Range-checked view of [base, base + bytes) (base 4-byte aligned, bytes a
 // multiple of 4).  A buffer load returns zeros for every dword that does not
@@ -486,10 +483,10 @@ __device__ __forceinline__ void homsum_tile_lane(const Geom& g, const Tiling& tl
     // view of the tile bytes (one scan of the block sizes), and whether the
     // tile lies inside its stream.  The view starts at the 4-byte aligned
     // address at or below the tile's bytes and ends with the stream's last
-    // dword (lim: its length).
+    // dword.
     struct Loc {
         View v;
-        uint32_t w, bs, o, lim, tot;
+        uint32_t w, bs, o, tot;
         bool skip;
     };
     auto locate = [&](const Op& p, uint32_t wq) {
@@ -506,7 +503,6 @@ __device__ __forceinline__ void homsum_tile_lane(const Geom& g, const Tiling& tl
         const uint8_t* base = p.bytes + p.goff;
         const uint32_t delta = (uint32_t) ((uintptr_t) base & 3u);
         const uint64_t len = c.skip ? 0ull : align_up(delta + (p.size - p.goff), 4);
-        c.lim = len > 0xFFFFFFFCull ? 0xFFFFFFFCu : (uint32_t) len;
         c.v = make_view(base - delta, len);
         c.o = delta + incl - c.bs;
         c.tot += delta;  // bytes of the view that hold the tile
