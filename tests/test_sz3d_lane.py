@@ -1,5 +1,5 @@
-"""Host replay of the lane kernels' work split of the 3-D codec, block side 4
-(tests/sz3d_lane_check.cpp)."""
+"""Host replay of the lane kernels' work split: the 3-D codec with block side 4,
+and the carries of the 1-D index (tests/sz3d_lane_check.cpp)."""
 import os
 import subprocess
 
