@@ -1713,7 +1713,7 @@ __global__ void __launch_bounds__(kParseSpecThreads) k_parse_spec(ParseArgs a, P
     // workgroups no longer stand between those with work (2^24 values in 16
     // chunks: 65.7 -> 59.1 us; the emit, four tiles to a workgroup, in the same
     // order: 37.3 -> 29.6)
-    const uint32_t c = blockIdx.x % a.g.T, t = blockIdx.x / a.g.T;
+    const uint32_t t = blockIdx.x / a.g.T, c = parse_chunk(t, blockIdx.x % a.g.T, a.g.T);
     const uint64_t gt = (uint64_t) c * pl.tpc + t;
     uint64_t cs, ce;
     if (!parse_region(a, pl, c, cs, ce))
@@ -1960,7 +1960,7 @@ __global__ void __launch_bounds__(256) k_parse_emit(ParseArgs a, ParseLayout pl)
     // (the wave index read as uniform: the walk below then runs on scalar registers)
     const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const Geom& g = a.g;
-    const uint32_t c = blockIdx.x % g.T, t = 4 * (blockIdx.x / g.T) + wv;
+    const uint32_t row = blockIdx.x / g.T, c = parse_chunk(row, blockIdx.x % g.T, g.T), t = 4 * row + wv;
     if (t >= pl.tpc)
         return;
     const uint64_t gt = (uint64_t) c * pl.tpc + t;
