@@ -19,7 +19,10 @@
  *     Every device stream travels with an index (block widths, tile and seed
  *     offsets, stream size, for 36-value blocks the quantized value before
  *     every 64 blocks) that the kernels use instead of walking the bytes; its
- *     layout belongs to the library version that wrote it.
+ *     layout belongs to the library version that wrote it.  These calls take no
+ *     index size: an index must be of zccl_index_bytes() bytes, from this
+ *     library's compress, sum or zccl_parse_dev (the Python layer, which knows
+ *     the size, parses the bytes again under an index kept from another).
  *
  * Streams are byte-identical to the reference's for the same input, error
  * bound, block length and chunk count.
@@ -218,7 +221,7 @@ int zccl_homsum_dev_noalloc(const unsigned char *const *ins, const void *const *
  * CPU library); reads at most in_cap bytes of `in`.  The reference walks
  * each chunk sequentially (ZCCL/src/ZCCLd_float.c:597-745); with a workspace
  * of zccl_parse_workspace_bytes() bytes and chunks of at least 256 blocks
- * (blockSize <= 64) the walk runs in parallel over 4 KB tiles of every
+ * (blockSize <= 64) the walk runs in parallel over 2 KB tiles of every
  * chunk, otherwise one wave walks each chunk. */
 int zccl_parse_dev(const unsigned char *in, size_t in_cap, size_t nbEle, int blockSize,
     int nchunks, void *index, unsigned long long *d_size, void *workspace, size_t workspace_bytes,

@@ -13,7 +13,8 @@ Knobs (C ABI ``zccl_tune_*``; none changes the stream bytes):
                   workgroup of four waves;
 * ``stage``    -- smallest operand stage of the slot-layout sum, in bytes;
 * ``two_pass`` -- sums of at least this many tiles take the two-pass form;
-* ``groups``   -- workgroups per CU of the persistent lane decompress.
+* ``groups``   -- workgroups per CU of the persistent lane decompress (four are
+                  resident; of five, the fifth waits for another's LDS).
 
 ``tune`` times a caller-supplied run at each configuration of an op's space
 and keeps the fastest.  ``run`` must build whatever depends on the tiling

@@ -40,7 +40,7 @@ def _ptr(t: torch.Tensor) -> ctypes.c_void_p:
 
 # Sizes that follow from (n, L, T) alone are kept: a call into the library for
 # each is a microsecond of the host, which sets the pace of the smallest passes
-# (64 Ki values: kernel 9.4 us).  num_tiles depends on the tunables and is not.
+# (16384 values: kernel 9.4 us).  num_tiles depends on the tunables and is not.
 
 @functools.lru_cache(maxsize=4096, typed=True)
 def worst_case_bytes(n: int, L: int, T: int) -> int:

@@ -1710,9 +1710,9 @@ __global__ void __launch_bounds__(kParseSpecThreads) k_parse_spec(ParseArgs a, P
     const uint32_t tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
     // the first tiles of all chunks, then the second ones, ...: a chunk's last
     // tiles are mostly past its region (sized for the worst case), and their
-    // workgroups no longer stand between those with work (2^24 values in 16
-    // chunks: 65.7 -> 59.1 us; the emit, four tiles to a workgroup, in the same
-    // order: 37.3 -> 29.6)
+    // workgroups do not stand between those with work (2^24 values in 16 chunks, us
+    // chunk after chunk / so: 65.7 / 59.7; the emit, four tiles to a workgroup, 37.3 /
+    // 31.0)
     const uint32_t t = blockIdx.x / a.g.T, c = parse_chunk(t, blockIdx.x % a.g.T, a.g.T);
     const uint64_t gt = (uint64_t) c * pl.tpc + t;
     uint64_t cs, ce;

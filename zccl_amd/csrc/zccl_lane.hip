@@ -1,8 +1,9 @@
 // zccl_lane.hip -- block-per-lane kernels for 36-value blocks, the
 // reference's default block length (examples/compression_allreduce.c,
-// jobs/*.sh): the fused homomorphic sum.
+// jobs/*.sh): the fused homomorphic sum, decompress with the carries of a parsed
+// stream, and compress.
 //
-// Layout.  A wave owns one tile of 64 consecutive blocks of one segment and
+// Layout (of the sum; the others' stand at their sections).  A wave owns one tile of 64 consecutive blocks of one segment and
 // every lane owns one whole block.  An operand's tile bytes move into the
 // wave's LDS buffer with range-checked direct-to-LDS loads (a read past the
 // operand's stream returns zeros, so no read ever leaves the stream) and each
@@ -23,11 +24,10 @@
 // their own, after the others of their tile; tiles larger than half the buffer
 // take a pass of their own through the whole buffer.
 // Measured against one decoder for whole blocks below width 16 with the others
-// read value by value from memory, and an FP64 quantizer: two 1 MB operands
-// 15.8 -> 13.8 us, sixteen 8 MB ones 60 -> 31 us, 8 sums of 8 x 2^24 values
-// 458 -> 421 us, the allreduce of velocities (widths 15 to 17) 383 -> 241 us,
-// compress of 2^24 values 50.6 -> 48.2 us, decompress of 16411 values (a short
-// block in every tile) 11.4 -> 8.7 us.
+// read value by value from memory: two 1 MB operands 15.7 -> 13.8 us, sixteen 8 MB
+// ones 60 -> 31 us, 8 sums of 8 x 2^24 values 457 -> 422 us, the staged allreduce of
+// 4 ranks' velocities (widths 15 to 17) 383 -> 220 us, decompress of 16411 values (a
+// short block in every tile) 11.4 -> 8.9 us.
 //
 // Wire format and arithmetic (reference):
 //   block      width byte, sign bitmap MSB first, (w>>3) high bytes per
@@ -1210,10 +1210,11 @@ __device__ __forceinline__ void carry_scan(const Geom& g, const uint8_t* bytes, 
 //
 // A workgroup of four waves owns a tile of 256 blocks (make_lane_wg_tiling),
 // wave w blocks 64w .. 64w + 63, one block per lane.  Each wave stages its
-// blocks' values and the one before them into its LDS buffer (16-byte
-// direct-to-LDS loads through a range-checked view of the input; reads past
-// the input return zeros), each lane reads its block's 36 values and the one
-// before, quantizes them (FP64 product, truncation), takes the deltas, the
+// blocks' values into its LDS buffer (16-byte direct-to-LDS loads through a
+// range-checked view of them; reads past it return zeros) and lane 0 loads the
+// value before them; each lane reads its block's 36 values, quantizes them
+// (FP32 products rounded toward zero, below; FP64 where a wave's values reach
+// further), takes the last quantized value of the lane below, the deltas, the
 // sign words, the magnitudes and the width, and the wave scans the block
 // sizes.  The workgroup adds its waves' sizes, publishes the tile's
 // aggregate, encodes every block into the wave buffers (the lane encoders of
@@ -1222,8 +1223,9 @@ __device__ __forceinline__ void carry_scan(const Geom& g, const uint8_t* bytes, 
 // Arithmetic: ZCCL/src/ZCCL_float.c:563,577-606 (quantize, delta, width),
 // ZCCL/src/ZCCL_TypeManager.c:12-91, 824-848 (packing, signs).
 
-// Quantize by FP32: x / bound is exact in 48 bits, and FP32 rounding toward
-// zero keeps its integer part below 2^24; a second product with 2^-149,
+// Quantize by FP32: the reciprocal of the bound is an FP32 number (inverse_bound;
+// the kernels' double holds no more, and turning it back loses nothing), its
+// product with x is exact in 48 bits, and FP32 rounding toward zero keeps its integer part below 2^24; a second product with 2^-149,
 // rounded toward zero too, drops the fraction and leaves the integer as a
 // denormal's bits, so deltas are FP32 differences (exact below 2^23).  Two
 // 2-cycle instructions and one to turn -0 into +0 in place of an FP64 product
@@ -1253,18 +1255,18 @@ __device__ __forceinline__ float from_lane_below(float v, float first)
     return as_f((uint32_t) __builtin_amdgcn_update_dpp((int) as_u(first), (int) as_u(v), 0x138, 0xF, 0xF, false));  // wave_shr:1
 }
 
-constexpr uint32_t kCompBuf = 9728;  // a wave's values (<= 2305 floats) or a worst-case 64-block encode + reach
+constexpr uint32_t kCompBuf = 9728;  // a wave's values (2304 floats) or a worst-case 64-block encode + reach
 static_assert(kCompBuf >= kLaneTileBlocks * kWorstBlock + 64 && kCompBuf >= (kLaneTileBlocks - 1) * kWorstBlock + kReach &&
         kCompBuf >= 4 * kLaneTileBlocks * L,
     "a compress wave buffer holds the staged values and the worst-case encode");
 static_assert(kCompBuf % 16 == 0, "compress wave buffers stay 16-byte aligned");
 
 // Tiles a workgroup takes with one ticket.  Tickets are adds to one address, 12
-// ns each: the 1820 of a 2^24-value stream took 22 us of the kernel's 47; two
-// tiles a ticket: 37 us (four: 34, but 136 us against 116 for the 8 streams of a
-// staged allreduce, whose tiles then end together).  Up to kCompFew tiles, one
-// for each compute unit, a tile has a workgroup of its own (7 tiles: 9.4 us
-// against 10.1).
+// ns each: the 1820 of a 2^24-value stream took 22 us of the kernel's 48; two
+// tiles a ticket: 37 us (four: 35, but 131 us against 110 for the 16 streams that 4
+// ranks of a staged allreduce compress, whose tiles then end together).  Up to
+// kCompFew tiles, one for each compute unit, a tile has a workgroup of its own (16
+// tiles: 9.4 us against 10.0; 336 tiles: 14.8 against 13.0).
 constexpr uint32_t kCompPair = 2, kCompFew = 256;
 
 struct CompShared {

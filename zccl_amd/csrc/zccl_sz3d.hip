@@ -12,9 +12,9 @@
 //              payload sizes -> k3_encode (one wave per block: width header
 //              byte, sub-volume offset, sign bitmap and fixed-length bits with
 //              the one-writer-per-byte unit encoder of the 1-D sum)
-//   decompress k3_table -> for block side 4 and rows of 32 to 256 blocks
-//              k3l_sizes, k3l_decode, k3l_ypass (one lane per block, two passes
-//              over the volume); others k3_dsizes (widths read from the stream's own
+//   decompress k3_table -> for block side 4, rows of 32 to 256 blocks and enough of
+//              them to fill the chip k3l_sizes, k3l_decode, k3l_ypass (one lane
+//              per block, two passes over the volume); others k3_dsizes (widths read from the stream's own
 //              header) -> scan -> k3_decode (residuals into the output buffer
 //              as int32) -> k3_zpass / k3_ypass (inclusive prefix sums along z
 //              and y) -> k3_xpass (along x, then x' = (float)(q * 2 eb) in place)
@@ -1240,7 +1240,7 @@ __global__ void __launch_bounds__(64 * W, 3) k3l_compress(Sz3Args a)
 // place.  The residuals never reach memory, which the tiled decoder's chunks
 // wrote (330 us for a 512^3 volume at a relative bound of 1e-3), the y pass (248)
 // and the x pass (238) read and wrote again: 849 us with the sizes.  This takes
-// 391: decode 146 (512 MB written; four waves a SIMD, 142 us at its registers'
+// 385: decode 146 (512 MB written; four waves a SIMD, 142 us at its registers'
 // limit, 176 with three), y pass 206 (1 GB at 5.2 TB/s, a copy reaches 5.5),
 // sizes and kept planes 30.  Volumes with blocks of fewer values (Edges) need 156
 // registers to move those to their places: 510^3 962 -> 565 us; in one kernel for
