@@ -970,8 +970,10 @@ __device__ __forceinline__ DecLoc dec_locate(const Args& a, const DecPre& p, uin
     const uint32_t binc = wave_scan_dpp(bs);
     const uint32_t tot0 = __builtin_amdgcn_readlane(binc, 63);
     // (the same in every lane: scalar, so that what depends on them branches)
+    // (a tile without blocks starts right behind its segment's seed, so this is
+    // the seed's check too; size 0: an index that holds no stream)
     const uint64_t goff = uniform64(p.goff), size = uniform64(p.size);
-    c.skip = goff > size || tot0 > size - goff;
+    c.skip = !size || goff > size || tot0 > size - goff;
     const uint8_t* base = d.bytes + goff;
     const uint32_t delta = (uint32_t) ((uintptr_t) base & 3u);
     const uint64_t vlen = c.skip ? 0ull : align_up(delta + (size - goff), 4);

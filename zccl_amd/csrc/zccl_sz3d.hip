@@ -14,10 +14,11 @@
 //              the one-writer-per-byte unit encoder of the 1-D sum)
 //   decompress k3_table -> for block side 4, rows of 32 to 256 blocks and enough of
 //              them to fill the chip k3l_sizes, k3l_decode, k3l_ypass (one lane
-//              per block, two passes over the volume); others k3_dsizes (widths read from the stream's own
-//              header) -> scan -> k3_decode (residuals into the output buffer
-//              as int32) -> k3_zpass / k3_ypass (inclusive prefix sums along z
-//              and y) -> k3_xpass (along x, then x' = (float)(q * 2 eb) in place)
+//              per block, two passes over the volume); others k3_dsizes (widths
+//              read from the stream's own header) -> scan -> k3_decode (residuals
+//              into the output buffer as int32) -> k3_zpass / k3_ypass (inclusive
+//              prefix sums along z and y) -> k3_xpass (along x, then
+//              x' = (float)(q * 2 eb) in place)
 // Arithmetic: q = (int)floor((double)x * (0.5 / eb) + 0.5) with the product and
 // the sum rounded separately (the reference is built without FMA; this file is
 // built with -ffp-contract=off); residuals and sums wrap in 32 bits.
